@@ -343,7 +343,7 @@ def hf_llama_decode(torch, prompt_len: int = 16, new_tokens: int = 64) -> dict:
 
 def mfma16_copy_report(model) -> dict:
     """Device memory of the MFMA-16 weight copies int4_gemm attached to the model's INT4 weights
-    (built on the first skinny-kernel call per weight: here the 16-token prefill), against the
+    (built on the first small-M GEMM call per weight: here the 16-token prefill), against the
     INT4 weights themselves."""
     from kernelforge import ops
 
@@ -361,7 +361,7 @@ def mfma16_copy_report(model) -> dict:
     int4 = sum(storages.values())
     return {"weights_with_copy": copies, "copy_bytes": copy_bytes, "int4_weight_bytes": int4,
             "copy_over_int4_weights": round(copy_bytes / int4, 3) if int4 else None,
-            "note": "second layout of each weight the skinny kernel has run on (ops.MFMA16_CACHE)"}
+            "note": "second layout of each weight a small-M GEMM has run on (ops.MFMA16_CACHE)"}
 
 
 def log(msg: str) -> None:

@@ -152,9 +152,9 @@ int kf_int4_gemv_qkv_rope(const void* x, const void* packed, const void* scales,
 size_t kf_int4_gemm_workspace_bytes(int M, int N, int K, int group_size);
 
 /* The kernel kf_int4_gemm() runs for (M, N, K, G) on the current device: *kernel is
- * KF_GEMM_SKINNY or a tile-table index in [0, *num_kernels), *splits the split-K factor
- * (1 = no workspace), *block_m x *block_n the output tile (0 x 0 for the skinny kernel).
- * Any output pointer may be NULL.  For diagnostics and tests; no reference counterpart. */
+ * KF_GEMM_SKINNY (a streaming tile at M <= 32) or the index of a kernel family in [0, *num_kernels)
+ * (kf_gemm.hip lists them), *splits the split-K factor (1 = no workspace), *block_m x *block_n the
+ * output tile.  Any output pointer may be NULL.  For diagnostics and tests; no reference counterpart. */
 #define KF_GEMM_SKINNY (-1)
 int kf_int4_gemm_plan(int M, int N, int K, int group_size, int* kernel, int* num_kernels,
                       int* splits, int* block_m, int* block_n);
@@ -198,10 +198,11 @@ int kf_int4_mfma16_sizes(int N, int K, int group_size, size_t* packed_bytes, siz
 int kf_int4_reorder_mfma16(const void* packed, const void* scales, void* packed_r, void* scales_r,
                            int N, int K, int group_size, void* stream);
 
-/* kf_int4_gemm with the MFMA-16 copy of the same weight: where the skinny kernel runs it
- * streams packed_r / scales_r (contiguous 1 KiB wavefront loads, 7-15% faster), elsewhere
- * packed / scales.  Results are bit-identical to kf_int4_gemm.  Same requirements, plus
- * K % 128 == 0.  No reference counterpart (see kf_int4_reorder_mfma16). */
+/* kf_int4_gemm for a caller that holds the MFMA-16 copy of the same weight.  The kernels read
+ * packed / scales: their copies of the public layout into LDS are contiguous per row and faster than
+ * the skinny kernel that read the copy was (5632 x 2048 at M = 16: 4.8 us against 5.05).  Results are
+ * bit-identical to kf_int4_gemm.  Same requirements, plus a valid copy and K % 128 == 0.  No
+ * reference counterpart (see kf_int4_reorder_mfma16). */
 int kf_int4_gemm_mfma16(const void* x, const void* packed, const void* scales, const void* packed_r,
                         const void* scales_r, void* y, void* ws, size_t ws_bytes,
                         int M, int N, int K, int group_size, void* stream);

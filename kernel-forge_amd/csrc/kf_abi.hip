@@ -121,10 +121,8 @@ int scratch_ptr(void** out) {
 
 // kf_int4_gemm, kf_int4_gemm_mfma16 and kf_int4_gemm_noalloc: validation, plan, workspace check,
 // launch.  With use_scratch the split-K partials go to this device's scratch array (ws is ignored).
-int gemm_entry(const void* x, const void* packed, const void* scales, const void* packed_r, const void* scales_r,
-               void* y, void* ws, size_t ws_bytes, int M, int N, int K, int group_size, void* stream,
-               bool use_scratch = false) {
-
+int gemm_entry(const void* x, const void* packed, const void* scales, void* y, void* ws, size_t ws_bytes, int M, int N,
+               int K, int group_size, void* stream, bool use_scratch = false) {
   int st = check_common(x, packed, scales, y, M, N, K, group_size);
   if (st) return st;
   if (N % 64 != 0) return fail(KF_ERR_UNSUPPORTED, "int4_gemm needs N to be a multiple of 64, got N=%d", N);
@@ -135,9 +133,9 @@ int gemm_entry(const void* x, const void* packed, const void* scales, const void
   int cus = 0;
   if ((st = cu_count(&cus))) return st;
   const kf::GemmPlan plan = kf::gemm_plan(M, N, K, cus);
-  // One workgroup (<= 512 threads) per output tile and split, all in grid dimension x.
+  // One workgroup per output tile and split, all in grid dimension x.
   const long long tiles = (long long)((M + plan.block_m - 1) / plan.block_m) * ((N + plan.block_n - 1) / plan.block_n);
-  if (!plan.skinny && (tiles * plan.splits + 8) * 512 > 0x7FFFFFFFLL)
+  if ((tiles * plan.splits + 8) * plan.threads > 0x7FFFFFFFLL)
     return fail(KF_ERR_UNSUPPORTED, "M=%d, N=%d exceed the grid limit for %dx%d tiles", M, N, plan.block_m,
                 plan.block_n);
   const size_t need = kf::gemm_workspace_bytes(plan, M, N);
@@ -155,7 +153,7 @@ int gemm_entry(const void* x, const void* packed, const void* scales, const void
     if (!aligned(ws, 16)) return fail(KF_ERR_INVALID_ARG, "workspace must be 16-byte aligned");
   }
   return hip_status(kf::gemm_launch(plan, x, packed, scales, y, ws, M, N, K, group_size,
-                                    static_cast<hipStream_t>(stream), packed_r, scales_r),
+                                    static_cast<hipStream_t>(stream)),
                     "int4_gemm launch");
 }
 
@@ -310,22 +308,22 @@ int kf_int4_gemm_plan(int M, int N, int K, int group_size, int* kernel, int* num
   const int st = cu_count(&cus);
   if (st) return st;
   const kf::GemmPlan p = kf::gemm_plan(M, N, K, cus);
-  if (kernel) *kernel = p.skinny ? KF_GEMM_SKINNY : p.tile;
-  if (num_kernels) *num_kernels = kf::gemm_num_tiles();
-  if (splits) *splits = p.skinny ? 1 : p.splits;
-  if (block_m) *block_m = p.skinny ? 0 : p.block_m;
-  if (block_n) *block_n = p.skinny ? 0 : p.block_n;
+  if (kernel) *kernel = p.family;
+  if (num_kernels) *num_kernels = kf::gemm_num_families();
+  if (splits) *splits = p.splits;
+  if (block_m) *block_m = p.block_m;
+  if (block_n) *block_n = p.block_n;
   return KF_OK;
 }
 
 int kf_int4_gemm(const void* x, const void* packed, const void* scales, void* y, void* ws, size_t ws_bytes, int M,
                  int N, int K, int group_size, void* stream) {
-  return gemm_entry(x, packed, scales, nullptr, nullptr, y, ws, ws_bytes, M, N, K, group_size, stream);
+  return gemm_entry(x, packed, scales, y, ws, ws_bytes, M, N, K, group_size, stream);
 }
 
 int kf_int4_gemm_noalloc(const void* x, const void* packed, const void* scales, void* y, int M, int N, int K,
                          int group_size, void* stream) {
-  return gemm_entry(x, packed, scales, nullptr, nullptr, y, nullptr, 0, M, N, K, group_size, stream, true);
+  return gemm_entry(x, packed, scales, y, nullptr, 0, M, N, K, group_size, stream, true);
 }
 
 int kf_int4_mfma16_sizes(int N, int K, int group_size, size_t* packed_bytes, size_t* scales_bytes) {
@@ -357,7 +355,7 @@ int kf_int4_gemm_mfma16(const void* x, const void* packed, const void* scales, c
   int st = kf_int4_mfma16_sizes(N, K, group_size, nullptr, nullptr);
   if (st) return st;
   if (!aligned(packed_r, 16) || !aligned(scales_r, 2)) return fail(KF_ERR_INVALID_ARG, "packed_r / scales_r misaligned");
-  return gemm_entry(x, packed, scales, packed_r, scales_r, y, ws, ws_bytes, M, N, K, group_size, stream);
+  return gemm_entry(x, packed, scales, y, ws, ws_bytes, M, N, K, group_size, stream);
 }
 
 int kf_int4_quantize(const void* w, int dtype, void* packed, void* scales, int N, int K, int group_size,

@@ -126,6 +126,34 @@ __global__ __launch_bounds__(kArgmaxThreads) void decode_argmax_kernel(const hal
   }
 }
 
+// MFMA-16 block layout: one thread per 16-byte piece of the output (grid-stride).  Piece
+// o = ((nb * nss) + s) * 64 + lane holds words 16 s + 4 g .. + 3 of row min(16 nb + lane % 16,
+// N - 1), g = lane / 16; the rows past N repeat row N - 1 (their columns are never stored).
+__global__ __launch_bounds__(256) void reorder_mfma16_kernel(const u32x4* __restrict__ packed,
+                                                             const half_t* __restrict__ scales,
+                                                             u32x4* __restrict__ packed_r, half_t* __restrict__ scales_r,
+                                                             int N, int K, int groups) {
+  const int nss = K >> 7;
+  const int nblk = (N + 15) >> 4;
+  const size_t pieces = (size_t)nblk * nss * 64;
+  for (size_t o = (size_t)blockIdx.x * 256 + threadIdx.x; o < pieces; o += (size_t)gridDim.x * 256) {
+    const int lane = (int)(o & 63);
+    const size_t bs = o >> 6;
+    const int s = (int)(bs % nss);
+    const int nb = (int)(bs / nss);
+    const int n = min(16 * nb + (lane & 15), N - 1);
+    packed_r[o] = packed[(size_t)n * (K >> 5) + 4 * s + (lane >> 4)];
+  }
+  const size_t nscales = (size_t)nblk * groups * 16;
+  for (size_t o = (size_t)blockIdx.x * 256 + threadIdx.x; o < nscales; o += (size_t)gridDim.x * 256) {
+    const int col = (int)(o & 15);
+    const size_t bj = o >> 4;
+    const int j = (int)(bj % groups);
+    const int nb = (int)(bj / groups);
+    scales_r[o] = scales[(size_t)min(16 * nb + col, N - 1) * groups + j];
+  }
+}
+
 }  // namespace
 
 hipError_t decode_argmax_launch(const void* logits, int n, void* token, void* pos, void* history, int max_seq,
@@ -168,6 +196,20 @@ hipError_t bw_read_store_launch(const void* src, void* out, size_t bytes, int gr
 
 hipError_t bw_write_launch(void* dst, size_t bytes, int grid, hipStream_t stream) {
   hipLaunchKernelGGL(bw_write_kernel, dim3(grid), dim3(256), 0, stream, static_cast<u32x4*>(dst), bytes / 16);
+  return hipGetLastError();
+}
+
+size_t mfma16_packed_words(int N, int K) { return (size_t)ceil_div(N, 16) * 16 * (K / 8); }
+size_t mfma16_scale_count(int N, int K, int group_size) { return (size_t)ceil_div(N, 16) * 16 * (K / group_size); }
+
+hipError_t reorder_mfma16_launch(const void* packed, const void* scales, void* packed_r, void* scales_r, int N, int K,
+                                 int group_size, hipStream_t stream) {
+  const size_t pieces = mfma16_packed_words(N, K) / 4;
+  size_t blocks = (pieces + 255) / 256;
+  if (blocks > 8192) blocks = 8192;
+  hipLaunchKernelGGL(reorder_mfma16_kernel, dim3((unsigned)blocks), dim3(256), 0, stream,
+                     static_cast<const u32x4*>(packed), static_cast<const half_t*>(scales),
+                     static_cast<u32x4*>(packed_r), static_cast<half_t*>(scales_r), N, K, K / group_size);
   return hipGetLastError();
 }
 

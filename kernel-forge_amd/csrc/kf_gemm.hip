@@ -6,32 +6,22 @@
 // fixed split order (deterministic), the behaviour of the reference's splitk_reduce
 // (dequant_gemm_tc_kernel.cuh:156-162).
 //
-// Three kernel families share one tile table (kTiles below; gemm_plan picks an entry and a
-// split-K factor with a fitted cost model):
-//   * gemm_kernel<TileCfg>: register-staged LDS tiles, 64 x 128 down to 16 x 64;
-//   * gemm_dma_kernel<KW>: 128 x 128 tiles fed by LDS-DMA, 2 (4 wavefronts) or 4 (8 wavefronts)
-//     k-groups; see the comment above the kernel;
+// Kernel families (gemm_plan picks one, its tile and a split-K factor with a fitted cost model):
+//   * streaming tiles (kf_stream.hip), 8 x 16 up to 64 x 64: small and medium M;
+//   * gemm_dma4_kernel<TM, TN, NS>: (16 TM) x (32 TN) tiles fed by LDS-DMA, 8 wavefronts as 4 k-groups x
+//     2 column halves, 128-k stages, for grids of up to about one tile per CU;
+//   * gemm_dma2_kernel: 128 x 128 tiles fed by LDS-DMA, 4 wavefronts, for grids of several tiles per CU;
 //   * gemm_wide_kernel: 192 x 256 tiles fed by LDS-DMA, 8 wavefronts, one workgroup per CU, for
 //     grids of about one tile per CU (half the L2 -> LDS bytes per output of the 128 x 128 tiles).
 //
-// Design of gemm_kernel (gfx950: 4 SIMDs per CU, ~2 VALU ops hide under one 16x16x32 MFMA,
-// LDS reads ~150-200 B/clk per CU):
-//   * Workgroup tile BM x BN; WGM x WGN wavefronts tile it, and WK such groups split each
-//     stage's k range (in-block split-K, summed in fixed order through LDS at the end).
-//   * A stage covers SK = 64 * WK k.  x is staged in LDS as fp16; the weights stay PACKED
-//     in LDS (4 bits per weight: 4x less LDS traffic than an fp16 W_hat tile).  Each
-//     wavefront dequantizes only its own columns, with one scale per column and stage, so
-//     a weight is dequantized once per (workgroup, M-wavefront row); with WGM = 1 that is
-//     once per workgroup.
-//   * Global -> registers two stages ahead, registers -> LDS one stage ahead, LDS double
-//     buffered: one barrier per stage.
-//   * LDS layouts are XOR-swizzled so every fragment read and tile write is free of bank
-//     conflicts on gfx950's 64-bank LDS: x rows are 16-byte chunks c stored at slot
-//     c ^ f(row); packed rows are 8-byte units u stored at u ^ f'(row).
-//   * MFMA operands: lane l serves row / column l % 16 and k-group g = l / 16.  In sub-step
-//     t (0, 1) of k-group kw it supplies k = 64 kw + 16 g + 8 t .. +7 for both A (one
-//     16-byte x chunk) and B (one packed word, dequantized with dequant8), so one 8-byte
-//     LDS read gives a lane both sub-steps' weights.
+// Common to the DMA tiles (gfx950: 4 SIMDs per CU, ~2 VALU ops hide under one 16x16x32 MFMA, LDS
+// reads ~150-200 B/clk per CU):
+//   * Every byte of a stage goes global -> LDS through LDS-DMA; the weights stay PACKED in LDS (4
+//     bits per weight: 4x less LDS traffic than an fp16 W_hat tile) and each wavefront dequantizes
+//     its own columns' words.
+//   * LDS layouts are XOR-swizzled so every fragment read is free of bank conflicts on gfx950's
+//     64-bank LDS.
+//   * MFMA operands: lane l serves row / column l % 16 and k-group g = l / 16.
 //   * Tiles are ordered in bands of group_m M-tiles (all N-tiles of a band before the next
 //     band); the (split, tile) jobs of a launch, split-major, are dealt to the 8 XCDs in
 //     contiguous runs of equal length, so the x rows an XCD uses stay in its L2, each weight
@@ -60,288 +50,7 @@ __device__ __forceinline__ bool gemm_job(int tiles, int splits, int& split, int&
   return true;
 }
 
-template <int BM_, int BN_, int WGM_, int WGN_, int WK_, int WAVES_PER_SIMD_ = 2>
-struct TileCfg {
-  static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, WK = WK_;
-  // Occupancy target: 2 wavefronts per SIMD leave 256 registers per lane, 1 leaves 512.
-  static constexpr int WAVES_PER_SIMD = WAVES_PER_SIMD_;
-  static constexpr int THREADS = 64 * WGM * WGN * WK;
-  static constexpr int SK = 64 * WK;                  // k per stage
-  static constexpr int A_ROW = 2 * SK;                // bytes per x row in LDS
-  static constexpr int A_CHUNKS_ROW = SK / 8;         // 16-byte chunks per x row
-  static constexpr int B_ROW = SK / 2;                // bytes per packed row in LDS
-  static constexpr int B_CHUNKS_ROW = SK / 32;        // 16-byte chunks per packed row
-  static constexpr int B_UNITS_ROW = SK / 16;         // 8-byte units per packed row
-  static constexpr int A_STAGE = BM * A_ROW;
-  static constexpr int B_STAGE = BN * B_ROW;
-  static constexpr int S_STAGE = WK * BN * 2;         // fp16 scales [WK][BN]
-  static constexpr int STAGE = A_STAGE + B_STAGE + S_STAGE;
-  static constexpr int A_CHUNKS = BM * A_CHUNKS_ROW;
-  static constexpr int B_CHUNKS = BN * B_CHUNKS_ROW;
-  static constexpr int A_PER_T = A_CHUNKS / THREADS;
-  static constexpr int B_PER_T = (B_CHUNKS + THREADS - 1) / THREADS;
-  static constexpr int TM = BM / WGM / 16;            // 16x16 blocks per wavefront along M
-  static constexpr int TN = BN / WGN / 16;            // ... along N
-  static constexpr int RED = (WK - 1) * WGM * WGN * TM * TN * 256 * 4;  // bytes of k-group partials
-  static_assert(A_CHUNKS % THREADS == 0, "x tile must split evenly over the threads");
-  static_assert(TM >= 1 && TN >= 1 && BM % (16 * WGM) == 0 && BN % (16 * WGN) == 0, "wave tile");
-  static_assert(16 % B_UNITS_ROW == 0, "packed-row swizzle needs 4, 8 or 16 units per row");
-  static_assert(STAGE % 16 == 0, "stage alignment");
-  static_assert(RED <= 2 * STAGE, "k-group reduction must fit in the stage buffers");
-  static_assert(2 * STAGE <= 160 * 1024, "LDS");
-};
-
-// Swizzle of 8-byte units in packed row `row`: rows that a 16-lane phase of an 8-byte read
-// touches land on distinct banks.
-template <class C>
-__device__ __forceinline__ int b_swizzle(int row) {
-  return (row / (16 / C::B_UNITS_ROW)) & (C::B_UNITS_ROW - 1);
-}
-
-template <class C>
-struct StageRegs {
-  u32x4 a[C::A_PER_T];
-  u32x4 b[C::B_PER_T];
-  half_t s[C::B_PER_T];
-};
-
-template <class C>
-__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(C::WAVES_PER_SIMD, C::WAVES_PER_SIMD)))
-void gemm_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ packed, const half_t* __restrict__ scales,
-                 half_t* __restrict__ y, float* __restrict__ ws, int M, int N, int K, int log2_group,
-                 int stages_per_split, int splits, int tiles_m, int tiles_n, int group_m) {
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2 * C::STAGE];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kw = wave / (C::WGM * C::WGN);
-  const int wmn = wave - kw * (C::WGM * C::WGN);
-  const int wm = wmn / C::WGN;
-  const int wn = wmn - wm * C::WGN;
-  const int g = lane >> 4;
-  const int l16 = lane & 15;
-
-  // Split and tile of this workgroup (see the header comment for the order).
-  int split, t;
-  if (!gemm_job(tiles_m * tiles_n, splits, split, t)) return;
-  const int band = group_m * tiles_n;
-  const int bi = t / band;
-  const int tb = t - bi * band;
-  const int gm = min(group_m, tiles_m - bi * group_m);
-  const int mt = bi * group_m + tb % gm;
-  const int nt = tb / gm;
-  const int m0 = mt * C::BM;
-  const int n0 = nt * C::BN;
-
-  const int nst = K / C::SK;
-  const int st_begin = split * stages_per_split;
-  const int st_end = min(nst, st_begin + stages_per_split);
-  const int ns = st_end - st_begin;
-  const int words_per_row = K >> 3;
-  const int groups_per_row = K >> log2_group;
-
-  // Global -> registers.  Rows of x past M are clamped (they only feed output rows that
-  // are never stored); weight rows past N are clamped the same way.  Every thread loads
-  // every stage unconditionally (stage indices are clamped instead), which keeps the
-  // compiler's per-register load tracking exact: a wait covers only the stage it needs.
-  const half_t* a_src[C::A_PER_T];
-#pragma unroll
-  for (int j = 0; j < C::A_PER_T; ++j) {
-    const int i = tid + C::THREADS * j;
-    const int row = i / C::A_CHUNKS_ROW, c = i % C::A_CHUNKS_ROW;
-    a_src[j] = x + (size_t)min(m0 + row, M - 1) * K + 8 * c;
-  }
-  const uint32_t* b_src[C::B_PER_T];
-  const half_t* s_src[C::B_PER_T];
-#pragma unroll
-  for (int j = 0; j < C::B_PER_T; ++j) {
-    const int i = min(tid + C::THREADS * j, C::B_CHUNKS - 1);
-    const int row = i / C::B_CHUNKS_ROW, h = i % C::B_CHUNKS_ROW;
-    const int n = min(n0 + row, N - 1);
-    b_src[j] = packed + (size_t)n * words_per_row + 4 * h;
-    s_src[j] = scales + (size_t)n * groups_per_row;
-  }
-  auto load = [&](StageRegs<C>& R, int st) {
-    const int k0 = st * C::SK;
-#pragma unroll
-    for (int j = 0; j < C::A_PER_T; ++j) R.a[j] = load_u32x4(a_src[j] + k0);
-#pragma unroll
-    for (int j = 0; j < C::B_PER_T; ++j) {
-      const int h = (tid + C::THREADS * j) % C::B_CHUNKS_ROW;
-      R.b[j] = load_u32x4(b_src[j] + (k0 >> 3));
-      R.s[j] = s_src[j][(k0 + 32 * (h & ~1)) >> log2_group];
-    }
-  };
-
-  // x tile: 16-byte chunk c of row r sits at slot c ^ a_swizzle(r).  Sixteen consecutive
-  // rows (one 16-lane phase of a 16-byte read) then cover all 64 banks.
-  auto a_slot = [](int row, int c) {
-    constexpr int RSH = C::A_ROW >= 256 ? 0 : 1;  // rows per 256-byte bank window: 1 or 2
-    return c ^ ((row >> RSH) & (C::A_CHUNKS_ROW - 1));
-  };
-
-  // Registers -> LDS stage buffer (swizzled).
-  auto store = [&](const StageRegs<C>& R, unsigned char* st) {
-#pragma unroll
-    for (int j = 0; j < C::A_PER_T; ++j) {
-      const int i = tid + C::THREADS * j;
-      const int row = i / C::A_CHUNKS_ROW, c = i % C::A_CHUNKS_ROW;
-      *reinterpret_cast<u32x4*>(st + row * C::A_ROW + 16 * a_slot(row, c)) = R.a[j];
-    }
-#pragma unroll
-    for (int j = 0; j < C::B_PER_T; ++j) {
-      const int i = tid + C::THREADS * j;
-      if (C::B_CHUNKS % C::THREADS == 0 || i < C::B_CHUNKS) {
-        const int row = i / C::B_CHUNKS_ROW, h = i % C::B_CHUNKS_ROW;
-        const int sw = b_swizzle<C>(row);
-        unsigned char* rb = st + C::A_STAGE + row * C::B_ROW;
-        *reinterpret_cast<uint2*>(rb + 8 * ((2 * h) ^ sw)) = uint2{R.b[j].x, R.b[j].y};
-        *reinterpret_cast<uint2*>(rb + 8 * ((2 * h + 1) ^ sw)) = uint2{R.b[j].z, R.b[j].w};
-        if ((h & 1) == 0)
-          reinterpret_cast<half_t*>(st + C::A_STAGE + C::B_STAGE)[(h >> 1) * C::BN + row] = R.s[j];
-      }
-    }
-  };
-
-  float4_t acc[C::TM][C::TN];
-#pragma unroll
-  for (int i = 0; i < C::TM; ++i)
-#pragma unroll
-    for (int j = 0; j < C::TN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
-
-  // Packed words (both sub-steps) and scales of this wave's columns for one stage.
-  uint2 bw[C::TN];
-  half2_t s2[C::TN];
-  auto read_b = [&](const unsigned char* st) {
-#pragma unroll
-    for (int j = 0; j < C::TN; ++j) {
-      const int row = (wn * C::TN + j) * 16 + l16;
-      const int u = 4 * kw + g;
-      bw[j] = *reinterpret_cast<const uint2*>(st + C::A_STAGE + row * C::B_ROW + 8 * (u ^ b_swizzle<C>(row)));
-      const half_t sc = reinterpret_cast<const half_t*>(st + C::A_STAGE + C::B_STAGE)[kw * C::BN + row];
-      s2[j] = half2_t{sc, sc};
-    }
-  };
-  auto read_a = [&](const unsigned char* st, int sub, half8_t (&a)[C::TM]) {
-#pragma unroll
-    for (int i = 0; i < C::TM; ++i) {
-      const int row = (wm * C::TM + i) * 16 + l16;
-      a[i] = *reinterpret_cast<const half8_t*>(st + row * C::A_ROW + 16 * a_slot(row, 8 * kw + 2 * g + sub));
-    }
-  };
-  auto mfma_sub = [&](const half8_t (&a)[C::TM], const uint32_t (&w)[C::TN], const half2_t (&sc)[C::TN]) {
-#pragma unroll
-    for (int j = 0; j < C::TN; ++j) {
-      const half8_t b = dequant8(w[j], sc[j]);
-#pragma unroll
-      for (int i = 0; i < C::TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, a[i], acc[i][j], 0, 0, 0);
-    }
-  };
-
-  // Software pipeline, one barrier per stage.  Stage s lives in LDS buffer s % 2 and is
-  // computed in two sub-steps; the LDS reads for the next sub-step are issued before the
-  // MFMAs of the current one, and the barrier sits between the two sub-steps:
-  //   read x(sub 1) | MFMA sub 0 | write stage s+1 to the other buffer, load stage s+3 |
-  //   barrier | read words, scales, x(sub 0) of stage s+1 | MFMA sub 1
-  // Registers R[(s+1) % 2] carry stage s+1 from global memory to LDS (loaded two stages
-  // ahead).  Stage indices past the split's end are clamped to its last stage; those
-  // duplicate loads, writes and reads are never used.
-  unsigned char* const L0 = smem;
-  unsigned char* const L1 = smem + C::STAGE;
-  const int last = st_end - 1;
-  auto stage_at = [&](int i) { return min(st_begin + i, last); };
-  StageRegs<C> R0, R1;
-  half8_t a0[C::TM], a1[C::TM];
-  if (ns > 0) {
-    load(R0, stage_at(0));
-    load(R1, stage_at(1));
-    store(R0, L0);
-    load(R0, stage_at(2));
-    __syncthreads();
-    read_b(L0);
-    read_a(L0, 0, a0);
-
-    auto half_iter = [&](auto cur_c, int s) {
-      constexpr int CUR = decltype(cur_c)::value;
-      unsigned char* const cur = CUR ? L1 : L0;
-      unsigned char* const nxt = CUR ? L0 : L1;
-      StageRegs<C>& Rn = CUR ? R0 : R1;
-      uint32_t w0[C::TN], w1[C::TN];
-      half2_t sc[C::TN];
-#pragma unroll
-      for (int j = 0; j < C::TN; ++j) {
-        w0[j] = bw[j].x;
-        w1[j] = bw[j].y;
-        sc[j] = s2[j];
-      }
-      read_a(cur, 1, a1);
-      mfma_sub(a0, w0, sc);
-      store(Rn, nxt);
-      load(Rn, stage_at(s + 3));
-      __syncthreads();
-      read_b(nxt);
-      read_a(nxt, 0, a0);
-      mfma_sub(a1, w1, sc);
-    };
-    for (int s = 0; s < ns; s += 2) {
-      half_iter(std::integral_constant<int, 0>(), s);
-      if (s + 1 >= ns) break;
-      half_iter(std::integral_constant<int, 1>(), s + 1);
-    }
-  }
-  __syncthreads();
-
-  // In-block split-K: k-groups 1.. hand their partial tiles to k-group 0 through LDS (the
-  // stage buffers are free after the barrier above) and it adds them in fixed order.
-  if constexpr (C::WK > 1) {
-    float* red = reinterpret_cast<float*>(smem);
-    constexpr int WAVE_FLOATS = C::TM * C::TN * 256;
-    if (kw > 0) {
-#pragma unroll
-      for (int i = 0; i < C::TM; ++i)
-#pragma unroll
-        for (int j = 0; j < C::TN; ++j)
-          *reinterpret_cast<float4_t*>(
-              &red[((kw - 1) * C::WGM * C::WGN + wmn) * WAVE_FLOATS + (i * C::TN + j) * 256 + 4 * lane]) = acc[i][j];
-    }
-    __syncthreads();
-    if (kw > 0) return;
-#pragma unroll
-    for (int q = 1; q < C::WK; ++q)
-#pragma unroll
-      for (int i = 0; i < C::TM; ++i)
-#pragma unroll
-        for (int j = 0; j < C::TN; ++j)
-          acc[i][j] += *reinterpret_cast<const float4_t*>(
-              &red[((q - 1) * C::WGM * C::WGN + wmn) * WAVE_FLOATS + (i * C::TN + j) * 256 + 4 * lane]);
-  }
-
-  // The MFMAs take the weights as their first operand, so each 16 x 16 block comes out transposed:
-  // lane l, element r holds y row l%16, column 4*(l/16)+r.  A lane stores its four consecutive
-  // columns at once (8 bytes of y or 16 of fp32 partials); N % 64 == 0 keeps them inside the row.
-  float* part = ws ? ws + (size_t)split * M * N : nullptr;
-#pragma unroll
-  for (int i = 0; i < C::TM; ++i) {
-    const int row = m0 + (wm * C::TM + i) * 16 + l16;
-    if (row >= M) continue;
-#pragma unroll
-    for (int j = 0; j < C::TN; ++j) {
-      const int col = n0 + (wn * C::TN + j) * 16 + 4 * g;
-      if (col >= N) continue;
-      if (part) {
-        *reinterpret_cast<float4_t*>(part + (size_t)row * N + col) = acc[i][j];
-      } else {
-        const half2_t lo = {(half_t)acc[i][j][0], (half_t)acc[i][j][1]};
-        const half2_t hi = {(half_t)acc[i][j][2], (half_t)acc[i][j][3]};
-        *reinterpret_cast<u32x2*>(y + (size_t)row * N + col) = u32x2{bit_cast<uint32_t>(lo), bit_cast<uint32_t>(hi)};
-      }
-    }
-  }
-}
-
-// ---- DMA-fed kernel: 128 x 128 tile, KW k-groups (KW = 2: 4 wavefronts, 64-k stages;
-// KW = 4: 8 wavefronts, 128-k stages) ------------------------------------------------
+// ---- gemm_dma2_kernel: 128 x 128 tile, 2 k-groups (4 wavefronts), 64-k stages ---------------
 //
 // Every byte of a stage goes global -> LDS through the gfx950 LDS-DMA loads
 // (global_load_lds_dwordx4 / _ushort: lane l's data lands at M0 + 16 l, or M0 + 4 l for
@@ -352,10 +61,9 @@ void gemm_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ pack
 // stay well under the LDS bandwidth).
 //
 // Wavefront (kw, wn): column half wn (64 columns) and k-group kw, which takes k 32 kw ..
-// 32 kw + 31 of every stage; the k-groups' accumulators are summed in fixed order through LDS
-// at the end (in-block split-K).  KW = 2 gives four wave tasks per 128 x 128 tile, enough to
-// spread evenly over the 1024 SIMDs when the grid has several tiles per CU; KW = 4 gives one
-// workgroup of two wavefronts per SIMD when the grid has about one tile per CU.
+// 32 kw + 31 of every 64-k stage; the k-groups' accumulators are summed in fixed order through LDS
+// at the end (in-block split-K).  Four wave tasks per 128 x 128 tile spread evenly over the 1024
+// SIMDs when the grid has several tiles per CU.
 //
 // The DMA loads are issued from inline assembly with a "memory" clobber: the compiler
 // neither tracks them nor moves LDS accesses across them, and the loop contains no
@@ -367,18 +75,12 @@ void gemm_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ pack
 // LDS stage layout (bytes): x rows of A_ROW = 2 BK bytes with 16-byte chunk c at slot
 // c ^ a_swz(row); packed rows of BK / 2 bytes with 16-byte chunk h at h ^ b_swz(row).  Every
 // read phase of the MFMA fragments is free of bank conflicts.  Three stages rotate.  Scales:
-// with KW = 2 a stage lies inside one group (G >= 64 = BK), so they live in their own ring of
-// three slabs of 4-byte slots, one slab per group, fetched by the k-group 0 wavefronts with
-// the first stage of the group (that stage costs those two wavefronts one more DMA, and their
-// wait count for it is one higher); with KW = 4 each stage carries the slabs of its one or two
-// groups, fetched by the first one or two k-groups with every stage.
-// Constants of the DMA-fed kernel with KW k-groups (KW = 2: 4 wavefronts, 64-k stages;
-// KW = 4: 8 wavefronts, 128-k stages).  Every wavefront owns a 128 x 64 wave tile over a 32-k
-// slice of each stage, so the VALU/MFMA and LDS/MFMA ratios are the same for both; KW = 4 puts
-// two wavefronts per SIMD into one workgroup per CU, for grids with about one tile per CU.
-template <int KW>
+// a stage lies inside one group (G >= 64 = BK), so they live in their own ring of three slabs of
+// 4-byte slots, one slab per group, fetched by the k-group 0 wavefronts with the first stage of the
+// group (that stage costs those two wavefronts one more DMA, and their wait count for it is one
+// higher).
 struct DmaCfg {
-  static constexpr int BM = 128, BN = 128, BK = 32 * KW, NS = 3, WAVES = 2 * KW, THREADS = 64 * WAVES;
+  static constexpr int KW = 2, BM = 128, BN = 128, BK = 32 * KW, NS = 3, WAVES = 2 * KW, THREADS = 64 * WAVES;
   static constexpr int TM = 8, TN = 4;
   static constexpr int A_ROW = BK * 2;               // bytes of x per row and stage (128 / 256)
   static constexpr int A_CH = BK / 8;                // 16-byte chunks per x row (8 / 16)
@@ -388,15 +90,10 @@ struct DmaCfg {
   static constexpr int B_ROW = BK / 2;               // bytes of packed weights per row and stage
   static constexpr int B_CH = BK / 32;               // 16-byte chunks per packed row (2 / 4)
   static constexpr int B_BYTES = BN * B_ROW;
-  // Scales.  KW = 2: a stage lies inside one group (G >= 64 = BK), so the scales live in a ring
-  // of NS per-group slabs after the stages and are fetched once per group.  KW = 4: a stage
-  // holds one (G = 128) or two (G = 64) groups, fetched with the stage into its own slabs.
-  static constexpr bool STAGE_SCALES = KW == 4;
-  static constexpr int S_SLAB = BN * 4;              // [BN] 4-byte slots
-  static constexpr int S_OFF = B_OFF + B_BYTES;      // per-stage slabs (KW = 4): [2][BN]
-  static constexpr int STAGE = STAGE_SCALES ? S_OFF + 2 * S_SLAB : S_OFF;
-  static constexpr int S_RING = NS * STAGE;          // per-group ring (KW = 2): [NS][BN]
-  static constexpr int RING_END = S_RING + (STAGE_SCALES ? 0 : NS * S_SLAB);
+  static constexpr int STAGE = B_OFF + B_BYTES;
+  static constexpr int S_SLAB = BN * 4;              // [BN] 4-byte scale slots
+  static constexpr int S_RING = NS * STAGE;          // per-group ring: [NS][BN]
+  static constexpr int RING_END = S_RING + NS * S_SLAB;
   static constexpr int OUT_ROW = BN * 2 + 16;        // epilogue fp16 tile row stride (bytes), padded
   static constexpr int WAVE_TILE = TM * TN * 256 * 4;  // fp32 partial tile of one wavefront
   static constexpr int RED_BYTES = (KW / 2) * 2 * WAVE_TILE;  // k-group partials staged at once
@@ -414,13 +111,12 @@ __device__ __forceinline__ void dma_u16(uint32_t lds, const void* src) {
   asm volatile("global_load_lds_ushort %1, off" ::"{m0}"(lds), "v"(src) : "memory");
 }
 
-template <int KW>
-__global__ __launch_bounds__(DmaCfg<KW>::THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void gemm_dma_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ packed,
+__global__ __launch_bounds__(DmaCfg::THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gemm_dma2_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ packed,
                      const half_t* __restrict__ scales, half_t* __restrict__ y, float* __restrict__ ws, int M, int N,
                      int K, int log2_group, int stages_per_split, int splits, int tiles_m, int tiles_n,
                      int group_m) {
-  using C = DmaCfg<KW>;
+  using C = DmaCfg;
   constexpr int BM = C::BM, BN = C::BN, BK = C::BK, NS = C::NS, THREADS = C::THREADS, TM = C::TM, TN = C::TN;
   constexpr int A_ROW = C::A_ROW, B_ROW = C::B_ROW, B_OFF = C::B_OFF, STAGE = C::STAGE, OUT_ROW = C::OUT_ROW;
   constexpr int kDmaPerStage = C::kDmaPerStage;
@@ -469,10 +165,10 @@ void gemm_dma_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ 
   const half_t* s_src = scales + (size_t)min(n0 + 64 * wn + lane, N - 1) * groups;
   const uint32_t smem_base = (uint32_t)(uintptr_t)smem;
 
-  // KW = 2, per-group scale ring: split-local stage i (clamped) starts a scale group when
+  // Per-group scale ring: split-local stage i (clamped) starts a scale group when
   // i == 0 or its k0 is a multiple of G; groups are numbered from the split's first stage.
   // The clamped repeats of the last stage past the split's end never start one.
-  const int log2_spg = log2_group - 6;  // log2(stages per group), KW = 2
+  const int log2_spg = log2_group - 6;  // log2(stages per group)
   auto starts_group = [&](int i) {
     const int st = st_begin + i;
     return i == 0 || (st <= last && (st & ((1 << log2_spg) - 1)) == 0);
@@ -480,11 +176,6 @@ void gemm_dma_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ 
   auto group_of = [&](int i) {  // split-local group index of split-local stage i (i <= ns - 1)
     return ((st_begin + i) >> log2_spg) - (st_begin >> log2_spg);
   };
-  // KW = 4, per-stage scales: a stage holds gps = BK / G groups (1 or 2); k-group kw < gps
-  // fetches group gps * st + kw for its wavefronts' 64 columns, and k-group kw reads slab
-  // (32 kw) >> log2_group.
-  const int gps = BK >> log2_group;
-  const bool stage_scale_loader = C::STAGE_SCALES && kw < gps;
   // DMA of split-local stage i (clamped) into buffer i % NS, plus scales.  Returns whether
   // this wavefront issued a scale load (one more outstanding load).
   auto issue = [&](int i, int buf) {  // buf == i % NS
@@ -494,21 +185,13 @@ void gemm_dma_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ 
 #pragma unroll
     for (int q = 0; q < 4; ++q) dma_16B(base + 1024 * (4 * wave + q), a_src[q] + k0);
     dma_16B(base + B_OFF + 1024 * wave, b_src + (k0 >> 3));
-    if constexpr (C::STAGE_SCALES) {
-      if (stage_scale_loader) {
-        dma_u16(__builtin_amdgcn_readfirstlane(base + (uint32_t)(C::S_OFF + kw * C::S_SLAB + 256 * wn)),
-                s_src + gps * st + kw);
-      }
-      return stage_scale_loader;
-    } else {
-      const bool sc = kw == 0 && starts_group(i);
-      if (sc) {
-        const uint32_t sbase = __builtin_amdgcn_readfirstlane(
-            smem_base + (uint32_t)(C::S_RING + (group_of(i) % NS) * C::S_SLAB + 256 * wn));
-        dma_u16(sbase, s_src + (k0 >> log2_group));
-      }
-      return sc;
+    const bool sc = kw == 0 && starts_group(i);
+    if (sc) {
+      const uint32_t sbase = __builtin_amdgcn_readfirstlane(
+          smem_base + (uint32_t)(C::S_RING + (group_of(i) % NS) * C::S_SLAB + 256 * wn));
+      dma_u16(sbase, s_src + (k0 >> log2_group));
     }
+    return sc;
   };
   auto wait_older = [&](bool newer_has_scales) {  // all but the newest stage's loads landed
     if (newer_has_scales)
@@ -527,7 +210,7 @@ void gemm_dma_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ 
   // packed: row 64 wn + 16 j + l16, dword 4 kw + g.  scales: column 64 wn + 16 j + l16.
   const int a_off = l16 * A_ROW + 16 * ((4 * kw + g) ^ a_swz(l16));
   const int b_off = B_OFF + (64 * wn + l16) * B_ROW + 16 * (kw ^ b_swz(l16)) + 4 * g;
-  const int s_off = 4 * (64 * wn + l16) + (C::STAGE_SCALES ? C::S_OFF + ((32 * kw) >> log2_group) * C::S_SLAB : 0);
+  const int s_off = 4 * (64 * wn + l16);
 
   const UnpackConsts uc = unpack_consts();
   half8_t a[TM];
@@ -535,7 +218,7 @@ void gemm_dma_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ 
   half2_t s2[TN];
   auto read_frags = [&](int i, int buf) {  // buf == i % NS, a compile-time constant at the call
     const unsigned char* st = smem + buf * STAGE;
-    const unsigned char* slab = C::STAGE_SCALES ? st : smem + C::S_RING + (group_of(i) % NS) * C::S_SLAB;
+    const unsigned char* slab = smem + C::S_RING + (group_of(i) % NS) * C::S_SLAB;
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
       w[j] = *reinterpret_cast<const uint32_t*>(st + b_off + 16 * B_ROW * j);
@@ -550,7 +233,7 @@ void gemm_dma_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ 
   // wavefront waits for its own loads of it and the barrier publishes it; at iteration i
   // its fragments are read and its MFMAs run.  The DMA of stage i + 2 (iteration i)
   // overwrites the buffer of stage i - 1, whose reads completed before the barrier of
-  // iteration i - 1 (lgkmcnt(0) precedes every barrier).  Likewise (KW = 2) the scale slab
+  // iteration i - 1 (lgkmcnt(0) precedes every barrier).  Likewise the scale slab
   // of group q is fetched with q's first stage i (iteration i - 2) into the slab of group
   // q - 3, last read at a stage <= i - 3 (groups span >= 1 stage), before that barrier.
   // The loop is unrolled by NS so every buffer offset is a compile-time immediate.
@@ -580,32 +263,20 @@ void gemm_dma_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ 
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clamped tail loads, before LDS is reused
   __syncthreads();
 
-  // The k-groups' partial tiles are added in fixed order through LDS: KW = 2: a0 + a1;
-  // KW = 4: (a0 + a2) + (a1 + a3).  Round r hands k-group giver's tile to k-group taker through
-  // slot h (one 2 x wave-tile region per slot); straight-line code keeps acc in registers.
-  float* red = reinterpret_cast<float*>(smem);
-  constexpr int ROUNDS = KW == 4 ? 2 : 1;
+  // The k-groups' partial tiles are added in fixed order (a0 + a1) through LDS.
+  float* red = reinterpret_cast<float*>(smem) + wn * TM * TN * 256 + 4 * lane;
+  if (kw == 1) {
 #pragma unroll
-  for (int r = 0; r < ROUNDS; ++r) {
-    const bool last_round = r == ROUNDS - 1;
-    const bool give = last_round ? kw == 1 : kw >= 2;
-    const bool take = last_round ? kw == 0 : kw < 2;
-    const int h = last_round ? 0 : (kw & 1);
-    float* base = red + ((h * 2 + wn) * TM * TN) * 256 + 4 * lane;
-    if (r > 0) __syncthreads();  // the previous round's tiles have been read
-    if (give) {
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
+      for (int j = 0; j < TN; ++j) *reinterpret_cast<float4_t*>(red + (i * TN + j) * 256) = acc[i][j];
+  }
+  __syncthreads();
+  if (kw == 0) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j) *reinterpret_cast<float4_t*>(base + (i * TN + j) * 256) = acc[i][j];
-    }
-    __syncthreads();
-    if (take) {
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] += *reinterpret_cast<const float4_t*>(base + (i * TN + j) * 256);
-    }
+      for (int j = 0; j < TN; ++j) acc[i][j] += *reinterpret_cast<const float4_t*>(red + (i * TN + j) * 256);
   }
 
   // The MFMAs take the weights as their first operand, so each 16 x 16 block comes out
@@ -618,12 +289,8 @@ void gemm_dma_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ 
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-          const int row = m0 + 16 * i + l16;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int col = n0 + 64 * wn + 16 * j + 4 * g + r;
-            if (row < M && col < N) part[(size_t)row * N + col] = acc[i][j][r];
-          }
+          const int row = m0 + 16 * i + l16, col = n0 + 64 * wn + 16 * j + 4 * g;
+          if (row < M && col < N) *reinterpret_cast<float4_t*>(part + (size_t)row * N + col) = acc[i][j];
         }
     }
     return;
@@ -652,13 +319,237 @@ void gemm_dma_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ 
   }
 }
 
+// ---- gemm_dma4_kernel: (16 TM) x (32 TN) tile, 4 k-groups (8 wavefronts), 128-k stages ------------
+//
+// The tile for grids of up to about one workgroup per CU: eight wavefronts as 2 column halves x 4
+// k-groups, so a small tile still keeps two wavefronts on every SIMD, and TM row blocks per
+// dequantized word.  The row count is the point of the template: the tile height is chosen so that M
+// pads little and the grid fills the CUs (M = 517 in 112-row tiles is 560 rows, in 128-row tiles 640;
+// M = 200 in 80-row tiles is three tiles).  Stages rotate through NS buffers, NS - 1 of them in
+// flight, and the loop is rolled (buffer offsets in registers): each wavefront issues the same
+// number of copies per stage, so one counted wait serves the whole loop.  Copies past a tile's last
+// instruction repeat that instruction (same bytes to the same place).
+// MI355X, against the 64 x 128 register-staged and 128 x 128 tiles chosen before: N x K = 2048 x 5632 at
+// M = 517 / 768: 42.8 / 43.9 -> 24.8 / 29.0 us; 4096 x 4096 at M = 517: 34.4 -> 26.5; 1536 x 8960 at
+// M = 517 / 1024: 45.8 / 55.4 -> 27.4 / 42.7; 128 x 128 itself (2048 x 5632 at M = 2048): 52.1 -> 47.9.
+template <int TM_, int TN_, int NS_>
+struct Dma4Cfg {
+  static constexpr int TM = TM_, TN = TN_, NS = NS_;
+  static constexpr int BM = 16 * TM, BN = 32 * TN, BK = 128, WAVES = 8, THREADS = 64 * WAVES;
+  static constexpr int A_ROW = 2 * BK;                         // bytes of x per row and stage
+  static constexpr int A_INST = BM * A_ROW / 1024;             // copies of 4 rows
+  static constexpr int A_PW = (A_INST + WAVES - 1) / WAVES;    // ... per wavefront
+  static constexpr int B_ROW = BK / 2;                         // bytes of packed weights per row and stage
+  static constexpr int B_OFF = BM * A_ROW;
+  static constexpr int B_INST = BN * B_ROW / 1024;             // copies of 16 rows
+  static constexpr int B_PW = (B_INST + WAVES - 1) / WAVES;
+  static constexpr int S_OFF = B_OFF + BN * B_ROW;             // 4-byte scale slots [BN][2]: one per 64 k
+  static constexpr int S_INST = BN / 32;                       // copies of 32 columns
+  static constexpr int S_PW = (S_INST + WAVES - 1) / WAVES;
+  static constexpr int STAGE = S_OFF + BN * 8;
+  static constexpr int kDmaPerStage = A_PW + B_PW + S_PW;
+  static constexpr int OUT_ROW = BN * 2 + 16;
+  static constexpr int RED = 4 * TM * TN * 1024;               // two k-groups' partial tiles
+  static constexpr int OUT = BM * OUT_ROW;
+  static constexpr int SMEM = NS * STAGE > RED ? (NS * STAGE > OUT ? NS * STAGE : OUT) : (RED > OUT ? RED : OUT);
+  static_assert(BN % 64 == 0 && SMEM <= 160 * 1024, "tile");
+};
+
+template <class C>
+__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_dma4_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ packed,
+                      const half_t* __restrict__ scales, half_t* __restrict__ y, float* __restrict__ ws, int M, int N,
+                      int K, int log2_group, int stages_per_split, int splits, int tiles_m, int tiles_n,
+                      int group_m) {
+  constexpr int BM = C::BM, BN = C::BN, BK = C::BK, NS = C::NS, TM = C::TM, TN = C::TN, WAVES = C::WAVES;
+  constexpr int A_ROW = C::A_ROW, B_ROW = C::B_ROW, OUT_ROW = C::OUT_ROW;
+  extern __shared__ __attribute__((aligned(1024))) unsigned char dyn_smem[];
+  unsigned char* const smem = dyn_smem;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave & 1;
+  const int kw = wave >> 1;
+  const int g = lane >> 4;
+  const int l16 = lane & 15;
+
+  int split, t;
+  if (!gemm_job(tiles_m * tiles_n, splits, split, t)) return;
+  const int band = group_m * tiles_n;
+  const int bi = t / band;
+  const int tb = t - bi * band;
+  const int gm = min(group_m, tiles_m - bi * group_m);
+  const int m0 = (bi * group_m + tb % gm) * BM;
+  const int n0 = (tb / gm) * BN;
+
+  const int st_begin = split * stages_per_split;
+  const int ns = min(K / BK - st_begin, stages_per_split);  // >= 1: no split is empty
+
+  // x chunk c (16 bytes) of row r at slot c ^ (r & 15); packed chunk h at h ^ ((r >> 2) & 3).
+  const half_t* a_src[C::A_PW];
+  uint32_t a_dst[C::A_PW];
+#pragma unroll
+  for (int q = 0; q < C::A_PW; ++q) {
+    const int i = min(q * WAVES + wave, C::A_INST - 1);
+    const int row = 4 * i + (lane >> 4);
+    a_src[q] = x + (size_t)min(m0 + row, M - 1) * K + (size_t)st_begin * BK + 8 * ((lane & 15) ^ (row & 15));
+    a_dst[q] = 1024 * i;
+  }
+  const uint32_t* b_src[C::B_PW];
+  uint32_t b_dst[C::B_PW];
+#pragma unroll
+  for (int q = 0; q < C::B_PW; ++q) {
+    const int i = min(q * WAVES + wave, C::B_INST - 1);
+    const int row = 16 * i + (lane >> 2);
+    b_src[q] = packed + (size_t)min(n0 + row, N - 1) * (K >> 3) + (size_t)st_begin * (BK / 8) +
+               4 * ((lane & 3) ^ ((row >> 2) & 3));
+    b_dst[q] = C::B_OFF + 1024 * i;
+  }
+  const half_t* s_src[C::S_PW];
+  uint32_t s_dst[C::S_PW];
+#pragma unroll
+  for (int q = 0; q < C::S_PW; ++q) {
+    const int i = min(q * WAVES + wave, C::S_INST - 1);
+    s_src[q] = scales + (size_t)min(n0 + 32 * i + (lane >> 1), N - 1) * (K >> log2_group);
+    s_dst[q] = C::S_OFF + 256 * i;
+  }
+  const uint32_t smem_base = (uint32_t)(uintptr_t)smem;
+  auto issue = [&](int i, uint32_t slot) {  // split-local stage i (clamped) into the buffer at `slot`
+    const size_t st = min(i, ns - 1);
+    const uint32_t base = smem_base + slot;
+    const int group = ((st_begin + (int)st) * BK + 64 * (lane & 1)) >> log2_group;
+#pragma unroll
+    for (int q = 0; q < C::A_PW; ++q) dma_16B(__builtin_amdgcn_readfirstlane(base + a_dst[q]), a_src[q] + st * BK);
+#pragma unroll
+    for (int q = 0; q < C::B_PW; ++q)
+      dma_16B(__builtin_amdgcn_readfirstlane(base + b_dst[q]), b_src[q] + st * (BK / 8));
+#pragma unroll
+    for (int q = 0; q < C::S_PW; ++q)
+      dma_u16(__builtin_amdgcn_readfirstlane(base + s_dst[q]), s_src[q] + group);
+  };
+
+  float4_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+  // Lane offsets inside a stage: x row l16, chunk 4 kw + g; packed row of column 16 TN wn + l16, dword
+  // 4 kw + g; its scale for this k-group's 64 k.
+  const int a_off = l16 * A_ROW + 16 * ((4 * kw + g) ^ l16);
+  const int b_off = C::B_OFF + (16 * TN * wn + l16) * B_ROW + 16 * (kw ^ ((l16 >> 2) & 3)) + 4 * g;
+  const int s_off = C::S_OFF + 8 * (16 * TN * wn + l16) + 4 * (kw >> 1);
+  const UnpackConsts uc = unpack_consts();
+
+  // Stage s is copied NS - 1 iterations ahead.  At iteration s every wavefront reads its fragments
+  // of stage s, issues stage s + NS - 1 into the buffer of stage s - 1 (whose reads completed before
+  // the barrier of iteration s - 1), waits until its own copies of stage s + 1 have landed, and the
+  // barrier publishes them.
+  constexpr int kInFlight = (NS - 2) * C::kDmaPerStage;
+  static_assert(kInFlight <= 63, "vmcnt is six bits");
+#pragma unroll
+  for (int i = 0; i < NS - 1; ++i) issue(i, i * C::STAGE);
+  wait_vmcnt<kInFlight>();
+  __syncthreads();
+  uint32_t slot = 0, next = (NS - 1) * C::STAGE;
+#pragma unroll 1
+  for (int s = 0; s < ns; ++s) {
+    half8_t a[TM];
+    uint32_t w[TN];
+    half2_t s2[TN];
+    const unsigned char* st = smem + slot;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      w[j] = *reinterpret_cast<const uint32_t*>(st + b_off + 16 * B_ROW * j);
+      const half_t sc = *reinterpret_cast<const half_t*>(st + s_off + 128 * j);
+      s2[j] = half2_t{sc, sc};
+    }
+#pragma unroll
+    for (int q = 0; q < TM; ++q) a[q] = *reinterpret_cast<const half8_t*>(st + a_off + 16 * A_ROW * q);
+    issue(s + NS - 1, next);
+    next = slot;
+    slot = slot + C::STAGE == NS * C::STAGE ? 0 : slot + C::STAGE;
+    wait_vmcnt<kInFlight>();
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const half8_t b = dequant8(w[j], s2[j], uc);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b, a[i], acc[i][j], 0, 0, 0);
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the clamped tail copies, before LDS is reused
+  __syncthreads();
+
+  // The k-groups' partial tiles are added in fixed order through LDS: (a0 + a2) + (a1 + a3).  Round
+  // r hands k-group giver's tile to k-group taker through slot h (one 2 x wave-tile region per
+  // slot); straight-line code keeps acc in registers.
+  float* red = reinterpret_cast<float*>(smem);
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    const bool give = r ? kw == 1 : kw >= 2;
+    const bool take = r ? kw == 0 : kw < 2;
+    const int h = r ? 0 : (kw & 1);
+    float* base = red + ((h * 2 + wn) * TM * TN) * 256 + 4 * lane;
+    if (r > 0) __syncthreads();  // the first round's tiles have been read
+    if (give) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) *reinterpret_cast<float4_t*>(base + (i * TN + j) * 256) = acc[i][j];
+    }
+    __syncthreads();
+    if (take) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] += *reinterpret_cast<const float4_t*>(base + (i * TN + j) * 256);
+    }
+  }
+
+  if (ws) {
+    if (kw == 0) {
+      float* part = ws + (size_t)split * M * N;
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+          const int row = m0 + 16 * i + l16, col = n0 + 16 * TN * wn + 16 * j + 4 * g;
+          if (row < M && col < N) *reinterpret_cast<float4_t*>(part + (size_t)row * N + col) = acc[i][j];
+        }
+    }
+    return;
+  }
+  // fp16 tile through LDS, then 16-byte row-major stores by all wavefronts.
+  __syncthreads();  // the partial tiles have been read
+  if (kw == 0) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) {
+        const half2_t lo = {(half_t)acc[i][j][0], (half_t)acc[i][j][1]};
+        const half2_t hi = {(half_t)acc[i][j][2], (half_t)acc[i][j][3]};
+        *reinterpret_cast<u32x2*>(smem + (16 * i + l16) * OUT_ROW + 2 * (16 * TN * wn + 16 * j + 4 * g)) =
+            u32x2{bit_cast<uint32_t>(lo), bit_cast<uint32_t>(hi)};
+      }
+  }
+  __syncthreads();
+  for (int c = tid; c < BM * BN / 8; c += C::THREADS) {
+    const int row = c / (BN / 8), chunk = c % (BN / 8);
+    const int gr = m0 + row, gc = n0 + 8 * chunk;
+    if (gr < M && gc < N)
+      *reinterpret_cast<u32x4*>(y + (size_t)gr * N + gc) = *reinterpret_cast<const u32x4*>(smem + row * OUT_ROW + 16 * chunk);
+  }
+}
+
 // Wide DMA-fed tile: 192 x 256 per workgroup, 8 wavefronts as 2 x 4 wave tiles of 96 x 64, every
 // wavefront over the whole 64-k stage (no k split, no partial-tile reduction), one workgroup per
 // CU (99 KiB of stages and scale ring).  Per 64-k stage a CU moves 32 KiB from L2 into LDS for
-// 192 x 256 outputs, against 40 KiB for the two 128 x 128 tiles of gemm_dma_kernel<2> (half the
+// 192 x 256 outputs, against 40 KiB for the two 128 x 128 tiles of gemm_dma2_kernel (half the
 // outputs): x, fp16 and the larger operand, is re-read from L2 once per 256 columns instead of
 // once per 128.  Stage pipeline, swizzles, scale ring and counted waits are those of
-// gemm_dma_kernel<2>.  MI355X, M = 2048, N = 5632, K = 2048 (242 tiles, one per CU): 52 us = 906
+// gemm_dma2_kernel.  MI355X, M = 2048, N = 5632, K = 2048 (242 tiles, one per CU): 52 us = 906
 // TFLOPS against 56 us for the 128 x 128 tiles.  A tile alone on its CU takes 44 us (K = 2048), so
 // the tile pays only where its count fills whole rounds of 256; gemm_plan weighs that.
 struct WideCfg {
@@ -802,7 +693,7 @@ void gemm_wide_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__
   issue(0, 0);
   wait_older(issue(1, 1));
   __syncthreads();
-  // Stage pipeline of gemm_dma_kernel: stage i's fragments (both 32-k steps) are read at
+  // Stage pipeline of gemm_dma2_kernel: stage i's fragments (both 32-k steps) are read at
   // iteration i, before the barrier after which stage i + 2's DMA may overwrite stage i - 1's
   // buffer; the scheduling barrier keeps the next stage's reads out of this stage's MFMAs.
   auto step = [&](auto buf_c, int s) {
@@ -861,178 +752,247 @@ void gemm_wide_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__
   }
 }
 
-__global__ __launch_bounds__(256) void splitk_reduce(const float* __restrict__ ws, half_t* __restrict__ y,
-                                                      size_t mn, int splits) {
-  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < mn; i += (size_t)gridDim.x * 256) {
-    float s = 0.0f;
-    for (int z = 0; z < splits; ++z) s += ws[(size_t)z * mn + i];
-    y[i] = (half_t)s;
+// y = fp16(sum over the splits of their fp32 partials, in split order), four outputs per thread; the
+// partials of four splits are loaded together (one at a time, 4 bytes each, it took 2.4-5 us at
+// M N = 131,072 .. 409,600 and 5-8 splits; now 2.2-2.9).
+__global__ __launch_bounds__(256) void splitk_reduce(const float4_t* __restrict__ ws, u32x2* __restrict__ y, size_t mn4,
+                                                      int splits) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < mn4; i += (size_t)gridDim.x * 256) {
+    float4_t s = ws[i];
+    int z = 1;
+    for (; z + 3 < splits; z += 4) {
+      const float4_t p0 = ws[z * mn4 + i], p1 = ws[(z + 1) * mn4 + i], p2 = ws[(z + 2) * mn4 + i],
+                     p3 = ws[(z + 3) * mn4 + i];
+      s += p0;
+      s += p1;
+      s += p2;
+      s += p3;
+    }
+    for (; z < splits; ++z) s += ws[z * mn4 + i];
+    const half2_t lo = {(half_t)s[0], (half_t)s[1]}, hi = {(half_t)s[2], (half_t)s[3]};
+    y[i] = u32x2{bit_cast<uint32_t>(lo), bit_cast<uint32_t>(hi)};
   }
 }
 
 typedef void (*GemmFn)(const half_t*, const uint32_t*, const half_t*, half_t*, float*, int, int, int, int, int, int,
                        int, int, int);
 
-struct TileEntry {
-  int bm, bn, sk, threads;  // tile, k per stage, workgroup size
-  // Cost terms of the dispatcher (see gemm_plan): workgroups resident per CU, and the time of
-  // one round of resident workgroups, us_per_gmac * 1e-9 * BM * BN * k + us_fixed microseconds
-  // for k = the split's k range.  0 blocks_per_cu: never chosen by the cost model.
-  int blocks_per_cu;
-  double us_per_gmac, us_fixed;
+// A tile of a DMA kernel: its size, k per stage, workgroup and dynamic LDS.
+struct DmaEntry {
+  int bm, bn, bk, threads, lds;
   GemmFn fn;
 };
-
-template <class C>
-TileEntry entry(int blocks_per_cu, double us_per_gmac, double us_fixed) {
-  return TileEntry{C::BM, C::BN, C::SK, C::THREADS, blocks_per_cu, us_per_gmac, us_fixed, gemm_kernel<C>};
+template <int TM, int TN, int NS>
+constexpr DmaEntry dma4_entry() {
+  using C = Dma4Cfg<TM, TN, NS>;
+  return DmaEntry{C::BM, C::BN, C::BK, C::THREADS, C::SMEM, gemm_dma4_kernel<C>};
 }
-
-// Tile table: index = GemmPlan::tile.  Cost terms: weighted least-squares fit (relative error)
-// of the model in gemm_plan to graph-replayed timings of every tile and split count 1..12 over
-// the TinyLlama and Qwen2.5 layer shapes, M = 48 .. 4096, weights rotated through more than
-// twice the MALL, on MI355X (4,172 points, rms error 7.7%).  Over those shapes the plan's
-// choices take 1.0074x the time of the best measured (tile, split) per shape (1.0122x without
-// the 192 x 256 tile).
-const TileEntry kTiles[] = {
-    entry<TileCfg<64, 128, 1, 4, 1>>(0, 0.0, 0.0),         // 0: 64 x 128, 4 waves; 64-k stages (any K)
-    entry<TileCfg<64, 128, 1, 4, 2>>(1, 702.21, 2.867),    // 1: 64 x 128, 8 waves (2 k-groups)
-    TileEntry{128, 128, DmaCfg<2>::BK, DmaCfg<2>::THREADS, 2, 557.73, 5.918, gemm_dma_kernel<2>},  // 2: DMA 128 x 128
-    entry<TileCfg<32, 128, 1, 4, 2>>(1, 999.91, 1.977),    // 3: 32 x 128, 8 waves (2 k-groups)
-    entry<TileCfg<32, 64, 1, 2, 4>>(1, 1081.97, 2.779),    // 4: 32 x 64, 8 waves (4 k-groups, 256-k stages)
-    entry<TileCfg<16, 64, 1, 2, 4>>(1, 1831.66, 2.117),    // 5: 16 x 64, 8 waves (4 k-groups, 256-k stages)
-    TileEntry{128, 128, DmaCfg<4>::BK, DmaCfg<4>::THREADS, 1, 388.59, 7.265, gemm_dma_kernel<4>},  // 6: DMA, 8 waves
-    TileEntry{192, 256, WideCfg::BK, WideCfg::THREADS, 1, 387.22, 4.351, gemm_wide_kernel},  // 7: DMA 192 x 256
+const DmaEntry kDma[] = {
+    dma4_entry<2, 4, 4>(), dma4_entry<3, 4, 4>(), dma4_entry<4, 4, 3>(),
+    dma4_entry<5, 4, 3>(), dma4_entry<7, 4, 3>(), dma4_entry<8, 4, 3>(),
+    DmaEntry{128, 128, DmaCfg::BK, DmaCfg::THREADS, 0, gemm_dma2_kernel},
+    DmaEntry{192, 256, WideCfg::BK, WideCfg::THREADS, 0, gemm_wide_kernel},
 };
-constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
-constexpr int kTile64 = 0, kDmaTile = 2, kWideTile = 7;
-// Split-K costs one more launch plus the fp32 partials: kSplitUs + kSplitUsPerElem * splits * M * N
-// (same fit), and is taken only when the model predicts it at least 10% faster.
-constexpr double kSplitUs = 4.352, kSplitUsPerElem = 1.3750e-6, kSplitMargin = 0.9;
-constexpr int kMaxSplits = 12;  // the largest split count the fit was measured on
+constexpr int kNumDma = sizeof(kDma) / sizeof(kDma[0]);
 
-GemmPlan plan_for(int K, int tile, int splits) {
-  GemmPlan p;
-  p.skinny = false;
-  p.sk = SkinnyPlan{0, 0, 0, false, 0, 1};
-  p.tile = tile;
-  p.block_m = kTiles[tile].bm;
-  p.block_n = kTiles[tile].bn;
-  const int nst = K / kTiles[tile].sk;
+}  // namespace
+
+int gemm_num_configs() { return stream_num_configs() + kNumDma; }
+
+// Plan with an explicit configuration (streaming tiles first, then kDma) and split count.
+GemmPlan gemm_plan_with(int cfg, int splits, int K) {
+  GemmPlan p = {};
+  p.cfg = cfg;
+  if (cfg < stream_num_configs()) {
+    const StreamTile t = stream_tile_of(cfg);
+    p.block_m = t.bm;
+    p.block_n = t.bn;
+    p.threads = 64 * t.ks;
+    p.splits = splits;  // the kernel balances the 64-k pieces over them
+    return p;
+  }
+  const DmaEntry& e = kDma[cfg - stream_num_configs()];
+  p.block_m = e.bm;
+  p.block_n = e.bn;
+  p.threads = e.threads;
+  const int nst = K / e.bk;
   p.kt_per_split = ceil_div(nst, splits);
   p.splits = ceil_div(nst, p.kt_per_split);  // no empty splits
   return p;
 }
 
+namespace {
+
+// Cost of a configuration, in microseconds (see gemm_plan): workgroups resident per CU, and the
+// coefficients of 1, w, w k, k, r k and the weight's size, where w = workgroups of the busiest CU, r =
+// rounds of resident workgroups, k = thousands of K per split.  Weighted least squares (relative
+// error, no negative terms) over graph-replayed timings of every configuration and split count on
+// 685 (M, N, K) points: the TinyLlama, Qwen2.5 and hidden-4096 layer shapes and other sizes, N = 64 ..
+// 28672, K = 384 .. 14336, M = 6 .. 2048, weights rotated through more than the MALL, on MI355X
+// (rms error 5.9%).  Over those points the plan takes 1.014x the time of the best configuration measured.
+struct CostTerms {
+  int resident;
+  double c[6];
+};
+const CostTerms kCost[] = {
+    {2, {2.129, 0.7869, 0.1713, 0.02396, 0.3003, 0.04607}},  // 8 x 16, 8 wavefronts
+    {2, {2.143, 0.7569, 0.2216, 0, 0.3414, 0.05218}},  // 16 x 16, 8 wavefronts
+    {1, {1.162, 1.967, 0, 0.08763, 0.6969, 0.05839}},  // 16 x 32, 8 wavefronts
+    {1, {1.363, 1.95, 1.486, 0.07655, 0, 0.05032}},  // 16 x 64, 8 wavefronts
+    {1, {1.004, 2.048, 0.4376, 0.1616, 0, 0.07321}},  // 24 x 16, 8 wavefronts
+    {1, {1.223, 1.762, 0.7307, 0, 0, 0.05263}},  // 32 x 16, 8 wavefronts
+    {1, {1.208, 2.044, 1.037, 0.004844, 0, 0.05858}},  // 32 x 32, 8 wavefronts
+    {1, {1.311, 2.252, 1.366, 0.04656, 0, 0.05716}},  // 32 x 48, 8 wavefronts
+    {1, {1.295, 1.864, 0.867, 0, 0, 0.06072}},  // 48 x 16, 8 wavefronts
+    {1, {1.302, 2.157, 1.21, 0, 0, 0.06888}},  // 48 x 32, 8 wavefronts
+    {1, {1.481, 2.409, 1.656, 0, 0, 0.06151}},  // 48 x 48, 8 wavefronts
+    {3, {2.394, 0.4783, 0.6288, 0, 0.7739, 0.0546}},  // 32 x 32, 4 wavefronts
+    {2, {2.722, 0.8287, 1.052, 0, 0.9426, 0.05652}},  // 48 x 48, 4 wavefronts
+    {2, {2.397, 0.8561, 0.9821, 0, 0.8571, 0.06422}},  // 64 x 32, 4 wavefronts
+    {1, {1.425, 2.497, 2.208, 0, 0, 0.05632}},  // 64 x 48, 4 wavefronts
+    {1, {1.376, 2.837, 2.713, 0.05566, 0, 0.05154}},  // 64 x 64, 4 wavefronts
+    {4, {2.31, 0.362, 0.2047, 0, 0.3752, 0.05386}},  // 8 x 16, 4 wavefronts
+    {3, {2.172, 0.3817, 0.1033, 0, 0.804, 0.07325}},  // 16 x 16, 4 wavefronts
+    {2, {2.526, 1.187, 2.55, 0, 0.741, 0.07091}},  // 32 x 128, 8 wavefronts
+    {1, {1.142, 3.062, 3.798, 0, 0, 0.06154}},  // 48 x 128, 8 wavefronts
+    {2, {2.393, 1.985, 3.469, 0, 0.7973, 0.06033}},  // 64 x 128, 8 wavefronts
+    {1, {0.6948, 4.308, 4.743, 0, 0, 0.06921}},  // 80 x 128, 8 wavefronts
+    {1, {0.7089, 4.945, 6.034, 0, 0, 0.07693}},  // 112 x 128, 8 wavefronts
+    {1, {0.5876, 5.629, 6.673, 0, 0, 0.0669}},  // 128 x 128, 8 wavefronts
+    {2, {3.084, 1.742, 3.432, 0, 5.492, 0.06297}},  // 128 x 128, 4 wavefronts
+    {1, {0, 5.689, 17.9, 0, 0, 0.2662}},  // 192 x 256, 8 wavefronts
+};
+// Split-K costs one more launch plus the fp32 partials (same fit), and is taken only when the
+// model predicts it at least 3% faster.
+constexpr double kSplitUs = 2.324, kSplitUsPerMElem = 1.624, kSplitMargin = 1.03;
+// Layers much deeper than wide (K >= 4096, K >= 2.5 N) are split unless the model puts the split more
+// than 1 / 0.78 behind: there the model is too careful as often as not, and these layers' plans have
+// always asked for a workspace, which callers of the workspace entry points are written against.
+// Best unsplit / best split (us): 4096 x 14336 at M = 160: 45.1 / 34.3; 1536 x 8960 at M = 517: 33.0 /
+// 28.3; 640 x 8960 at M = 64: 9.5 / 7.9; 1536 x 8960 at M = 27: 9.0 / 9.7; the worst, 2048 x 5632 at
+// M = 64: 7.9 / 9.5 (11.6 with the kernels before).
+constexpr double kDeepSplitMargin = 0.78;
+constexpr int kMaxSplits = 8;        // the largest split count the fit was measured on
+constexpr int kMinSplitK = 512;      // k per split
+constexpr size_t kMaxSplitBytes = 32u << 20;  // partials of a plan; see gemm_plan
+
 }  // namespace
 
-int gemm_num_tiles() { return kNumTiles; }
+int gemm_num_families() { return 7; }
 
-GemmPlan gemm_plan_with_tile(int M, int N, int K, int cu_count, int tile) {
-  if (K % kTiles[tile].sk != 0) tile = kTile64;  // its 64-k stage divides every K here
-  const int nst = K / kTiles[tile].sk;
-  const long tiles = (long)ceil_div(N, kTiles[tile].bn) * ceil_div(M, kTiles[tile].bm);
-  const long want = cu_count > 0 ? cu_count : 256;
-  int splits = 1;
-  if (tiles < want) {
-    splits = (int)((want + tiles - 1) / tiles);
-    const int max_splits = nst / 4 > 0 ? nst / 4 : 1;  // at least 4 stages per split
-    if (splits > max_splits) splits = max_splits;
-    if (splits < 1) splits = 1;
+// Kernel family reported for a configuration: streaming tiles at M <= 32 (-1), with K over 4 wavefronts
+// (0), over 8 with up to 24 rows (1), 32 rows (5) or 48 (2); DMA tiles of up to 64 rows (3), of 80 to
+// 128 rows (6); 192 x 256 (4).
+static int family_of(int cfg, int M) {
+  if (cfg < stream_num_configs()) {
+    const StreamTile t = stream_tile_of(cfg);
+    return M <= 32 ? -1 : (t.ks == 4 ? 0 : (t.bm <= 24 ? 1 : (t.bm == 32 ? 5 : 2)));
   }
-  return plan_for(K, tile, splits);
+  const int bm = kDma[cfg - stream_num_configs()].bm;
+  return bm == 192 ? 4 : (bm <= 64 ? 3 : 6);
 }
 
-// Kernel choice.
-//   * The skinny kernel (one weight stream, K split inside the workgroup) for M <= 8, for
-//     M <= 16 when K <= 4096, and up to M = 32 for small matrices (N*K <= 4.2M: TinyLlama q/o
-//     and k/v) or grids of at most one workgroup per CU (TinyLlama gate/up, whose workgroups
-//     take two column blocks, M = 20..32: 7.3 -> 6.0-7.0 us; q|k|v fused 7.1 -> 5.1-6.0 us; Qwen2.5
-//     gate/up at 560 workgroups and TinyLlama gate|up fused at 704 stay faster tiled).  The rule
-//     depends on N only through those last two clauses, so concatenated q|k|v or gate|up rows
-//     take the same kernel as the separate layers for M <= 16 (bit-identical columns).
-//   * Otherwise the tile and split-K factor that minimise a fitted cost: each XCD runs its
-//     share of the tiles x splits workgroups in rounds of blocks_per_cu * cu_count / 8; a round
-//     costs the tile entry's us_per_gmac * 1e-9 * BM * BN * (K / splits) + us_fixed, and
-//     splitting adds its own cost (see kSplitUs).  Measured effect: small tiles (16 x 64,
-//     32 x 64) at medium M and for narrow N (k/v projections), the DMA tile once it fills the
-//     GPU, split-K only for long K.
+// Modelled time of `tiles` workgroups of a configuration per split.  Each XCD runs its share of the
+// workgroups, spread over its CUs.
+static double plan_cost(int cfg, long tiles, int splits, int M, double n, int K, int cus) {
+  const CostTerms& t = kCost[cfg];
+  const int cus_per_xcd = std::max(1, cus / kXcds);
+  const long per_cu = (((tiles * splits + kXcds - 1) / kXcds) + cus_per_xcd - 1) / cus_per_xcd;
+  const long rounds = (per_cu + t.resident - 1) / t.resident;
+  const double k = K * 1e-3 / splits;
+  const double cost =
+      t.c[0] + (t.c[1] + t.c[2] * k) * per_cu + (t.c[3] + t.c[4] * rounds) * k + t.c[5] * n * K * 1e-6;
+  return splits == 1 ? cost : (cost + kSplitUs + kSplitUsPerMElem * 1e-6 * splits * (double)M * n) *
+                                  (K >= 4096 && K >= 2.5 * n ? kDeepSplitMargin : kSplitMargin);
+}
+
+// At M <= 16 the K split over wavefronts depends on M and K alone (see gemm_plan).  Four wavefronts
+// leave room for more workgroups per CU, which wide layers want; eight shorten a long K.  Best tile
+// with 4 / 8 (us): 17920 x 1536 at M = 6 / 16: 8.6 / 10.2 and 9.6 / 12.1; 11264 x 2048: 6.3 / 7.4 and
+// 7.1 / 7.2; 2560 x 2048: 4.1 / 4.1 and 4.7 / 4.4; 28672 x 4096: 19.6 / 22.3 and 25.1 / 23.9; 4096 x
+// 4096: 5.8 / 5.4 and 7.2 / 5.9; 4096 x 14336: 13.2 / 12.0 and 17.8 / 14.1.
+static int small_m_waves(int M, int K) { return K < 2048 || (M <= 8 && K <= 4096) ? 4 : 8; }
+
+// Kernel choice: the configuration and split-K factor with the smallest modelled time.
+//   * M <= 16: streaming tiles of small_m_waves(M, K) wavefronts without split-K only, so the K split
+//     (and with it every bit of a column) does not depend on N and concatenated q|k|v or gate|up rows
+//     give the separate layers' results.
+//   * Partials of a split are held to the scratch of kf_int4_gemm_noalloc, so that entry point takes
+//     every shape, except where K >= 16384: there a few tiles may need more splits than that.
 GemmPlan gemm_plan(int M, int N, int K, int cu_count) {
+  static_assert(sizeof(kCost) / sizeof(kCost[0]) == kNumStreamConfigs + kNumDma, "one cost entry per configuration");
   const int cus = cu_count > 0 ? cu_count : 256;
-  const bool k128 = K % 128 == 0;
-  const bool one_round = (long)ceil_div(N, 16 * skinny_col_blocks(N, cus)) <= cus;
-  if (M <= kSkinnyMaxM && k128 && (M <= 8 || (K <= 4096 && (M <= 16 || (long)N * K <= 4200000L || one_round)))) {
-    GemmPlan p = plan_for(K, kTile64, 1);
-    p.skinny = true;
-    p.sk = skinny_plan(M, N, K, cu_count);
-    return p;
-  }
-  if (!k128) {  // K % 64 == 0 only: the 64-k-stage kernels
-    const long dma_tiles = (long)ceil_div(M, 128) * ceil_div(N, 128);
-    return gemm_plan_with_tile(M, N, K, cu_count, dma_tiles >= cus ? kDmaTile : kTile64);
-  }
-  int best_tile = kDmaTile, best_splits = 1;
+  const int num_stream = stream_num_configs();
+  int best_cfg = -1, best_splits = 1;
   double best = 1e300;
-  for (int tile = 0; tile < kNumTiles; ++tile) {
-    const TileEntry& e = kTiles[tile];
-    if (e.blocks_per_cu == 0 || K % e.sk != 0) continue;
-    const int nst = K / e.sk;
-    const long tiles = (long)ceil_div(M, e.bm) * ceil_div(N, e.bn);
-    // >= 4 stages per split; the 192 x 256 tile never splits (its kernel writes no partials)
-    const int max_splits = tile == kWideTile ? 1 : std::min(kMaxSplits, std::max(1, nst / 4));
-    int prev = 0;
+  for (int cfg = 0; cfg < gemm_num_configs(); ++cfg) {
+    int bm, bn, threads;
+    if (cfg < num_stream) {
+      const StreamTile t = stream_tile_of(cfg);
+      bm = t.bm, bn = t.bn, threads = 64 * t.ks;
+      if (M <= 16 && t.ks != small_m_waves(M, K)) continue;
+    } else {
+      const DmaEntry& e = kDma[cfg - num_stream];
+      bm = e.bm, bn = e.bn, threads = e.threads;
+      if (M <= 16 || K % e.bk || (cfg == gemm_num_configs() - 1 && K % 128)) continue;
+    }
+    const long tiles = (long)ceil_div(M, bm) * ceil_div(N, bn);
+    if ((tiles + kXcds) * threads > 0x7FFFFFFFL) continue;
+    // The 192 x 256 tile writes no partials; more splits than two rounds of workgroups never pay.
+    const bool can_split = M > 16 && tiles < 2 * cus && cfg != gemm_num_configs() - 1;
+    const int max_splits = can_split ? std::min(kMaxSplits, std::max(1, K / kMinSplitK)) : 1;
     for (int s = 1; s <= max_splits; ++s) {
-      const int splits = ceil_div(nst, ceil_div(nst, s));
-      if (splits == prev) continue;
-      prev = splits;
-      // Jobs are dealt evenly to the XCDs (gemm_job); each XCD runs its share in rounds.
-      const long per_xcd = (tiles * splits + kXcds - 1) / kXcds;
-      const long slots = std::max(1L, (long)e.blocks_per_cu * cus / kXcds);
-      const long rounds = (per_xcd + slots - 1) / slots;
-      double cost = rounds * (e.us_per_gmac * 1e-9 * e.bm * e.bn * ((double)K / splits) + e.us_fixed);
-      if (splits > 1) cost = (cost + kSplitUs + kSplitUsPerElem * splits * (double)M * N) / kSplitMargin;
+      if (s > 1 && K < 16384 && (size_t)s * M * N * sizeof(float) > kMaxSplitBytes) break;
+      const double cost = plan_cost(cfg, tiles, s, M, N, K, cus);
       if (cost < best) {
         best = cost;
-        best_tile = tile;
-        best_splits = splits;
+        best_cfg = cfg;
+        best_splits = s;
       }
     }
   }
-  return plan_for(K, best_tile, best_splits);
+  if (best_cfg < 0) best_cfg = num_stream;  // past every grid limit; the caller's check refuses it
+  GemmPlan p = gemm_plan_with(best_cfg, best_splits, K);
+  p.family = family_of(best_cfg, M);
+  return p;
 }
 
 size_t gemm_workspace_bytes(const GemmPlan& p, int M, int N) {
-  return !p.skinny && p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
+  return p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
 }
 
 hipError_t gemm_launch(const GemmPlan& p, const void* x, const void* packed, const void* scales, void* y,
-                       void* ws, int M, int N, int K, int group_size, hipStream_t stream, const void* packed_r,
-                       const void* scales_r) {
-  if (p.skinny) {
-    const bool blocked = packed_r != nullptr && scales_r != nullptr;
-    return skinny_launch(p.sk, x, blocked ? packed_r : packed, blocked ? scales_r : scales, y, M, N, K, group_size,
-                         blocked, stream);
-  }
-  const TileEntry& e = kTiles[p.tile];
-  const int log2_group = group_size == 128 ? 7 : 6;
-  const int tiles_m = ceil_div(M, e.bm);
-  const int tiles_n = ceil_div(N, e.bn);
-  const int grid_x = ceil_div(tiles_m * tiles_n * p.splits, kXcds) * kXcds;
-  // Bands of M-tiles: one band per XCD when the M-tiles divide evenly, else single rows.
-  int group_m = tiles_m / kXcds;
-  if (group_m < 1) group_m = 1;
+                       void* ws, int M, int N, int K, int group_size, hipStream_t stream) {
   float* part = p.splits > 1 ? static_cast<float*>(ws) : nullptr;
-  hipLaunchKernelGGL(e.fn, dim3(grid_x), dim3(e.threads), 0, stream, static_cast<const half_t*>(x),
-                     static_cast<const uint32_t*>(packed), static_cast<const half_t*>(scales),
-                     static_cast<half_t*>(y), part, M, N, K, log2_group, p.kt_per_split, p.splits, tiles_m, tiles_n,
-                     group_m);
-  hipError_t err = hipGetLastError();
+  hipError_t err;
+  if (p.cfg < stream_num_configs()) {
+    err = stream_launch(p.cfg, p.splits, x, packed, scales, y, part, M, N, K, group_size, stream);
+  } else {
+    const DmaEntry& e = kDma[p.cfg - stream_num_configs()];
+    const int log2_group = group_size == 128 ? 7 : 6;
+    const int tiles_m = ceil_div(M, e.bm);
+    const int tiles_n = ceil_div(N, e.bn);
+    const int grid_x = ceil_div(tiles_m * tiles_n * p.splits, kXcds) * kXcds;
+    // Bands of M-tiles: one band per XCD when the M-tiles divide evenly, else single rows.
+    int group_m = tiles_m / kXcds;
+    if (group_m < 1) group_m = 1;
+    if (e.lds > 65536) {  // dynamic LDS beyond 64 KiB is opted into per kernel
+      err = hipFuncSetAttribute(reinterpret_cast<const void*>(e.fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                kLdsPerCu);
+      if (err != hipSuccess) return err;
+    }
+    hipLaunchKernelGGL(e.fn, dim3(grid_x), dim3(e.threads), e.lds, stream, static_cast<const half_t*>(x),
+                       static_cast<const uint32_t*>(packed), static_cast<const half_t*>(scales),
+                       static_cast<half_t*>(y), part, M, N, K, log2_group, p.kt_per_split, p.splits, tiles_m, tiles_n,
+                       group_m);
+    err = hipGetLastError();
+  }
   if (err != hipSuccess || p.splits == 1) return err;
-  const size_t mn = (size_t)M * N;
-  size_t blocks = (mn + 255) / 256;
+  const size_t mn4 = (size_t)M * N / 4;  // N % 64 == 0
+  size_t blocks = (mn4 + 255) / 256;
   if (blocks > 4096) blocks = 4096;
-  hipLaunchKernelGGL(splitk_reduce, dim3((unsigned)blocks), dim3(256), 0, stream, static_cast<const float*>(ws),
-                     static_cast<half_t*>(y), mn, p.splits);
+  hipLaunchKernelGGL(splitk_reduce, dim3((unsigned)blocks), dim3(256), 0, stream, static_cast<const float4_t*>(ws),
+                     static_cast<u32x2*>(y), mn4, p.splits);
   return hipGetLastError();
 }
 

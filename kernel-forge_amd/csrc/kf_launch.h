@@ -134,24 +134,20 @@ struct GemvRope {
 hipError_t gemv_qkv_rope_launch(const GemvProblem& problem, const GemvFused& f, const GemvRope& rope, int unroll,
                                 int group_size, hipStream_t stream);
 
-// ---- skinny MFMA GEMM (M <= 32, K % 128 == 0): one weight stream, K split in-block ----
-// gemm_plan (kf_gemm.hip) picks it for small M by the measured rule stated there.
-constexpr int kSkinnyMaxM = 32;
-struct SkinnyPlan {
-  int m_tiles;    // 16-row tiles of M (1..2)
-  int ks_waves;   // wavefronts per workgroup, each a contiguous run of 128-k super-steps
-  int unroll;     // super-steps whose weight loads are in flight together
-  bool x_lds;     // x fragments from each wavefront's LDS copy of its k range (else from L2)
-  int lds_bytes;  // dynamic LDS per workgroup
-  int col_blocks; // 16-column blocks per workgroup (1..2)
+// ---- streaming GEMM tiles (kf_stream.hip): small and medium M, N % 64 == 0 --------------------
+struct StreamTile {
+  int bm, bn;  // output tile
+  int ks;      // wavefronts, which split K
+  int lds;     // bytes per workgroup
 };
-constexpr int kSkinnyMaxLds = 160 * 1024;  // LDS of a gfx950 CU
-SkinnyPlan skinny_plan(int M, int N, int K, int cu_count);
-// 16-column blocks per skinny workgroup for N on cu_count CUs (SkinnyPlan::col_blocks).
-int skinny_col_blocks(int N, int cu_count);
-hipError_t skinny_launch(const SkinnyPlan& p, const void* x, const void* packed, const void* scales, void* y, int M,
-                         int N, int K, int group_size, bool blocked, hipStream_t stream);
-// MFMA-16 block copy of packed / scales (kf_skinny.hip): sizes in int32 words and fp16 scales.
+constexpr int kNumStreamConfigs = 18;
+inline int stream_num_configs() { return kNumStreamConfigs; }
+StreamTile stream_tile_of(int cfg);
+// part: splits x M x N fp32 partials when splits > 1 (the caller reduces them), else unused.
+hipError_t stream_launch(int cfg, int splits, const void* x, const void* packed, const void* scales, void* y,
+                         float* part, int M, int N, int K, int group_size, hipStream_t stream);
+
+// ---- MFMA-16 block copy of packed / scales (kf_aux.hip): sizes in int32 words and fp16 scales --
 size_t mfma16_packed_words(int N, int K);
 size_t mfma16_scale_count(int N, int K, int group_size);
 hipError_t reorder_mfma16_launch(const void* packed, const void* scales, void* packed_r, void* scales_r, int N, int K,
@@ -159,24 +155,22 @@ hipError_t reorder_mfma16_launch(const void* packed, const void* scales, void* p
 
 // ---- MFMA GEMM (any M, N % 64 == 0) --------------------------------------
 struct GemmPlan {
-  bool skinny;     // true: the skinny kernel (fields below unused except sk)
-  SkinnyPlan sk;
-  int tile;        // index into the tile table (kf_gemm.hip)
-  int block_m;     // BM
-  int block_n;     // BN
+  int cfg;         // configuration: streaming tiles first, then the DMA tiles (kf_gemm.hip)
+  int family;      // kernel family reported by kf_int4_gemm_plan (-1: streaming tiles at M <= 32)
+  int block_m;     // output tile
+  int block_n;
+  int threads;     // workgroup size
   int splits;      // split-K factor (1 = no workspace)
-  int kt_per_split;// k stages (of the tile's stage depth) per split
+  int kt_per_split;// k stages per split (DMA tiles)
 };
 GemmPlan gemm_plan(int M, int N, int K, int cu_count);
-// Plan with an explicit tile-table entry and the fill-the-CUs split rule (the K % 128 != 0
-// fallback of gemm_plan, and tuning).
-GemmPlan gemm_plan_with_tile(int M, int N, int K, int cu_count, int tile);
-int gemm_num_tiles();
+// Plan with an explicit configuration and split count (tuning).
+GemmPlan gemm_plan_with(int cfg, int splits, int K);
+int gemm_num_configs();
+int gemm_num_families();
 size_t gemm_workspace_bytes(const GemmPlan& p, int M, int N);
-// packed_r / scales_r: the MFMA-16 block copy, read where the skinny kernel runs (may be null).
 hipError_t gemm_launch(const GemmPlan& p, const void* x, const void* packed, const void* scales, void* y,
-                       void* ws, int M, int N, int K, int group_size, hipStream_t stream,
-                       const void* packed_r = nullptr, const void* scales_r = nullptr);
+                       void* ws, int M, int N, int K, int group_size, hipStream_t stream);
 
 // ---- on-device quantize + pack (kf_quant.hip) -------------------------------
 constexpr int kQuantF32 = 0, kQuantF16 = 1, kQuantBF16 = 2;  // == KF_DTYPE_* of the C ABI
@@ -192,7 +186,6 @@ hipError_t bw_read_store_launch(const void* src, void* out, size_t bytes, int gr
 hipError_t bw_write_launch(void* dst, size_t bytes, int grid, hipStream_t stream);
 hipError_t decode_argmax_launch(const void* logits, int n, void* token, void* pos, void* history, int max_seq,
                                 void* mask, hipStream_t stream);
-
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 }  // namespace kf

@@ -25,7 +25,7 @@ from kernelforge import _lib
 # Measured GEMV/GEMM crossover on one MI355X (dispatch_sweep.py beside bench.py): the
 # largest M at which the sum of GEMV times over the layer shapes beats the GEMM's
 # (reference rule, bench/sweep_int4_dispatch.py:51-57).  Above it int4_gemm runs the
-# skinny MFMA kernel for small M, then the tiled MFMA kernels.
+# streaming MFMA kernel for small and medium M, then the LDS-DMA tiles.
 GEMV_MAX_M = 4
 # The reference's int4_matmul sends M <= 7 to its GEMV, which accepts every N, and M >= 8
 # to its GEMM, which rejects N % 64 != 0 (kernelforge/ops.py:193,204-214).  Our MFMA kernels
@@ -151,14 +151,13 @@ def _launch_gemv(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, gr
     return y
 
 
-# The MFMA-16 block copy of a weight (kf_int4_reorder_mfma16) makes the skinny MFMA kernel's
-# weight loads contiguous (7-15% faster at M <= 32) and is bit-identical in results, at the cost
-# of a second copy of the weight in device memory (0.74x the INT4 weights of a TinyLlama whose
-# layers all run the skinny kernel once) and one host wait when it is built.  Opt-in, two ways:
-# prepare_mfma16(packed, scales) attaches a copy to one weight, which int4_gemm then reads
-# whenever it runs the skinny kernel on it; MFMA16_CACHE = True makes int4_gemm build and attach
-# one by itself the first time any weight runs the skinny kernel at M <= MFMA16_MAX_M (outside
-# HIP-graph capture).  Off, the skinny kernel reads the public layout.
+# The MFMA-16 block copy of a weight (kf_int4_reorder_mfma16): the weight in MFMA fragment order, a
+# second copy in device memory and one host wait when it is built.  The streaming kernels read the
+# public layout through LDS in whole lines, faster than fragment-order loads of this copy were (see
+# csrc/kf_stream.hip), so kf_int4_gemm_mfma16 checks the copy and runs the same kernels.  Kept for
+# programs that use it: prepare_mfma16(packed, scales) attaches a copy to one weight, which int4_gemm
+# passes along at M <= MFMA16_MAX_M; MFMA16_CACHE = True makes int4_gemm build and attach one by itself
+# the first time a weight runs a "skinny" plan at M <= MFMA16_MAX_M (outside HIP-graph capture).
 MFMA16_CACHE = False
 MFMA16_MAX_M = 32
 _MFMA16_ATTR = "_kf_mfma16"
@@ -168,7 +167,7 @@ def int4_reorder_mfma16(packed: torch.Tensor, scales: torch.Tensor,
                         group_size: int = 128) -> tuple[torch.Tensor, torch.Tensor]:
     """The MFMA-16 block copy (packed_r int32, scales_r fp16) of a packed weight; K % 128 == 0.
 
-    An internal layout (the public packed format is unchanged); kernel csrc/kf_skinny.hip.
+    An internal layout (the public packed format is unchanged); kernel csrc/kf_aux.hip.
     """
     if packed.dtype != torch.int32 or scales.dtype != torch.float16 or not packed.is_cuda:
         raise TypeError("int4_reorder_mfma16 expects int32 packed and fp16 scales on a CUDA device")
@@ -196,13 +195,12 @@ def _mfma16_key(packed: torch.Tensor, scales: torch.Tensor, group_size: int) -> 
 def prepare_mfma16(packed: torch.Tensor, scales: torch.Tensor, group_size: int = 128) -> None:
     """Builds the MFMA-16 copy of a weight now and keeps it on `packed` for int4_gemm.
 
-    The per-weight opt-in: int4_gemm reads the copy whenever it runs the skinny kernel on this
-    weight (with MFMA16_CACHE on it would build one by itself on first use, except for tensors
+    The per-weight opt-in: int4_gemm passes the copy along at M <= MFMA16_MAX_M (with MFMA16_CACHE on it would build one by itself on first use, except for tensors
     created under torch.inference_mode(), which have no version counter to notice in-place
     updates: for those this is the only way, and the caller promises not to modify packed /
     scales in place afterwards).  An in-place update of a weight with version counters makes
     int4_gemm ignore the stale copy.  Not during HIP-graph capture.  The host waits for the copy
-    to be written before it is attached, so a later int4_gemm on any stream reads a complete copy.
+    to be written before it is attached, so a later int4_gemm on any stream sees a complete copy.
     """
     if torch.cuda.is_current_stream_capturing():
         raise RuntimeError("prepare_mfma16 launches a kernel and allocates; call it outside HIP-graph capture")
@@ -227,7 +225,7 @@ def _mfma16_copy(packed: torch.Tensor, scales: torch.Tensor, group_size: int, m:
     if not MFMA16_CACHE or key[3] is None or torch.cuda.is_current_stream_capturing():
         return None  # inference tensors: only a copy made by prepare_mfma16
     if gemm_plan(m, packed.shape[0], packed.shape[1] * 8, group_size, packed.device)["kernel"] != "skinny":
-        return None  # only the skinny kernel reads the copy
+        return None  # copies are built for small-M plans only
     prepare_mfma16(packed, scales, group_size)
     cached = getattr(packed, _MFMA16_ATTR)
     return cached[1], cached[2]
@@ -236,7 +234,7 @@ def _mfma16_copy(packed: torch.Tensor, scales: torch.Tensor, group_size: int, m:
 def int4_gemm(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, group_size: int = 128) -> torch.Tensor:
     """Fused INT4 dequant GEMM on the MFMA matrix cores, any M, N a multiple of 64.
 
-    Reference kernelforge/ops.py:196-201; kernels csrc/kf_gemm.hip, csrc/kf_skinny.hip.
+    Reference kernelforge/ops.py:196-201; kernels csrc/kf_stream.hip, csrc/kf_gemm.hip.
     """
     _check_int4(x, packed, scales, group_size)
     if packed.shape[0] % 64 != 0:
@@ -273,8 +271,8 @@ def _launch_gemm(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, gr
 def gemm_plan(m: int, n: int, k: int, group_size: int = 128, device: torch.device | None = None) -> dict:
     """The kernel int4_gemm runs for an [m, k] x [n, k]^T problem on `device` (default: current).
 
-    Returns {"kernel": "skinny" or the tile-table index, "num_kernels": table size,
-    "splits": split-K factor, "tile": (BM, BN)}.  Diagnostics; no reference counterpart.
+    Returns {"kernel": "skinny" (a streaming tile at M <= 32) or the kernel family's index,
+    "num_kernels": families, "splits": split-K factor, "tile": (BM, BN)}.  Diagnostics; no reference counterpart.
     """
     lib = _lib.load()
     out = [ctypes.c_int() for _ in range(5)]

@@ -9,7 +9,7 @@ kernelforge/modules.py:51-65); embedding and lm_head stay fp16.
 
 ``fuse_decoder_linears_`` replaces q|k|v and gate|up by one INT4 module each whose packed rows are
 the concatenation of the originals (the packed format is per row, so this is the same format).
-For M <= 16 (decode and short prompts: the GEMV and the skinny kernel, whose per-column
+For M <= 16 (decode and short prompts: the GEMV and the streaming kernel, whose per-column
 arithmetic does not depend on N) the fused results are bit-identical; for larger M the fused and
 the separate matrices can take different tiled kernels or split-K counts, which changes only the
 fp32 summation order.
@@ -82,7 +82,7 @@ def _int4_fused(lin, x, **kw):
 class FusedInt4Linear(nn.Module):
     """Several INT4 linears on the same input as ONE GEMV/GEMM over their concatenated rows.
 
-    Bit-identical to running them separately for M <= 16 (GEMV and skinny kernels compute each
+    Bit-identical to running them separately for M <= 16 (GEMV and streaming kernels compute each
     column independently of N); above that the tiled kernels' choice or split-K count may differ,
     which only reorders fp32 sums.  Returns the per-part outputs.
     """

@@ -1,0 +1,59 @@
+"""Every tile of int4_gemm at its edges against an exact reference (needs a GPU).
+
+Shapes are the smallest that the dispatcher gives to each tile on a 256-CU device, with rows left over in
+the last row tile, columns in the last column tile where N allows it, K = 64 mod 128 where the tile takes
+it, and one split-K case per tile that splits.  The reference is float64 on the operand the kernels
+use, W = fp16(q * s).  Error bound per element: K fp32 additions of exact products, and the fp16
+rounding of the result: K 2^-24 sum |x w| + 2^-11 |y| (+ the smallest fp16 step).
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from kernelforge import ops
+from oracle import int4_oracle as o
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# (tile, splits, M, N, K)
+CASES = [
+    ((8, 16), 1, 5, 64, 448), ((8, 16), 1, 9, 64, 2112), ((8, 16), 8, 17, 64, 4096),
+    ((16, 16), 1, 257, 128, 448), ((16, 16), 1, 257, 128, 1088), ((16, 16), 8, 81, 64, 4096),
+    ((16, 16), 4, 79, 192, 4096), ((16, 32), 1, 385, 320, 1088), ((16, 32), 7, 33, 384, 8960),
+    ((16, 64), 1, 129, 1728, 448), ((24, 16), 1, 193, 320, 576), ((24, 16), 8, 81, 128, 6272),
+    ((32, 16), 1, 257, 256, 448), ((32, 16), 8, 97, 128, 4096), ((32, 32), 1, 513, 384, 1088),
+    ((32, 32), 5, 113, 384, 5632), ((32, 32), 1, 513, 256, 448), ((32, 32), 7, 257, 128, 4096),
+    ((32, 48), 1, 193, 1728, 832), ((32, 48), 2, 97, 1472, 4096), ((48, 16), 1, 513, 256, 576),
+    ((48, 16), 5, 129, 256, 4224), ((48, 32), 1, 385, 640, 448), ((48, 32), 5, 193, 320, 4480),
+    ((48, 48), 1, 513, 1024, 1088), ((48, 48), 4, 385, 320, 5632), ((48, 48), 1, 513, 1024, 448),
+    ((48, 48), 4, 81, 1472, 4096), ((64, 32), 1, 600, 640, 448), ((64, 32), 5, 300, 320, 4480),
+    ((64, 48), 1, 769, 768, 448), ((64, 48), 3, 513, 384, 5632), ((64, 64), 1, 385, 2048, 1344),
+    ((64, 64), 5, 300, 640, 5632), ((32, 128), 1, 769, 1024, 384), ((32, 128), 5, 513, 384, 6272),
+    ((48, 128), 1, 900, 1280, 384), ((48, 128), 5, 257, 1024, 5632), ((64, 128), 1, 900, 1728, 384),
+    ((64, 128), 5, 300, 1280, 4096), ((80, 128), 1, 900, 2560, 384), ((80, 128), 3, 769, 1024, 4096),
+    ((112, 128), 1, 900, 3072, 384), ((112, 128), 2, 900, 1472, 4096), ((128, 128), 1, 900, 4096, 640),
+    ((128, 128), 1, 900, 2560, 448), ((128, 128), 3, 900, 2304, 6272), ((192, 256), 1, 900, 8960, 384),
+]
+
+
+@pytest.mark.parametrize("tile,splits,m,n,k", CASES)
+def test_tile_edges(tile, splits, m, n, k):
+    group = 128 if k % 128 == 0 else 64
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        plan = ops.gemm_plan(m, n, k, group)
+        assert (plan["tile"], plan["splits"]) == (tile, splits)
+    rng = np.random.Generator(np.random.PCG64(m * 7 + n + k))
+    w = (rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02)).astype(np.float32)
+    packed, scales = o.quantize_weight(w, group)
+    x = torch.from_numpy(rng.standard_normal((m, k), dtype=np.float32).astype(np.float16))
+    w64 = torch.from_numpy(o.dequantize_fp16(packed, scales, group)).to(DEV, torch.float64)
+    x64 = x.to(DEV, torch.float64)
+    ref = x64 @ w64.T
+    bound = k * 2.0 ** -24 * (x64.abs() @ w64.abs().T) + 2.0 ** -11 * ref.abs() + 2.0 ** -24
+    out = ops.int4_gemm(x.to(DEV), torch.from_numpy(packed).to(DEV), torch.from_numpy(scales).to(DEV), group)
+    err = (out.to(torch.float64) - ref).abs()
+    assert bool((err <= bound).all()), f"largest error / bound {float((err / bound).max()):.2f}"
