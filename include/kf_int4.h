@@ -254,6 +254,19 @@ int kf_bw_read_store(const void* src, void* out, size_t bytes, int grid_blocks, 
 int kf_decode_argmax_step(const void* logits, int n, void* token, void* pos, void* history, int max_seq,
                           void* mask, void* stream);
 
+/* Attention of one decode token over the KV cache, one launch:
+ *   out[h] = softmax(mask[h] + q[h] . K[kv] / sqrt(head_dim)) . V[kv],  kv = h / (heads / kv_heads),
+ * over all max_seq keys, fp32 inside, one fp16 rounding of out.  q, out fp16 [heads, head_dim]; cache_k
+ * fp16 [kv_heads, head_dim, max_seq] (K transposed); cache_v fp16 [kv_heads, max_seq, head_dim]; mask
+ * fp16, head h's row of max_seq additive values at mask + h * mask_stride (0: one row for all).
+ * cache_v 16-byte aligned; head_dim a multiple of 8 up to KF_ATTN_MAX_HEAD_DIM, max_seq up to
+ * KF_ATTN_MAX_SEQ (its scores live in LDS).  out must not alias the inputs.  No reference counterpart:
+ * the reference's decode loop runs torch's attention. */
+#define KF_ATTN_MAX_HEAD_DIM 256
+#define KF_ATTN_MAX_SEQ 8192
+int kf_decode_attention(const void* q, const void* cache_k, const void* cache_v, const void* mask, void* out,
+                        int heads, int kv_heads, int head_dim, int max_seq, int mask_stride, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

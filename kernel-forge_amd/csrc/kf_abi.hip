@@ -6,6 +6,7 @@
 // thread-local message, and launches on the caller's stream.  It never
 // allocates, synchronizes, or reads device memory, so it is safe inside
 // hipGraph stream capture.
+#include <math.h>
 #include <stdarg.h>
 #include <stdint.h>
 #include <stdio.h>
@@ -444,6 +445,25 @@ int kf_bw_write(void* dst, size_t bytes, int grid_blocks, void* stream) {
   int st = bw_args(dst, bytes, &grid_blocks);
   if (st) return st;
   return hip_status(kf::bw_write_launch(dst, bytes, grid_blocks, static_cast<hipStream_t>(stream)), "bw_write");
+}
+
+int kf_decode_attention(const void* q, const void* cache_k, const void* cache_v, const void* mask, void* out, int heads,
+                        int kv_heads, int head_dim, int max_seq, int mask_stride, void* stream) {
+  if (!q || !cache_k || !cache_v || !mask || !out)
+    return fail(KF_ERR_INVALID_ARG, "q, cache_k, cache_v, mask and out must be non-null");
+  if (heads < 1 || kv_heads < 1 || heads % kv_heads || head_dim < 1 || max_seq < 1 || mask_stride < 0)
+    return fail(KF_ERR_INVALID_ARG,
+                "need kv_heads >= 1 dividing heads, head_dim, max_seq >= 1 and mask_stride >= 0, got %d, %d, %d, %d, %d",
+                kv_heads, heads, head_dim, max_seq, mask_stride);
+  if (head_dim % 8 || head_dim > KF_ATTN_MAX_HEAD_DIM || max_seq > KF_ATTN_MAX_SEQ)
+    return fail(KF_ERR_UNSUPPORTED, "decode_attention needs head_dim a multiple of 8 up to %d and max_seq up to %d, got %d, %d",
+                KF_ATTN_MAX_HEAD_DIM, KF_ATTN_MAX_SEQ, head_dim, max_seq);
+  if (!aligned(q, 2) || !aligned(cache_k, 2) || !aligned(mask, 2) || !aligned(out, 2) || !aligned(cache_v, 16))
+    return fail(KF_ERR_INVALID_ARG, "q, cache_k, mask and out must be 2-byte, cache_v 16-byte aligned");
+  return hip_status(kf::decode_attention_launch(q, cache_k, cache_v, mask, out, heads, kv_heads, head_dim, max_seq,
+                                                mask_stride, 1.0f / sqrtf((float)head_dim),
+                                                static_cast<hipStream_t>(stream)),
+                    "decode_attention launch");
 }
 
 }  // extern "C"

@@ -186,6 +186,11 @@ hipError_t bw_read_store_launch(const void* src, void* out, size_t bytes, int gr
 hipError_t bw_write_launch(void* dst, size_t bytes, int grid, hipStream_t stream);
 hipError_t decode_argmax_launch(const void* logits, int n, void* token, void* pos, void* history, int max_seq,
                                 void* mask, hipStream_t stream);
+// Attention of one token over the KV cache (kf_attn.hip); mask row h starts at mask + h * mask_stride.
+hipError_t decode_attention_launch(const void* q, const void* cache_k, const void* cache_v, const void* mask, void* out,
+                                   int heads, int kv_heads, int head_dim, int max_seq, int mask_stride, float scale,
+                                   hipStream_t stream);
+
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
 }  // namespace kf

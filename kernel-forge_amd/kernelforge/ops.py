@@ -688,3 +688,59 @@ def decode_argmax_step(logits: torch.Tensor, token: torch.Tensor, pos: torch.Ten
                                            max_seq, _ptr(mask) if mask is not None else None,
                                            _stream_ptr(logits.device))
     _lib.check(status, "decode_argmax_step")
+
+
+# KF_ATTN_MAX_HEAD_DIM / KF_ATTN_MAX_SEQ of the C ABI.
+_ATTN_MAX_HEAD_DIM, _ATTN_MAX_SEQ = 256, 8192
+
+
+def decode_attention_fits(head_dim: int, max_seq: int) -> bool:
+    """Whether decode_attention takes this head size and cache length."""
+    return head_dim % 8 == 0 and 0 < head_dim <= _ATTN_MAX_HEAD_DIM and 0 < max_seq <= _ATTN_MAX_SEQ
+
+
+def decode_attention_eager(q: torch.Tensor, cache_k: torch.Tensor, cache_v: torch.Tensor, mask: torch.Tensor) -> bool:
+    """Whether these operands can go to decode_attention's launch: plain tensors outside any tracer and
+    not tracked by autograd, fp16 on q's device, caches contiguous and 16-byte aligned, mask rows
+    contiguous."""
+    tensors = (q, cache_k, cache_v, mask)
+    if _traced(tensors) or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)):
+        return False
+    return (all(t.dtype == torch.float16 and t.device == q.device for t in tensors) and mask.stride(-1) == 1 and
+            all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (cache_k, cache_v)))
+
+
+def decode_attention(q: torch.Tensor, cache_k: torch.Tensor, cache_v: torch.Tensor, mask: torch.Tensor, *,
+                     kv_heads: int) -> torch.Tensor:
+    """Attention of one decode token over the KV cache in one launch (kf_decode_attention).
+
+    q fp16 [heads, d]; cache_k holds kv_heads x d x max_seq values (K transposed), cache_v kv_heads x
+    max_seq x d, both contiguous; mask fp16 [heads, max_seq] additive, rows contiguous (an expanded
+    row is fine).  Returns softmax(mask + q K / sqrt(d)) V, fp16 [heads, d], with fp32 scores and
+    sums; query head h reads KV head h // (heads / kv_heads).  No reference counterpart (its decode
+    loop runs torch's attention).
+    """
+    if q.dim() != 2 or mask.dim() != 2 or q.dtype != torch.float16 or not q.is_cuda:
+        raise TypeError("q must be a 2-D fp16 CUDA tensor [heads, d] and mask [heads, max_seq]")
+    heads, d = q.shape
+    max_seq = mask.shape[1]
+    if kv_heads < 1 or heads % kv_heads or mask.shape[0] != heads:
+        raise ValueError(f"kv_heads={kv_heads} must divide heads={heads}, and mask must have {heads} rows")
+    if not decode_attention_fits(d, max_seq):
+        raise ValueError(f"decode_attention needs head_dim a multiple of 8 up to {_ATTN_MAX_HEAD_DIM} and max_seq up "
+                         f"to {_ATTN_MAX_SEQ}, got {d} and {max_seq}")
+    for name, t, numel in (("q", q, heads * d), ("cache_k", cache_k, kv_heads * d * max_seq),
+                           ("cache_v", cache_v, kv_heads * max_seq * d)):
+        if t.dtype != torch.float16 or not t.is_contiguous() or t.numel() != numel or t.device != q.device:
+            raise ValueError(f"{name} must be a contiguous fp16 tensor of {numel} elements on {q.device}")
+    if mask.dtype != torch.float16 or mask.device != q.device or (max_seq > 1 and mask.stride(1) != 1):
+        raise ValueError(f"mask must be fp16 on {q.device} with contiguous rows")
+    if _traced((q, cache_k, cache_v, mask)):
+        raise RuntimeError("decode_attention launches a kernel; it cannot be traced")
+    lib = _lib.load()
+    out = torch.empty_like(q)
+    with _on(q.device):
+        status = lib.kf_decode_attention(_ptr(q), _ptr(cache_k), _ptr(cache_v), _ptr(mask), _ptr(out), q.shape[0],
+                                         kv_heads, q.shape[1], mask.shape[1], mask.stride(0), _stream_ptr(q.device))
+    _lib.check(status, "decode_attention")
+    return out

@@ -17,7 +17,8 @@ fp32 summation order.
 Decode follows the reference's graph method (bench/e2e_model.py:85-141): static KV cache,
 positions in device tensors, one decode step captured in a HIP graph and replayed; the greedy
 token is written back into the graph's input on the device, so replays run back to back.
-Attention is plain PyTorch (fp16 matmuls on contiguous operands, fp32 softmax).
+Attention of a decode step on the GPU is one launch (ops.decode_attention, fp32 inside); prompts and
+the CPU run plain PyTorch (fp16 matmuls on contiguous operands, fp32 softmax).
 """
 
 from __future__ import annotations
@@ -148,8 +149,8 @@ class Attention(nn.Module):
         pos int64 [T] positions; cos / sin [T, 1, d] RoPE rows of those positions (sin with the
         rotate-half sign folded in); cache_k / cache_v [kv_heads, max_seq, d] slabs, the key slab
         holding K transposed ([kv_heads, d, max_seq]); scores [kv_heads, rep * T, max_seq] holding
-        the additive causal mask repeated for the rep = heads / kv_heads query heads of a KV head,
-        overwritten with the scores (see attend)."""
+        the additive causal mask repeated for the rep = heads / kv_heads query heads of a KV head
+        (see attend)."""
         return self.attend(self.rope_cache(qk, v, pos, cos, sin, cache_k, cache_v), cache_k, cache_v, scores)
 
     def rope_cache(self, qk, v, pos, cos, sin, cache_k, cache_v):
@@ -166,20 +167,32 @@ class Attention(nn.Module):
     def attend(self, q, cache_k, cache_v, scores):
         """q [T, heads, d] (rotated) over the caches: [1, T, heads d], before o_proj.
 
-        scores: [kv_heads, rep * T, max_seq] holding the mask on entry; the scaled products are
-        added to it in place (baddbmm_ with C = D), which spares the copy of the mask into a fresh
-        output that an out-of-place baddbmm makes in every layer (same values)."""
+        scores: [kv_heads, rep * T, max_seq] holding the mask on entry.  One token on the GPU: the
+        fused launch reads it (fused_decode; it may be an expanded view).  Otherwise the scaled
+        products are added to it in place (baddbmm_ with C = D), which spares the copy of the mask
+        into a fresh output that an out-of-place baddbmm makes in every layer (same values)."""
         cfg = self.cfg
         t = q.shape[0]
         hq, hkv, d = cfg.heads, cfg.kv_heads, cfg.head_dim
         rep = hq // hkv
+        if t == 1 and self.fused_decode(q) and ops.decode_attention_eager(q, cache_k, cache_v, scores):
+            return ops.decode_attention(q.reshape(hq, d), cache_k, cache_v, scores.reshape(hq, cfg.max_seq),
+                                        kv_heads=hkv).view(1, 1, hq * d)
         # Query head h reads KV head h // rep: the rep heads of a KV head (and their T positions)
         # form the rows of one batch entry, so K and V are never repeated.
         qg = q.reshape(t, hkv, rep, d).permute(1, 2, 0, 3).reshape(hkv, rep * t, d)
+        scores = scores.contiguous()  # a copy only of an expanded mask
         scores = scores.baddbmm_(qg, cache_k.view(hkv, d, cfg.max_seq), alpha=1.0 / math.sqrt(d))
         probs = torch.softmax(scores, dim=-1)                            # fp32 inside
         out = torch.bmm(probs, cache_v)                                  # [hkv, rep * T, d]
         return out.view(hkv, rep, t, d).permute(2, 0, 1, 3).reshape(1, t, hq * d)
+
+    def fused_decode(self, x: torch.Tensor) -> bool:
+        """Whether attend runs one token of x's device and dtype as ops.decode_attention: one launch beats
+        torch's three up to about 131072 / d keys (measurements in csrc/kf_attn.hip)."""
+        cfg = self.cfg
+        return (x.is_cuda and x.dtype == torch.float16 and cfg.head_dim * cfg.max_seq <= 131072 and
+                ops.decode_attention_fits(cfg.head_dim, cfg.max_seq))
 
     def forward(self, x, pos, cos, sin, cache_k, cache_v, scores):
         """x [1, T, H] (already normalized); see core for the other arguments."""
@@ -290,14 +303,17 @@ class TinyLlama(nn.Module):
         Inference only (no autograd)."""
         cos, sin = rope
         x = self.embed_tokens(tokens).unsqueeze(0)
-        # Per-token inputs shared by every layer: RoPE rows of the positions, and every layer's
-        # score buffer filled with the mask (repeated for the query heads that share a KV head) by
-        # one copy; each layer adds its scores to its own buffer in place.
+        # Per-token inputs shared by every layer: RoPE rows of the positions, and the mask.  The fused
+        # decode attention reads the one row; otherwise every layer gets a score buffer filled with
+        # the mask (repeated for the query heads that share a KV head) by one copy and adds its
+        # scores to it in place.
         c_ = self.cfg
         t, rep = tokens.numel(), c_.heads // c_.kv_heads
         scores = mask.to(x.dtype).view(1, 1, 1, t, c_.max_seq).expand(c_.layers, c_.kv_heads, rep, t, c_.max_seq)
-        # contiguous() materializes the broadcast (reshape alone would stay a stride-0 view at T = 1).
-        scores = scores.contiguous().view(c_.layers, c_.kv_heads, rep * t, c_.max_seq)
+        if not (t == 1 and self.layers and self.layers[0].self_attn.fused_decode(x)):
+            # contiguous() materializes the broadcast (reshape alone would stay a stride-0 view at T = 1).
+            scores = scores.contiguous()
+        scores = scores.view(c_.layers, c_.kv_heads, rep * t, c_.max_seq)
         rope16 = (cos.to(x.dtype), sin.to(x.dtype)) if x.is_cuda and tokens.numel() == 1 else None
         # The per-position rows are only needed by layers that apply RoPE in torch.
         if rope16 is not None and all(ly.int4_fusable() and ly.self_attn.qkv is not None for ly in self.layers):
