@@ -185,6 +185,17 @@ int kf_int4_gemm(const void* x, const void* packed, const void* scales, void* y,
 int kf_int4_gemm_noalloc(const void* x, const void* packed, const void* scales, void* y, int M, int N, int K,
                          int group_size, void* stream);
 
+/* Up to KF_GEMV_MAX_GROUP independent GEMMs of one M (and G) in as few launches as their plans allow:
+ * problems of one K whose kernels sum in the same order share a launch where that is predicted to
+ * be faster.  Each output equals what kf_int4_gemm computes for that problem, bit for bit.  ws: at
+ * least kf_int4_gemm_grouped_workspace_bytes() (the largest of the problems' own needs; shared, the
+ * problems that split run one after the other).  The problems array is read on the host during the
+ * call.  Every problem is validated before the first launch.  No reference counterpart as an entry
+ * point. */
+size_t kf_int4_gemm_grouped_workspace_bytes(const kf_gemv_problem* problems, int count, int M, int group_size);
+int kf_int4_gemm_grouped(const kf_gemv_problem* problems, int count, int M, int group_size, void* ws,
+                         size_t ws_bytes, void* stream);
+
 /* MFMA-16 block copy of a packed weight (an internal layout; the public packed format is
  * unchanged): for every 16 rows of W and 128-k super-step, the 64 lanes' 16-byte pieces of
  * the MFMA fragments stored contiguously in lane order (lane l: row 16b + l%16, words

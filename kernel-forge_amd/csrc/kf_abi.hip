@@ -12,6 +12,7 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -120,10 +121,9 @@ int scratch_ptr(void** out) {
   return KF_OK;
 }
 
-// kf_int4_gemm, kf_int4_gemm_mfma16 and kf_int4_gemm_noalloc: validation, plan, workspace check,
-// launch.  With use_scratch the split-K partials go to this device's scratch array (ws is ignored).
-int gemm_entry(const void* x, const void* packed, const void* scales, void* y, void* ws, size_t ws_bytes, int M, int N,
-               int K, int group_size, void* stream, bool use_scratch = false) {
+// Validation and plan of one GEMM problem (cus: looked up once per entry point, 0 before).
+int gemm_check(const void* x, const void* packed, const void* scales, const void* y, int M, int N, int K,
+               int group_size, int* cus, kf::GemmPlan* plan) {
   int st = check_common(x, packed, scales, y, M, N, K, group_size);
   if (st) return st;
   if (N % 64 != 0) return fail(KF_ERR_UNSUPPORTED, "int4_gemm needs N to be a multiple of 64, got N=%d", N);
@@ -131,14 +131,25 @@ int gemm_entry(const void* x, const void* packed, const void* scales, void* y, v
   // The GEMM epilogues store y as 8- and 16-byte vectors (N % 64 == 0 keeps every row's start on
   // a 16-byte boundary once y's is).
   if (!aligned(y, 16)) return fail(KF_ERR_INVALID_ARG, "int4_gemm needs y to be 16-byte aligned");
-  int cus = 0;
-  if ((st = cu_count(&cus))) return st;
-  const kf::GemmPlan plan = kf::gemm_plan(M, N, K, cus);
+  if (*cus == 0 && (st = cu_count(cus))) return st;
+  *plan = kf::gemm_plan(M, N, K, *cus);
   // One workgroup per output tile and split, all in grid dimension x.
-  const long long tiles = (long long)((M + plan.block_m - 1) / plan.block_m) * ((N + plan.block_n - 1) / plan.block_n);
-  if ((tiles * plan.splits + 8) * plan.threads > 0x7FFFFFFFLL)
-    return fail(KF_ERR_UNSUPPORTED, "M=%d, N=%d exceed the grid limit for %dx%d tiles", M, N, plan.block_m,
-                plan.block_n);
+  const long long tiles =
+      (long long)((M + plan->block_m - 1) / plan->block_m) * ((N + plan->block_n - 1) / plan->block_n);
+  if ((tiles * plan->splits + 8) * plan->threads > 0x7FFFFFFFLL)
+    return fail(KF_ERR_UNSUPPORTED, "M=%d, N=%d exceed the grid limit for %dx%d tiles", M, N, plan->block_m,
+                plan->block_n);
+  return KF_OK;
+}
+
+// kf_int4_gemm, kf_int4_gemm_mfma16 and kf_int4_gemm_noalloc: validation, plan, workspace check,
+// launch.  With use_scratch the split-K partials go to this device's scratch array (ws is ignored).
+int gemm_entry(const void* x, const void* packed, const void* scales, void* y, void* ws, size_t ws_bytes, int M, int N,
+               int K, int group_size, void* stream, bool use_scratch = false) {
+  int cus = 0;
+  kf::GemmPlan plan;
+  int st = gemm_check(x, packed, scales, y, M, N, K, group_size, &cus, &plan);
+  if (st) return st;
   const size_t need = kf::gemm_workspace_bytes(plan, M, N);
   if (use_scratch) {
     ws = nullptr;
@@ -296,6 +307,66 @@ size_t kf_int4_gemm_workspace_bytes(int M, int N, int K, int group_size) {
   int cus = 0;
   if (cu_count(&cus)) return 0;
   return kf::gemm_workspace_bytes(kf::gemm_plan(M, N, K, cus), M, N);
+}
+
+size_t kf_int4_gemm_grouped_workspace_bytes(const kf_gemv_problem* problems, int count, int M, int group_size) {
+  size_t need = 0;
+  if (problems)
+    for (int i = 0; i < count; ++i)
+      need = std::max(need, kf_int4_gemm_workspace_bytes(M, problems[i].N, problems[i].K, group_size));
+  return need;
+}
+
+int kf_int4_gemm_grouped(const kf_gemv_problem* problems, int count, int M, int group_size, void* ws, size_t ws_bytes,
+                         void* stream) {
+  if (!problems) return fail(KF_ERR_INVALID_ARG, "problems must be non-null");
+  if (count < 1 || count > KF_GEMV_MAX_GROUP)
+    return fail(KF_ERR_INVALID_ARG, "count must be in [1, %d], got %d", KF_GEMV_MAX_GROUP, count);
+  static_assert(KF_GEMV_MAX_GROUP <= kf::kMaxGemmGroup, "group table");
+  kf::GemmPlan plans[KF_GEMV_MAX_GROUP];
+  int cus = 0, st;
+  for (int i = 0; i < count; ++i) {
+    const kf_gemv_problem& p = problems[i];
+    if ((st = gemm_check(p.x, p.packed, p.scales, p.y, M, p.N, p.K, group_size, &cus, &plans[i])))
+      return fail(st, "problem %d: %s", i, kf_last_error());
+    const size_t need = kf::gemm_workspace_bytes(plans[i], M, p.N);
+    if (need > 0) {
+      if (!ws) return fail(KF_ERR_WORKSPACE, "split-K workspace of %zu bytes required, got NULL", need);
+      if (ws_bytes < need)
+        return fail(KF_ERR_WORKSPACE, "split-K workspace of %zu bytes required, got %zu", need, ws_bytes);
+      if (!aligned(ws, 16)) return fail(KF_ERR_INVALID_ARG, "workspace must be 16-byte aligned");
+    }
+  }
+  // Problems of one K whose plans sum in one order share a launch; the others run by themselves, one
+  // after the other on the workspace.
+  bool done[KF_GEMV_MAX_GROUP] = {};
+  for (int i = 0; i < count; ++i) {
+    if (done[i]) continue;
+    kf::GemvProblem group[KF_GEMV_MAX_GROUP];
+    kf::GemmPlan group_plans[KF_GEMV_MAX_GROUP];
+    int ns[KF_GEMV_MAX_GROUP], n = 0;
+    bool member[KF_GEMV_MAX_GROUP] = {};
+    for (int j = i; j < count; ++j) {
+      const kf_gemv_problem& p = problems[j];
+      if (done[j] || p.K != problems[i].K || (j > i && !kf::gemm_same_sums(plans[i], plans[j]))) continue;
+      member[j] = true;
+      group[n] = {p.x, p.packed, p.scales, p.y, p.N, p.K};
+      group_plans[n] = plans[j];
+      ns[n++] = p.N;
+    }
+    const int cfg = n > 1 ? kf::gemm_group_config(group_plans, ns, n, M, problems[i].K, cus) : -1;
+    hipError_t err;
+    if (cfg >= 0) {
+      for (int j = i; j < count; ++j) done[j] = done[j] || member[j];
+      err = kf::gemm_grouped_launch(cfg, group, n, M, problems[i].K, group_size, static_cast<hipStream_t>(stream));
+    } else {
+      const kf_gemv_problem& p = problems[i];
+      err = kf::gemm_launch(plans[i], p.x, p.packed, p.scales, p.y, ws, M, p.N, p.K, group_size,
+                            static_cast<hipStream_t>(stream));
+    }
+    if (err != hipSuccess) return hip_status(err, "int4_gemm_grouped launch");
+  }
+  return KF_OK;
 }
 
 int kf_int4_gemm_plan(int M, int N, int K, int group_size, int* kernel, int* num_kernels, int* splits, int* block_m,

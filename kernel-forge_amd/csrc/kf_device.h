@@ -12,6 +12,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "kf_launch.h"
+
 namespace kf {
 
 typedef _Float16 half_t;
@@ -143,6 +145,30 @@ __device__ __forceinline__ u32x4 load_u32x4(const void* p) {
 // Streaming (non-temporal) 16-byte load for data read exactly once.
 __device__ __forceinline__ u32x4 load_u32x4_stream(const void* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
+}
+
+// The problem of a grouped GEMM launch that owns column tile nt: the slot index from scalar compares,
+// then the slot in two scalar loads.
+struct GroupEntry {
+  const half_t* x;
+  const uint32_t* packed;
+  const half_t* scales;
+  half_t* y;
+  int N, tile0;
+};
+__device__ __forceinline__ GroupEntry group_entry(const GroupTable& table, int count, int nt) {
+  int p = 0;
+#pragma unroll
+  for (int i = 1; i < kMaxGemmGroup; ++i) p += i < count && nt >= table.slot[i].tile0 ? 1 : 0;
+  typedef const __attribute__((address_space(1))) half_t* gh_t;
+  typedef const __attribute__((address_space(1))) uint32_t* gu_t;
+  typedef __attribute__((address_space(1))) half_t* gy_t;
+  typedef uint64_t u64x4_t __attribute__((ext_vector_type(4)));
+  const char* desc = reinterpret_cast<const char*>(&table.slot[p]);
+  const u64x4_t ptr = *reinterpret_cast<const u64x4_t*>(desc);
+  const GroupSlot& q = table.slot[p];
+  return GroupEntry{(const half_t*)(gh_t)ptr[0], (const uint32_t*)(gu_t)ptr[1], (const half_t*)(gh_t)ptr[2],
+                    (half_t*)(gy_t)ptr[3], q.N, q.tile0};
 }
 
 }  // namespace kf

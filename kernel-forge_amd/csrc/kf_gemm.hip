@@ -356,15 +356,12 @@ struct Dma4Cfg {
 };
 
 template <class C>
-__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
-void gemm_dma4_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ packed,
-                      const half_t* __restrict__ scales, half_t* __restrict__ y, float* __restrict__ ws, int M, int N,
-                      int K, int log2_group, int stages_per_split, int splits, int tiles_m, int tiles_n,
-                      int group_m) {
+__device__ __forceinline__ void dma4_tile(const half_t* x, const uint32_t* packed, const half_t* scales, half_t* y,
+                                          float* part, int M, int N, int K, int log2_group, int m0, int n0,
+                                          int st_begin, int ns) {
   constexpr int BM = C::BM, BN = C::BN, BK = C::BK, NS = C::NS, TM = C::TM, TN = C::TN, WAVES = C::WAVES;
   constexpr int A_ROW = C::A_ROW, B_ROW = C::B_ROW, OUT_ROW = C::OUT_ROW;
-  extern __shared__ __attribute__((aligned(1024))) unsigned char dyn_smem[];
-  unsigned char* const smem = dyn_smem;
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[C::SMEM];  // static: no attribute call above 64 KiB
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -373,18 +370,6 @@ void gemm_dma4_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__
   const int kw = wave >> 1;
   const int g = lane >> 4;
   const int l16 = lane & 15;
-
-  int split, t;
-  if (!gemm_job(tiles_m * tiles_n, splits, split, t)) return;
-  const int band = group_m * tiles_n;
-  const int bi = t / band;
-  const int tb = t - bi * band;
-  const int gm = min(group_m, tiles_m - bi * group_m);
-  const int m0 = (bi * group_m + tb % gm) * BM;
-  const int n0 = (tb / gm) * BN;
-
-  const int st_begin = split * stages_per_split;
-  const int ns = min(K / BK - st_begin, stages_per_split);  // >= 1: no split is empty
 
   // x chunk c (16 bytes) of row r at slot c ^ (r & 15); packed chunk h at h ^ ((r >> 2) & 3).
   const half_t* a_src[C::A_PW];
@@ -508,9 +493,8 @@ void gemm_dma4_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__
     }
   }
 
-  if (ws) {
+  if (part) {
     if (kw == 0) {
-      float* part = ws + (size_t)split * M * N;
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -541,6 +525,45 @@ void gemm_dma4_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__
     if (gr < M && gc < N)
       *reinterpret_cast<u32x4*>(y + (size_t)gr * N + gc) = *reinterpret_cast<const u32x4*>(smem + row * OUT_ROW + 16 * chunk);
   }
+}
+
+// Rows and columns of job t's tile: bands of group_m row tiles, all column tiles of a band before the next.
+__device__ __forceinline__ void band_tile(int t, int tiles_m, int tiles_n, int group_m, int& mt, int& nt) {
+  const int band = group_m * tiles_n;
+  const int bi = t / band;
+  const int tb = t - bi * band;
+  const int gm = min(group_m, tiles_m - bi * group_m);
+  mt = bi * group_m + tb % gm;
+  nt = tb / gm;
+}
+
+template <class C>
+__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_dma4_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ packed,
+                      const half_t* __restrict__ scales, half_t* __restrict__ y, float* __restrict__ ws, int M, int N,
+                      int K, int log2_group, int stages_per_split, int splits, int tiles_m, int tiles_n,
+                      int group_m) {
+  int split, t, mt, nt;
+  if (!gemm_job(tiles_m * tiles_n, splits, split, t)) return;
+  band_tile(t, tiles_m, tiles_n, group_m, mt, nt);
+  const int st_begin = split * stages_per_split;
+  const int ns = min(K / C::BK - st_begin, stages_per_split);  // >= 1: no split is empty
+  dma4_tile<C>(x, packed, scales, y, ws ? ws + (size_t)split * M * N : nullptr, M, N, K, log2_group, mt * C::BM,
+               nt * C::BN, st_begin, ns);
+}
+
+// Several problems of one M, K and group size in one launch (see stream_grouped_kernel): the tiles of
+// siblings fill the last round of workgroups together.
+template <class C>
+__global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
+void gemm_dma4_grouped_kernel(int count, int M, int K, int log2_group, int tiles_m, int tiles_n, int group_m,
+                              const GroupTable table) {
+  int split, t, mt, nt;
+  if (!gemm_job(tiles_m * tiles_n, 1, split, t)) return;
+  band_tile(t, tiles_m, tiles_n, group_m, mt, nt);
+  const GroupEntry e = group_entry(table, count, nt);
+  dma4_tile<C>(e.x, e.packed, e.scales, e.y, nullptr, M, e.N, K, log2_group, mt * C::BM, (nt - e.tile0) * C::BN, 0,
+               K / C::BK);
 }
 
 // Wide DMA-fed tile: 192 x 256 per workgroup, 8 wavefronts as 2 x 4 wave tiles of 96 x 64, every
@@ -777,21 +800,25 @@ __global__ __launch_bounds__(256) void splitk_reduce(const float4_t* __restrict_
 typedef void (*GemmFn)(const half_t*, const uint32_t*, const half_t*, half_t*, float*, int, int, int, int, int, int,
                        int, int, int);
 
-// A tile of a DMA kernel: its size, k per stage, workgroup and dynamic LDS.
+typedef void (*GemmGroupedFn)(int, int, int, int, int, int, int, const GroupTable);
+
+// A tile of a DMA kernel: its size, k per stage and workgroup.
 struct DmaEntry {
-  int bm, bn, bk, threads, lds;
+  int bm, bn, bk, threads;
   GemmFn fn;
+  GemmGroupedFn grouped;  // four k-groups only
 };
 template <int TM, int TN, int NS>
 constexpr DmaEntry dma4_entry() {
   using C = Dma4Cfg<TM, TN, NS>;
-  return DmaEntry{C::BM, C::BN, C::BK, C::THREADS, C::SMEM, gemm_dma4_kernel<C>};
+  return DmaEntry{C::BM, C::BN, C::BK, C::THREADS, gemm_dma4_kernel<C>,
+                  gemm_dma4_grouped_kernel<C>};
 }
 const DmaEntry kDma[] = {
     dma4_entry<2, 4, 4>(), dma4_entry<3, 4, 4>(), dma4_entry<4, 4, 3>(),
     dma4_entry<5, 4, 3>(), dma4_entry<7, 4, 3>(), dma4_entry<8, 4, 3>(),
-    DmaEntry{128, 128, DmaCfg::BK, DmaCfg::THREADS, 0, gemm_dma2_kernel},
-    DmaEntry{192, 256, WideCfg::BK, WideCfg::THREADS, 0, gemm_wide_kernel},
+    DmaEntry{128, 128, DmaCfg::BK, DmaCfg::THREADS, gemm_dma2_kernel, nullptr},
+    DmaEntry{192, 256, WideCfg::BK, WideCfg::THREADS, gemm_wide_kernel, nullptr},
 };
 constexpr int kNumDma = sizeof(kDma) / sizeof(kDma[0]);
 
@@ -865,7 +892,7 @@ const CostTerms kCost[] = {
 // Split-K costs one more launch plus the fp32 partials (same fit), and is taken only when the
 // model predicts it at least 3% faster.
 constexpr double kSplitUs = 2.324, kSplitUsPerMElem = 1.624, kSplitMargin = 1.03;
-// Layers much deeper than wide (K >= 4096, K >= 2.5 N) are split unless the model puts the split more
+// Layers much deeper than wide (K > 4096, K >= 2.5 N) are split unless the model puts the split more
 // than 1 / 0.78 behind: there the model is too careful as often as not, and these layers' plans have
 // always asked for a workspace, which callers of the workspace entry points are written against.
 // Best unsplit / best split (us): 4096 x 14336 at M = 160: 45.1 / 34.3; 1536 x 8960 at M = 517: 33.0 /
@@ -903,7 +930,7 @@ static double plan_cost(int cfg, long tiles, int splits, int M, double n, int K,
   const double cost =
       t.c[0] + (t.c[1] + t.c[2] * k) * per_cu + (t.c[3] + t.c[4] * rounds) * k + t.c[5] * n * K * 1e-6;
   return splits == 1 ? cost : (cost + kSplitUs + kSplitUsPerMElem * 1e-6 * splits * (double)M * n) *
-                                  (K >= 4096 && K >= 2.5 * n ? kDeepSplitMargin : kSplitMargin);
+                                  (K > 4096 && K >= 2.5 * n ? kDeepSplitMargin : kSplitMargin);
 }
 
 // At M <= 16 the K split over wavefronts depends on M and K alone (see gemm_plan).  Four wavefronts
@@ -917,6 +944,8 @@ static int small_m_waves(int M, int K) { return K < 2048 || (M <= 8 && K <= 4096
 //   * M <= 16: streaming tiles of small_m_waves(M, K) wavefronts without split-K only, so the K split
 //     (and with it every bit of a column) does not depend on N and concatenated q|k|v or gate|up rows
 //     give the separate layers' results.
+//   * Narrow layers above that take eight wavefronts (256 x 2048 at M = 27 / 48, four or eight: 3.68 / 3.64
+//     and 3.72 / 3.68 us), so that k and v can share a launch with q, whose plan has eight.
 //   * Partials of a split are held to the scratch of kf_int4_gemm_noalloc, so that entry point takes
 //     every shape, except where K >= 16384: there a few tiles may need more splits than that.
 GemmPlan gemm_plan(int M, int N, int K, int cu_count) {
@@ -931,6 +960,7 @@ GemmPlan gemm_plan(int M, int N, int K, int cu_count) {
       const StreamTile t = stream_tile_of(cfg);
       bm = t.bm, bn = t.bn, threads = 64 * t.ks;
       if (M <= 16 && t.ks != small_m_waves(M, K)) continue;
+      if (M > 16 && N <= 1024 && K >= 1536 && t.ks != 8) continue;
     } else {
       const DmaEntry& e = kDma[cfg - num_stream];
       bm = e.bm, bn = e.bn, threads = e.threads;
@@ -961,6 +991,60 @@ size_t gemm_workspace_bytes(const GemmPlan& p, int M, int N) {
   return p.splits > 1 ? (size_t)p.splits * M * N * sizeof(float) : 0;
 }
 
+bool gemm_same_sums(const GemmPlan& a, const GemmPlan& b) {
+  if (a.splits != 1 || b.splits != 1) return false;
+  const int ns = stream_num_configs();
+  if (a.cfg < ns || b.cfg < ns)
+    return a.cfg < ns && b.cfg < ns && stream_tile_of(a.cfg).ks == stream_tile_of(b.cfg).ks;
+  return kDma[a.cfg - ns].grouped && kDma[b.cfg - ns].grouped;
+}
+
+// Streaming tiles sum an element in an order that depends on K and their wavefronts only, the DMA tiles
+// of four k-groups in one that depends on K only, so any tile of the same kind gives a sibling the bits
+// of its own plan.  All plans have to be of one kind (gemm_same_sums); the tile is the one with the
+// smallest modelled time for all columns together, taken where that is less than the sum of the
+// separate launches.  Separate / grouped, us: q|k|v of 2048 + 2 x 256 columns, K = 2048, at M = 16 / 64 /
+// 200 (k|v): 11.3 / 4.4, 12.2 / 5.5, 15.4 / 12.1; gate|up of 2 x 5632: 10.7 / 7.4, 14.0 / 12.4, 25.9 / 19.2;
+// 2 x 14336, K = 4096, at M = 128 / 517 / 1024: 50.7 / 39.6, 164 / 160, 252 / 261 (the worst; asking for a
+// predicted gain of 3% left that one grouped and lost 8% at 2 x 8960, K = 1536, M = 200).
+int gemm_group_config(const GemmPlan* plans, const int* N, int count, int M, int K, int cu_count) {
+  const int cus = cu_count > 0 ? cu_count : 256;
+  double best = 0.0, columns = 0.0;
+  for (int i = 0; i < count; ++i) {
+    if (!gemm_same_sums(plans[0], plans[i])) return -1;
+    best += plan_cost(plans[i].cfg, (long)ceil_div(M, plans[i].block_m) * ceil_div(N[i], plans[i].block_n), 1, M, N[i],
+                      K, cus);
+    columns += N[i];
+  }
+  int best_cfg = -1;
+  for (int cfg = 0; cfg < gemm_num_configs(); ++cfg) {
+    const GemmPlan p = gemm_plan_with(cfg, 1, K);
+    if (!gemm_same_sums(plans[0], p)) continue;
+    long tiles = 0;
+    for (int i = 0; i < count; ++i) tiles += ceil_div(N[i], p.block_n);
+    tiles *= ceil_div(M, p.block_m);
+    if ((tiles + kXcds) * p.threads > 0x7FFFFFFFL) continue;
+    const double cost = plan_cost(cfg, tiles, 1, M, columns, K, cus);
+    if (cost < best) {
+      best = cost;
+      best_cfg = cfg;
+    }
+  }
+  return best_cfg;
+}
+
+hipError_t gemm_grouped_launch(int cfg, const GemvProblem* problems, int count, int M, int K, int group_size,
+                               hipStream_t stream) {
+  if (cfg < stream_num_configs()) return stream_grouped_launch(cfg, problems, count, M, K, group_size, stream);
+  const DmaEntry& e = kDma[cfg - stream_num_configs()];
+  GroupTable table = {};
+  const int tiles_m = ceil_div(M, e.bm), tiles_n = group_table(problems, count, e.bn, table);
+  const int grid = ceil_div(tiles_m * tiles_n, kXcds) * kXcds;
+  hipLaunchKernelGGL(e.grouped, dim3(grid), dim3(e.threads), 0, stream, count, M, K, group_size == 128 ? 7 : 6,
+                     tiles_m, tiles_n, std::max(1, tiles_m / kXcds), table);
+  return hipGetLastError();
+}
+
 hipError_t gemm_launch(const GemmPlan& p, const void* x, const void* packed, const void* scales, void* y,
                        void* ws, int M, int N, int K, int group_size, hipStream_t stream) {
   float* part = p.splits > 1 ? static_cast<float*>(ws) : nullptr;
@@ -976,12 +1060,7 @@ hipError_t gemm_launch(const GemmPlan& p, const void* x, const void* packed, con
     // Bands of M-tiles: one band per XCD when the M-tiles divide evenly, else single rows.
     int group_m = tiles_m / kXcds;
     if (group_m < 1) group_m = 1;
-    if (e.lds > 65536) {  // dynamic LDS beyond 64 KiB is opted into per kernel
-      err = hipFuncSetAttribute(reinterpret_cast<const void*>(e.fn), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                kLdsPerCu);
-      if (err != hipSuccess) return err;
-    }
-    hipLaunchKernelGGL(e.fn, dim3(grid_x), dim3(e.threads), e.lds, stream, static_cast<const half_t*>(x),
+    hipLaunchKernelGGL(e.fn, dim3(grid_x), dim3(e.threads), 0, stream, static_cast<const half_t*>(x),
                        static_cast<const uint32_t*>(packed), static_cast<const half_t*>(scales),
                        static_cast<half_t*>(y), part, M, N, K, log2_group, p.kt_per_split, p.splits, tiles_m, tiles_n,
                        group_m);

@@ -147,6 +147,25 @@ StreamTile stream_tile_of(int cfg);
 hipError_t stream_launch(int cfg, int splits, const void* x, const void* packed, const void* scales, void* y,
                          float* part, int M, int N, int K, int group_size, hipStream_t stream);
 
+// Several problems of one M and K (each N % 64 == 0) in one launch of a streaming or four-k-group DMA
+// tile: the table is the kernels' argument.
+constexpr int kMaxGemmGroup = 8;
+struct GroupSlot {
+  const void* x;
+  const void* packed;
+  const void* scales;
+  void* y;
+  int N;
+  int tile0;  // first column tile
+};
+struct GroupTable {
+  GroupSlot slot[kMaxGemmGroup];
+};
+// Fills the table for column tiles of bn; returns the number of column tiles.
+int group_table(const GemvProblem* problems, int count, int bn, GroupTable& table);
+hipError_t stream_grouped_launch(int cfg, const GemvProblem* problems, int count, int M, int K, int group_size,
+                                 hipStream_t stream);
+
 // ---- MFMA-16 block copy of packed / scales (kf_aux.hip): sizes in int32 words and fp16 scales --
 size_t mfma16_packed_words(int N, int K);
 size_t mfma16_scale_count(int N, int K, int group_size);
@@ -164,6 +183,13 @@ struct GemmPlan {
   int kt_per_split;// k stages per split (DMA tiles)
 };
 GemmPlan gemm_plan(int M, int N, int K, int cu_count);
+// The configuration that runs problems of these plans (one M and K) in one launch with the bits of
+// their own launches, or -1 when there is none or separate launches are predicted to be faster.
+int gemm_group_config(const GemmPlan* plans, const int* N, int count, int M, int K, int cu_count);
+hipError_t gemm_grouped_launch(int cfg, const GemvProblem* problems, int count, int M, int K, int group_size,
+                               hipStream_t stream);
+// Whether two plans sum every element in the same order (see gemm_group_config).
+bool gemm_same_sums(const GemmPlan& a, const GemmPlan& b);
 // Plan with an explicit configuration and split count (tuning).
 GemmPlan gemm_plan_with(int cfg, int splits, int K);
 int gemm_num_configs();

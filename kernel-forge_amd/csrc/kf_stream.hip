@@ -92,7 +92,7 @@ __device__ __forceinline__ void stream_tile(const half_t* x, const uint32_t* pac
                                             float* part, int M, int N, int K, int log2_group, int m0, int n0,
                                             int k_begin, int k_end, bool once) {
   constexpr int XG = C::XG, TN = C::TN, KS = C::KS, PP = C::PP, WS = C::WS, WP = C::WP, TM = C::TM;
-  extern __shared__ __attribute__((aligned(1024))) unsigned char smem[];
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS];  // static: no attribute call above 64 KiB
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, g = lane >> 4;
@@ -285,17 +285,36 @@ __global__ __launch_bounds__(64 * C::KS) void stream_kernel(const half_t* __rest
                  mt * 8 * C::XG, nt * 16 * C::TN, k0, k1, tiles_m == 1);
 }
 
+// Several problems of one M, K and group size in one launch: column tiles are numbered through the
+// problems, problem p owning tiles slot[p].tile0 up to the next problem's.  Each output has the bits of
+// its own stream_kernel launch at the same KS: the K split does not depend on N or on the tile.  A
+// launch of its own costs a small layer about 2 us of start and tail, more than its work.
+template <class C>
+__global__ __launch_bounds__(64 * C::KS) void stream_grouped_kernel(int count, int M, int K, int log2_group,
+                                                                    int tiles_m, int tiles_n, int rows_first,
+                                                                    const GroupTable table) {
+  const int job = stream_job(tiles_m * tiles_n);
+  if (job < 0) return;
+  const int mt = rows_first ? job % tiles_m : job / tiles_n;
+  const int nt = rows_first ? job / tiles_m : job % tiles_n;
+  const GroupEntry e = group_entry(table, count, nt);
+  stream_tile<C>(e.x, e.packed, e.scales, e.y, nullptr, M, e.N, K, log2_group, mt * 8 * C::XG,
+                 (nt - e.tile0) * 16 * C::TN, 0, K >> 6, tiles_m == 1);
+}
+
 typedef void (*StreamFn)(const half_t*, const uint32_t*, const half_t*, half_t*, float*, int, int, int, int, int, int,
                          int);
+typedef void (*StreamGroupedFn)(int, int, int, int, int, int, int, const GroupTable);
 
 struct StreamEntry {
   int xg, tn, ks, lds;
   StreamFn fn;
+  StreamGroupedFn grouped;
 };
 template <int XG, int TN, int KS, int PP, int WS>
 constexpr StreamEntry stream_entry() {
   using C = StreamCfg<XG, TN, KS, PP, WS>;
-  return StreamEntry{XG, TN, KS, C::LDS, stream_kernel<C>};
+  return StreamEntry{XG, TN, KS, C::LDS, stream_kernel<C>, stream_grouped_kernel<C>};
 }
 
 const StreamEntry kStream[] = {
@@ -319,16 +338,32 @@ hipError_t stream_launch(int cfg, int splits, const void* x, const void* packed,
                          float* part, int M, int N, int K, int group_size, hipStream_t stream) {
   const StreamEntry& e = kStream[cfg];
   const int tiles_m = ceil_div(M, 8 * e.xg), tiles_n = ceil_div(N, 16 * e.tn);
-  if (e.lds > 65536) {  // dynamic LDS beyond 64 KiB is opted into per kernel
-    const hipError_t err = hipFuncSetAttribute(reinterpret_cast<const void*>(e.fn),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, kLdsPerCu);
-    if (err != hipSuccess) return err;
-  }
   const int grid = ceil_div(tiles_m * tiles_n * splits, kXcds) * kXcds;
-  hipLaunchKernelGGL(e.fn, dim3(grid), dim3(64 * e.ks), e.lds, stream, static_cast<const half_t*>(x),
+  hipLaunchKernelGGL(e.fn, dim3(grid), dim3(64 * e.ks), 0, stream, static_cast<const half_t*>(x),
                      static_cast<const uint32_t*>(packed), static_cast<const half_t*>(scales),
                      static_cast<half_t*>(y), splits > 1 ? part : nullptr, M, N, K, group_size == 128 ? 7 : 6, tiles_m,
                      tiles_n, splits);
+  return hipGetLastError();
+}
+
+int group_table(const GemvProblem* problems, int count, int bn, GroupTable& table) {
+  int tiles_n = 0;
+  for (int i = 0; i < count; ++i) {
+    const GemvProblem& q = problems[i];
+    table.slot[i] = GroupSlot{q.x, q.packed, q.scales, q.y, q.N, tiles_n};
+    tiles_n += ceil_div(q.N, bn);
+  }
+  return tiles_n;
+}
+
+hipError_t stream_grouped_launch(int cfg, const GemvProblem* problems, int count, int M, int K, int group_size,
+                                 hipStream_t stream) {
+  const StreamEntry& e = kStream[cfg];
+  GroupTable table = {};
+  const int tiles_m = ceil_div(M, 8 * e.xg), tiles_n = group_table(problems, count, 16 * e.tn, table);
+  const int grid = ceil_div(tiles_m * tiles_n, kXcds) * kXcds;
+  hipLaunchKernelGGL(e.grouped, dim3(grid), dim3(64 * e.ks), 0, stream, count, M, K, group_size == 128 ? 7 : 6,
+                     tiles_m, tiles_n, 4L * M <= 16L * e.tn * tiles_n ? 1 : 0, table);
   return hipGetLastError();
 }
 

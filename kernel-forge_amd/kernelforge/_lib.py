@@ -63,6 +63,8 @@ SIGNATURES = {
     "kf_int4_gemm_noalloc": (_I, [_VP, _VP, _VP, _VP, _I, _I, _I, _I, _VP]),
     "kf_int4_mfma16_sizes": (_I, [_I, _I, _I, ctypes.POINTER(_SZ), ctypes.POINTER(_SZ)]),
     "kf_int4_reorder_mfma16": (_I, [_VP, _VP, _VP, _VP, _I, _I, _I, _VP]),
+    "kf_int4_gemm_grouped_workspace_bytes": (_SZ, [ctypes.POINTER(GemvProblem), _I, _I, _I]),
+    "kf_int4_gemm_grouped": (_I, [ctypes.POINTER(GemvProblem), _I, _I, _I, _VP, _SZ, _VP]),
     "kf_int4_gemm_mfma16": (_I, [_VP, _VP, _VP, _VP, _VP, _VP, _VP, _SZ, _I, _I, _I, _I, _VP]),
     "kf_int4_dequant_fp16": (_I, [_VP, _VP, _VP, _I, _I, _I, _VP]),
     "kf_int4_quantize": (_I, [_VP, _I, _VP, _VP, _I, _I, _I, _VP]),

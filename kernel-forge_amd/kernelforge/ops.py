@@ -423,9 +423,45 @@ def _matmul_grouped(xs: list[torch.Tensor], packed: list[torch.Tensor], scales: 
     """checked: _check_int4 has passed on every problem (int4_linear_grouped's eager path)."""
     if all(_use_gemv(x.shape[0], p.shape[0]) for x, p in zip(xs, packed)):
         return int4_gemv_grouped(xs, packed, scales, group_size, _checked=checked)
+    if _groupable(xs, packed):
+        return _launch_gemm_grouped(xs, packed, scales, group_size, checked)
     if xs[0].shape[0] <= _GEMV_LIMIT_M:
         return [int4_matmul(x, p, s, group_size) for x, p, s in zip(xs, packed, scales)]
     return [int4_gemm(x, p, s, group_size) for x, p, s in zip(xs, packed, scales)]
+
+
+def _groupable(xs: list[torch.Tensor], packed: list[torch.Tensor]) -> bool:
+    """Whether these problems go to kf_int4_gemm_grouped: one M above the GEMV's, one device, every N
+    a multiple of 64, and no MFMA-16 copies in use."""
+    m, dev = xs[0].shape[0], xs[0].device
+    return (m > GEMV_MAX_M and len(xs) > 1 and not MFMA16_CACHE and
+            all(x.shape[0] == m and x.device == dev and p.shape[0] % 64 == 0 and not hasattr(p, _MFMA16_ATTR)
+                for x, p in zip(xs, packed)))
+
+
+def _launch_gemm_grouped(xs: list[torch.Tensor], packed: list[torch.Tensor], scales: list[torch.Tensor],
+                         group_size: int, checked: bool) -> list[torch.Tensor]:
+    """int4_gemm of every problem through kf_int4_gemm_grouped, KF_GEMV_MAX_GROUP problems per call."""
+    for x, p, s in zip(xs, packed, scales):
+        if not checked:
+            _check_int4(x, p, s, group_size)
+        _check_native(x, p, s, group_size)
+    lib = _lib.load()
+    dev, m, group_size = xs[0].device, xs[0].shape[0], int(group_size)
+    ys = [torch.empty(m, p.shape[0], dtype=torch.float16, device=dev) for p in packed]
+    with _on(dev):
+        stream = _stream_ptr(dev)
+        for b0 in range(0, len(xs), _lib.GEMV_MAX_GROUP):
+            part = range(b0, min(b0 + _lib.GEMV_MAX_GROUP, len(xs)))
+            probs = (_lib.GemvProblem * len(part))(*[
+                _lib.GemvProblem(xs[i].data_ptr(), packed[i].data_ptr(), scales[i].data_ptr(), ys[i].data_ptr(),
+                                 packed[i].shape[0], xs[i].shape[1]) for i in part])
+            ws_bytes = lib.kf_int4_gemm_grouped_workspace_bytes(probs, len(part), m, group_size)
+            ws = torch.empty((ws_bytes + 3) // 4, dtype=torch.float32, device=dev) if ws_bytes else None
+            status = lib.kf_int4_gemm_grouped(probs, len(part), m, group_size, _ptr(ws) if ws is not None else None,
+                                              ws_bytes, stream)
+            _lib.check(status, "int4_gemm_grouped")
+    return ys
 
 
 @torch.library.custom_op("kernelforge::int4_matmul_grouped", mutates_args=())
@@ -443,7 +479,8 @@ def int4_linear_grouped(xs: list[torch.Tensor], packed: list[torch.Tensor], scal
                         group_size: int = 128, biases: list[torch.Tensor | None] | None = None
                         ) -> list[torch.Tensor]:
     """``[int4_linear(xs[i], packed[i], scales[i], group_size, biases[i]) ...]`` with one GEMV launch
-    for all problems at decode sizes (common flattened M <= GEMV_MAX_M); results are bit-identical."""
+    for all problems at decode sizes (common flattened M <= GEMV_MAX_M) and as few GEMM launches as
+    their plans allow above; results are bit-identical."""
     flat = []
     for x in xs:
         x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])

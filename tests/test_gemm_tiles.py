@@ -21,21 +21,21 @@ DEV = "cuda"
 
 # (tile, splits, M, N, K)
 CASES = [
-    ((8, 16), 1, 5, 64, 448), ((8, 16), 1, 9, 64, 2112), ((8, 16), 8, 17, 64, 4096),
-    ((16, 16), 1, 257, 128, 448), ((16, 16), 1, 257, 128, 1088), ((16, 16), 8, 81, 64, 4096),
-    ((16, 16), 4, 79, 192, 4096), ((16, 32), 1, 385, 320, 1088), ((16, 32), 7, 33, 384, 8960),
-    ((16, 64), 1, 129, 1728, 448), ((24, 16), 1, 193, 320, 576), ((24, 16), 8, 81, 128, 6272),
-    ((32, 16), 1, 257, 256, 448), ((32, 16), 8, 97, 128, 4096), ((32, 32), 1, 513, 384, 1088),
-    ((32, 32), 5, 113, 384, 5632), ((32, 32), 1, 513, 256, 448), ((32, 32), 7, 257, 128, 4096),
-    ((32, 48), 1, 193, 1728, 832), ((32, 48), 2, 97, 1472, 4096), ((48, 16), 1, 513, 256, 576),
-    ((48, 16), 5, 129, 256, 4224), ((48, 32), 1, 385, 640, 448), ((48, 32), 5, 193, 320, 4480),
-    ((48, 48), 1, 513, 1024, 1088), ((48, 48), 4, 385, 320, 5632), ((48, 48), 1, 513, 1024, 448),
-    ((48, 48), 4, 81, 1472, 4096), ((64, 32), 1, 600, 640, 448), ((64, 32), 5, 300, 320, 4480),
-    ((64, 48), 1, 769, 768, 448), ((64, 48), 3, 513, 384, 5632), ((64, 64), 1, 385, 2048, 1344),
-    ((64, 64), 5, 300, 640, 5632), ((32, 128), 1, 769, 1024, 384), ((32, 128), 5, 513, 384, 6272),
-    ((48, 128), 1, 900, 1280, 384), ((48, 128), 5, 257, 1024, 5632), ((64, 128), 1, 900, 1728, 384),
-    ((64, 128), 5, 300, 1280, 4096), ((80, 128), 1, 900, 2560, 384), ((80, 128), 3, 769, 1024, 4096),
-    ((112, 128), 1, 900, 3072, 384), ((112, 128), 2, 900, 1472, 4096), ((128, 128), 1, 900, 4096, 640),
+    ((8, 16), 1, 17, 64, 1856), ((8, 16), 8, 17, 64, 4224), ((16, 16), 1, 129, 256, 1088),
+    ((16, 16), 8, 65, 64, 4224), ((16, 32), 1, 385, 320, 1088), ((16, 32), 3, 97, 384, 4224),
+    ((16, 64), 1, 161, 1472, 448), ((24, 16), 1, 193, 320, 576), ((24, 16), 8, 161, 64, 5632),
+    ((32, 16), 1, 193, 320, 448), ((32, 16), 8, 97, 128, 4224), ((32, 32), 1, 513, 384, 1088),
+    ((32, 32), 5, 113, 384, 4480), ((32, 48), 1, 193, 1728, 832), ((32, 48), 4, 97, 768, 5632),
+    ((48, 16), 1, 513, 256, 576), ((48, 16), 5, 257, 128, 4224), ((48, 32), 1, 385, 640, 448),
+    ((48, 32), 5, 193, 320, 4480), ((48, 48), 1, 513, 1024, 1088), ((48, 48), 4, 385, 320, 5632),
+    ((32, 32), 1, 513, 256, 448), ((32, 32), 6, 17, 1280, 4224), ((48, 48), 1, 513, 1024, 448),
+    ((48, 48), 4, 81, 1472, 4224), ((64, 32), 1, 600, 640, 448), ((64, 32), 5, 49, 1472, 4224),
+    ((64, 48), 1, 900, 640, 448), ((64, 48), 3, 161, 1280, 5632), ((64, 64), 1, 513, 1472, 1856),
+    ((64, 64), 2, 257, 1472, 4224), ((8, 16), 1, 7, 64, 448), ((16, 16), 1, 257, 128, 448),
+    ((32, 128), 1, 769, 1024, 384), ((32, 128), 5, 513, 384, 5632), ((48, 128), 1, 900, 1280, 384),
+    ((48, 128), 3, 600, 768, 4480), ((64, 128), 1, 900, 1728, 384), ((64, 128), 5, 600, 640, 4224),
+    ((80, 128), 1, 769, 2560, 384), ((80, 128), 3, 769, 1024, 4224), ((112, 128), 1, 900, 3072, 384),
+    ((112, 128), 2, 900, 1472, 4224), ((128, 128), 1, 600, 6400, 640), ((128, 128), 2, 900, 2048, 5632),
     ((128, 128), 1, 900, 2560, 448), ((128, 128), 3, 900, 2304, 6272), ((192, 256), 1, 900, 8960, 384),
 ]
 
