@@ -892,12 +892,12 @@ const CostTerms kCost[] = {
 // Split-K costs one more launch plus the fp32 partials (same fit), and is taken only when the
 // model predicts it at least 3% faster.
 constexpr double kSplitUs = 2.324, kSplitUsPerMElem = 1.624, kSplitMargin = 1.03;
-// Layers much deeper than wide (K > 4096, K >= 2.5 N) are split unless the model puts the split more
-// than 1 / 0.78 behind: there the model is too careful as often as not, and these layers' plans have
-// always asked for a workspace, which callers of the workspace entry points are written against.
-// Best unsplit / best split (us): 4096 x 14336 at M = 160: 45.1 / 34.3; 1536 x 8960 at M = 517: 33.0 /
-// 28.3; 640 x 8960 at M = 64: 9.5 / 7.9; 1536 x 8960 at M = 27: 9.0 / 9.7; the worst, 2048 x 5632 at
-// M = 64: 7.9 / 9.5 (11.6 with the kernels before).
+// Layers much deeper than wide (K > 4096, K >= 2.5 N) at 32 to 64 rows and from 896 on are split unless
+// the model puts the split more than 1 / 0.78 behind.  Their plans have always asked for a workspace, and
+// callers of the workspace entry points are written against that; it costs up to 20% (best unsplit /
+// best split, us: 2048 x 5632 at M = 64: 7.9 / 9.5, 11.6 with the kernels before; 1536 x 8960 at M = 33 and
+// 1300: 9.9 / 10.5 and 51.9 / 55.0) and gains as much where the model is too careful (640 x 8960 at M = 64:
+// 9.5 / 7.9).  Between those rows the model decides: 2048 x 5632 at M = 128 9.8 unsplit, 12.0 split.
 constexpr double kDeepSplitMargin = 0.78;
 constexpr int kMaxSplits = 8;        // the largest split count the fit was measured on
 constexpr int kMinSplitK = 512;      // k per split
@@ -908,15 +908,15 @@ constexpr size_t kMaxSplitBytes = 32u << 20;  // partials of a plan; see gemm_pl
 int gemm_num_families() { return 7; }
 
 // Kernel family reported for a configuration: streaming tiles at M <= 32 (-1), with K over 4 wavefronts
-// (0), over 8 with up to 24 rows (1), 32 rows (5) or 48 (2); DMA tiles of up to 64 rows (3), of 80 to
-// 128 rows (6); 192 x 256 (4).
+// (0), over 8 with up to 24 rows (1) or more (2); DMA tiles of 32 or 64 rows (3), 48 or 80 (5), 112 or
+// 128 (6); 192 x 256 (4).
 static int family_of(int cfg, int M) {
   if (cfg < stream_num_configs()) {
     const StreamTile t = stream_tile_of(cfg);
-    return M <= 32 ? -1 : (t.ks == 4 ? 0 : (t.bm <= 24 ? 1 : (t.bm == 32 ? 5 : 2)));
+    return M <= 32 ? -1 : (t.ks == 4 ? 0 : (t.bm <= 24 ? 1 : 2));
   }
   const int bm = kDma[cfg - stream_num_configs()].bm;
-  return bm == 192 ? 4 : (bm <= 64 ? 3 : 6);
+  return bm == 192 ? 4 : (bm >= 112 ? 6 : (bm == 48 || bm == 80 ? 5 : 3));
 }
 
 // Modelled time of `tiles` workgroups of a configuration per split.  Each XCD runs its share of the
@@ -929,8 +929,9 @@ static double plan_cost(int cfg, long tiles, int splits, int M, double n, int K,
   const double k = K * 1e-3 / splits;
   const double cost =
       t.c[0] + (t.c[1] + t.c[2] * k) * per_cu + (t.c[3] + t.c[4] * rounds) * k + t.c[5] * n * K * 1e-6;
+  const bool deep = K > 4096 && K >= 2.5 * n && ((M >= 32 && M <= 64) || M >= 896);
   return splits == 1 ? cost : (cost + kSplitUs + kSplitUsPerMElem * 1e-6 * splits * (double)M * n) *
-                                  (K > 4096 && K >= 2.5 * n ? kDeepSplitMargin : kSplitMargin);
+                                  (deep ? kDeepSplitMargin : kSplitMargin);
 }
 
 // At M <= 16 the K split over wavefronts depends on M and K alone (see gemm_plan).  Four wavefronts
