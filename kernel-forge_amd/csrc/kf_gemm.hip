@@ -949,7 +949,7 @@ static int small_m_waves(int M, int K) { return K < 2048 || (M <= 8 && K <= 4096
 //     and 3.72 / 3.68 us), so that k and v can share a launch with q, whose plan has eight.
 //   * Partials of a split are held to the scratch of kf_int4_gemm_noalloc, so that entry point takes
 //     every shape, except where K >= 16384: there a few tiles may need more splits than that.
-GemmPlan gemm_plan(int M, int N, int K, int cu_count) {
+static GemmPlan choose_plan(int M, int N, int K, int cu_count) {
   static_assert(sizeof(kCost) / sizeof(kCost[0]) == kNumStreamConfigs + kNumDma, "one cost entry per configuration");
   const int cus = cu_count > 0 ? cu_count : 256;
   const int num_stream = stream_num_configs();
@@ -986,6 +986,20 @@ GemmPlan gemm_plan(int M, int N, int K, int cu_count) {
   GemmPlan p = gemm_plan_with(best_cfg, best_splits, K);
   p.family = family_of(best_cfg, M);
   return p;
+}
+
+// The plan is a function of its arguments; each thread keeps the last ones it asked for (the workspace
+// query and the launch of a call, and a model's few shapes), which is 0.6 us of an eager call's host time.
+GemmPlan gemm_plan(int M, int N, int K, int cu_count) {
+  struct Entry {
+    int M, N, K, cus;
+    GemmPlan plan;
+  };
+  constexpr uint32_t kEntries = 64;
+  static thread_local Entry entries[kEntries];  // M = 0: empty
+  Entry& e = entries[((uint32_t)M * 0x9E3779B1u ^ (uint32_t)N * 0x85EBCA6Bu ^ (uint32_t)K * 0xC2B2AE35u) >> 26];
+  if (e.M != M || e.N != N || e.K != K || e.cus != cu_count) e = Entry{M, N, K, cu_count, choose_plan(M, N, K, cu_count)};
+  return e.plan;
 }
 
 size_t gemm_workspace_bytes(const GemmPlan& p, int M, int N) {
