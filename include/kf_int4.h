@@ -271,7 +271,7 @@ int kf_decode_argmax_step(const void* logits, int n, void* token, void* pos, voi
  * fp16 [kv_heads, head_dim, max_seq] (K transposed); cache_v fp16 [kv_heads, max_seq, head_dim]; mask
  * fp16, head h's row of max_seq additive values at mask + h * mask_stride (0: one row for all).
  * cache_v 16-byte aligned; head_dim a multiple of 8 up to KF_ATTN_MAX_HEAD_DIM, max_seq up to
- * KF_ATTN_MAX_SEQ (its scores live in LDS).  out must not alias the inputs.  No reference counterpart:
+ * KF_ATTN_MAX_SEQ.  out must not alias the inputs.  No reference counterpart:
  * the reference's decode loop runs torch's attention. */
 #define KF_ATTN_MAX_HEAD_DIM 256
 #define KF_ATTN_MAX_SEQ 8192

@@ -1,8 +1,8 @@
 """The one-launch decode attention against float64 (needs a GPU).
 
 Sizes at the edges of the kernel's loops: head sizes that divide a workgroup's lanes and ones that do
-not, odd cache lengths (single-key loads), lengths below, at and past the V steps held in registers
-and the overlap of the LDS regions, one key, the longest cache.  Error bound per element, with eps =
+not, odd cache lengths (single-key loads), lengths below, at and past a wavefront's keys and a pass over
+the cache, one key, whole wavefronts masked, the longest cache.  Error bound per element, with eps =
 2^-24: the scores carry (d + 6) eps of sum |q k| / sqrt(d) + |mask| absolute error, which the softmax
 turns into a relative error of twice that; the exponential, the sums over max_seq keys and the division
 add (max_seq + 16) eps; the result is rounded to fp16.
@@ -24,6 +24,7 @@ EPS = 2.0 ** -24
     (32, 4, 64, 160, 78), (32, 4, 64, 160, 160), (12, 2, 128, 96, 1), (4, 4, 8, 1, 1), (6, 3, 24, 33, 20),
     (2, 1, 256, 97, 97), (8, 2, 64, 191, 190), (8, 2, 64, 192, 192), (8, 8, 64, 193, 150), (4, 1, 80, 683, 683),
     (4, 2, 64, 684, 300), (4, 1, 64, 2047, 2000), (3, 1, 128, 8192, 8192),
+    (8, 2, 64, 256, 33), (8, 2, 64, 258, 257), (4, 1, 128, 130, 129),
 ])
 @pytest.mark.parametrize("one_row", [True, False], ids=["row_for_all", "row_per_head"])
 def test_against_float64(heads, kv_heads, d, max_seq, live, one_row):
