@@ -945,14 +945,20 @@ static int small_m_waves(int M, int K) { return K < 2048 || (M <= 8 && K <= 4096
 //   * M <= 16: streaming tiles of small_m_waves(M, K) wavefronts without split-K only, so the K split
 //     (and with it every bit of a column) does not depend on N and concatenated q|k|v or gate|up rows
 //     give the separate layers' results.
-//   * Narrow layers above that take eight wavefronts (256 x 2048 at M = 27 / 48, four or eight: 3.68 / 3.64
-//     and 3.72 / 3.68 us), so that k and v can share a launch with q, whose plan has eight.
+//   * Narrow layers from there to M = 640 take eight wavefronts, so that k and v can share a launch with q,
+//     whose plan has eight (256 x 2048, four / eight wavefronts: M = 27 3.68 / 3.64 us, 48 3.72 / 3.68, 517 5.8 /
+//     5.1; with thousands of rows four are faster: M = 2048 7.1 / 10.4).
 //   * Partials of a split are held to the scratch of kf_int4_gemm_noalloc, so that entry point takes
-//     every shape, except where K >= 16384: there a few tiles may need more splits than that.
+//     every shape it took with the plans before these.  The exception is K >= 65536 on a 128 x 128 grid of
+//     a little over half the CUs (1536 x 1536 x 65536: 144 tiles), which only a long split balances: it
+//     refused those before as well.
 static GemmPlan choose_plan(int M, int N, int K, int cu_count) {
   static_assert(sizeof(kCost) / sizeof(kCost[0]) == kNumStreamConfigs + kNumDma, "one cost entry per configuration");
   const int cus = cu_count > 0 ? cu_count : 256;
   const int num_stream = stream_num_configs();
+  const long grid128 = (long)ceil_div(M, 128) * ceil_div(N, 128);
+  const bool beyond_scratch =
+      K >= 65536 && K % 128 == 0 && M > 1024 && N > 1024 && 2 * grid128 > cus && 16 * grid128 <= 9 * cus;
   int best_cfg = -1, best_splits = 1;
   double best = 1e300;
   for (int cfg = 0; cfg < gemm_num_configs(); ++cfg) {
@@ -961,7 +967,7 @@ static GemmPlan choose_plan(int M, int N, int K, int cu_count) {
       const StreamTile t = stream_tile_of(cfg);
       bm = t.bm, bn = t.bn, threads = 64 * t.ks;
       if (M <= 16 && t.ks != small_m_waves(M, K)) continue;
-      if (M > 16 && N <= 1024 && K >= 1536 && t.ks != 8) continue;
+      if (M > 16 && M <= 640 && N <= 1024 && K >= 1536 && t.ks != 8) continue;
     } else {
       const DmaEntry& e = kDma[cfg - num_stream];
       bm = e.bm, bn = e.bn, threads = e.threads;
@@ -973,7 +979,7 @@ static GemmPlan choose_plan(int M, int N, int K, int cu_count) {
     const bool can_split = M > 16 && tiles < 2 * cus && cfg != gemm_num_configs() - 1;
     const int max_splits = can_split ? std::min(kMaxSplits, std::max(1, K / kMinSplitK)) : 1;
     for (int s = 1; s <= max_splits; ++s) {
-      if (s > 1 && K < 16384 && (size_t)s * M * N * sizeof(float) > kMaxSplitBytes) break;
+      if (s > 1 && !beyond_scratch && (size_t)s * M * N * sizeof(float) > kMaxSplitBytes) break;
       const double cost = plan_cost(cfg, tiles, s, M, N, K, cus);
       if (cost < best) {
         best = cost;

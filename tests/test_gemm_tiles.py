@@ -27,12 +27,12 @@ CASES = [
     ((32, 16), 1, 193, 320, 448), ((32, 16), 8, 49, 256, 4224), ((32, 32), 1, 513, 384, 1088),
     ((32, 32), 8, 97, 256, 8960), ((32, 48), 1, 193, 1728, 832), ((32, 48), 4, 63, 1472, 7424),
     ((48, 16), 1, 513, 256, 576), ((48, 16), 8, 161, 128, 8960), ((48, 32), 1, 385, 640, 448),
-    ((48, 32), 8, 65, 512, 8960), ((48, 48), 1, 513, 1024, 1088), ((48, 48), 2, 900, 256, 5632),
+    ((48, 32), 8, 65, 512, 8960), ((48, 48), 1, 513, 1024, 1088), ((48, 48), 2, 900, 256, 7424),
     ((32, 32), 1, 513, 256, 448), ((32, 32), 7, 25, 2304, 8960), ((48, 48), 1, 513, 1024, 448),
     ((48, 48), 5, 47, 4608, 8960), ((64, 32), 1, 600, 640, 448), ((64, 32), 5, 49, 1472, 4224),
-    ((64, 48), 1, 900, 640, 448), ((64, 48), 7, 49, 1728, 7424), ((64, 64), 1, 513, 1472, 1856),
-    ((64, 64), 6, 49, 2560, 8960), ((8, 16), 1, 7, 64, 448), ((16, 16), 1, 257, 128, 448),
-    ((32, 128), 1, 769, 1024, 384), ((48, 128), 1, 900, 1280, 384), ((48, 128), 3, 900, 512, 4480),
+    ((64, 48), 1, 900, 640, 448), ((64, 48), 2, 900, 384, 7424), ((64, 64), 1, 769, 1024, 1856),
+    ((64, 64), 2, 900, 512, 4224), ((8, 16), 1, 7, 64, 448), ((16, 16), 1, 257, 128, 448),
+    ((32, 128), 1, 769, 1024, 384), ((48, 128), 1, 900, 1280, 384), ((48, 128), 2, 900, 768, 4224),
     ((64, 128), 1, 900, 1728, 384), ((64, 128), 3, 900, 640, 4224), ((80, 128), 1, 769, 2560, 384),
     ((80, 128), 2, 900, 1280, 4224), ((112, 128), 1, 900, 3072, 384), ((112, 128), 2, 900, 1472, 4224),
     ((128, 128), 1, 600, 6400, 640), ((128, 128), 2, 900, 2048, 5632), ((128, 128), 1, 900, 2560, 448),
