@@ -826,7 +826,13 @@ constexpr int kNumDma = sizeof(kDma) / sizeof(kDma[0]);
 
 int gemm_num_configs() { return stream_num_configs() + kNumDma; }
 
-// Plan with an explicit configuration (streaming tiles first, then kDma) and split count.
+// Whether a configuration runs this K: the DMA tiles take whole stages (the 192 x 256 tile, pairs of them).
+static bool config_takes_k(int cfg, int K) {
+  if (cfg < stream_num_configs()) return true;
+  return K % kDma[cfg - stream_num_configs()].bk == 0 && (cfg != gemm_num_configs() - 1 || K % 128 == 0);
+}
+
+// Plan with an explicit configuration (streaming tiles first, then kDma) that takes K, and split count.
 GemmPlan gemm_plan_with(int cfg, int splits, int K) {
   GemmPlan p = {};
   p.cfg = cfg;
@@ -971,7 +977,7 @@ static GemmPlan choose_plan(int M, int N, int K, int cu_count) {
     } else {
       const DmaEntry& e = kDma[cfg - num_stream];
       bm = e.bm, bn = e.bn, threads = e.threads;
-      if (M <= 16 || K % e.bk || (cfg == gemm_num_configs() - 1 && K % 128)) continue;
+      if (M <= 16 || !config_takes_k(cfg, K)) continue;
     }
     const long tiles = (long)ceil_div(M, bm) * ceil_div(N, bn);
     if ((tiles + kXcds) * threads > 0x7FFFFFFFL) continue;
@@ -1039,6 +1045,7 @@ int gemm_group_config(const GemmPlan* plans, const int* N, int count, int M, int
   }
   int best_cfg = -1;
   for (int cfg = 0; cfg < gemm_num_configs(); ++cfg) {
+    if (!config_takes_k(cfg, K)) continue;
     const GemmPlan p = gemm_plan_with(cfg, 1, K);
     if (!gemm_same_sums(plans[0], p)) continue;
     long tiles = 0;

@@ -2,7 +2,8 @@
 
 int4_linear_grouped above the GEMV's M: siblings of one streaming kind, of the four-k-group DMA tile,
 mixtures that share nothing, problems that split K (one workspace), several K in one call, more problems
-than one call takes, different inputs, ragged M on both sides of every row-tile height, K = 64 mod 128.
+than one call takes, different inputs, ragged M on both sides of every row-tile height, K = 64 mod 128,
+and the smallest K of each group size.
 """
 
 from __future__ import annotations
@@ -23,6 +24,8 @@ SIBLINGS = {
     "wide_narrow": [(64, 1536), (8960, 1536), (192, 1536)],
     "split_and_more": [(1536, 8960), (640, 8960), (320, 4224), (2048, 2048), (64, 4224)],
     "many": [(64 * (1 + i % 3), 448) for i in range(11)],
+    "k64": [(256, 64), (256, 64), (64, 64)],
+    "k128": [(256, 128), (320, 128)],
 }
 
 
@@ -30,7 +33,7 @@ SIBLINGS = {
 @pytest.mark.parametrize("name", SIBLINGS)
 def test_bits_of_separate_launches(name, m):
     rng = np.random.Generator(np.random.PCG64(m))
-    xs, packed, scales, group = [], [], [], 64 if name == "many" else 128
+    xs, packed, scales, group = [], [], [], 64 if name in ("many", "k64") else 128
     shared = {}
     for i, (n, k) in enumerate(SIBLINGS[name]):
         p, s = o.quantize_weight((rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02)), group)
