@@ -560,7 +560,11 @@ def int4_linear(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, gro
     shape = _eager_shape(x, packed, scales, group_size) if isinstance(x, torch.Tensor) else None
     if shape is not None:
         y = _launch(x, packed, scales, int(group_size), *shape)
-        return y if bias is None else y + bias
+        if bias is None:
+            return y
+        y = y + bias
+        # A bias of more dimensions broadcasts the sum: back to the output's shape, or refused, as below.
+        return y if y.shape == shape[:2] else y.reshape(shape[:2])
     lead = x.shape[:-1]
     x2 = x.reshape(-1, x.shape[-1])
     if not x2.is_contiguous():

@@ -68,7 +68,9 @@ def _outcome(args, group, bias):
 @pytest.mark.parametrize("form", FORMS)
 def test_same_outcome_as_the_checked_path(monkeypatch, form, m, n):
     args = FORMS[form](list(_operands(m, n)))
-    for group, bias in ((G, None), (G, torch.ones(n, device=DEV).half()), (64, None), (32, None)):
+    one = torch.ones(n, device=DEV).half()
+    for group, bias in ((G, None), (G, one), (G, one.float()), (G, one.view(1, 1, n)), (G, one.expand(m, n)),
+                        (G, one.expand(7, 1, n)), (G, one[:1]), (64, None), (32, None)):
         got = _outcome(args, group, bias)
         with monkeypatch.context() as patch:
             patch.setattr(ops, "_eager_shape", lambda *a: None)
