@@ -18,6 +18,7 @@ import ctypes
 from typing import Optional
 
 import torch
+from torch.autograd import forward_ad
 from torch._subclasses.fake_tensor import FakeTensor
 
 from kernelforge import _lib
@@ -59,6 +60,14 @@ def _traced(tensors) -> bool:
     if torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0:
         return True
     return any(t is not None and type(t) not in _PLAIN for t in tensors)
+
+
+def _transformed() -> bool:
+    """True inside a functorch transform (vmap, jvp, grad, functionalize), a forward-mode level or
+    torch.jit.trace: a kernel launched on the tensors' memory would drop the tangent, the batch
+    dimension or the record of the operation, where torch's own operations keep them."""
+    return (torch._C._functorch.maybe_current_level() is not None or forward_ad._current_level >= 0
+            or torch._C._get_tracing_state() is not None)
 
 
 def _on(device: torch.device):
@@ -795,11 +804,11 @@ def decode_attention_fits(head_dim: int, max_seq: int) -> bool:
 
 
 def decode_attention_eager(q: torch.Tensor, cache_k: torch.Tensor, cache_v: torch.Tensor, mask: torch.Tensor) -> bool:
-    """Whether these operands can go to decode_attention's launch: plain tensors outside any tracer and
-    not tracked by autograd, fp16 on q's device, caches contiguous and 16-byte aligned, mask rows
-    contiguous."""
+    """Whether these operands can go to decode_attention's launch: plain tensors outside any tracer or
+    transform and not tracked by autograd, fp16 on q's device, caches contiguous and 16-byte aligned,
+    mask rows contiguous."""
     tensors = (q, cache_k, cache_v, mask)
-    if _traced(tensors) or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)):
+    if _traced(tensors) or _transformed() or (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)):
         return False
     return (all(t.dtype == torch.float16 and t.device == q.device for t in tensors) and mask.stride(-1) == 1 and
             all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in (cache_k, cache_v)))
@@ -830,8 +839,8 @@ def decode_attention(q: torch.Tensor, cache_k: torch.Tensor, cache_v: torch.Tens
             raise ValueError(f"{name} must be a contiguous fp16 tensor of {numel} elements on {q.device}")
     if mask.dtype != torch.float16 or mask.device != q.device or (max_seq > 1 and mask.stride(1) != 1):
         raise ValueError(f"mask must be fp16 on {q.device} with contiguous rows")
-    if _traced((q, cache_k, cache_v, mask)):
-        raise RuntimeError("decode_attention launches a kernel; it cannot be traced")
+    if _traced((q, cache_k, cache_v, mask)) or _transformed():
+        raise RuntimeError("decode_attention launches a kernel; it cannot be traced or transformed")
     lib = _lib.load()
     out = torch.empty_like(q)
     with _on(q.device):
