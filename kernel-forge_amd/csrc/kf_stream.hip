@@ -40,8 +40,8 @@
 // Measured on MI355X (graph replays, weights rotated through HBM), against the kernels this one
 // replaced (a skinny kernel loading fragments from memory, register-staged 16 x 64 .. 64 x 128
 // tiles): N x K = 5632 x 2048 at M = 16 / 64 / 128: 6.1 / 8.9 / 12.3 -> 4.8 / 6.4 / 8.3 us;
-// 2048 x 2048: 4.6 / 7.2 / 7.7 -> 3.6 / 4.2 / 5.1; 256 x 2048 at M = 64: 6.8 -> 3.9; 2048 x 5632 at
-// M = 16 / 64: 8.8 / 12.1 -> 6.1 / 7.6; 28672 x 4096 at M = 8: 33.5 -> 18-20.
+// 2048 x 2048: 4.6 / 7.2 / 7.7 -> 3.6 / 4.2 / 5.1; 256 x 2048 at M = 64: 6.8 -> 3.0; 2048 x 5632 at
+// M = 16 / 64: 8.8 / 12.1 -> 6.1 / 7.6; 28672 x 4096 at M = 8: 33.5 -> 17.
 #include <algorithm>
 
 #include "kf_device.h"
@@ -94,13 +94,13 @@ __device__ __forceinline__ void stream_tile(const half_t* x, const uint32_t* pac
   constexpr int XG = C::XG, TN = C::TN, KS = C::KS, PP = C::PP, WS = C::WS, WP = C::WP, TM = C::TM;
   __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS];  // static: no attribute call above 64 KiB
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int l16 = lane & 15, g = lane >> 4;
 
   // This wavefront's pieces [p0, p0 + np).
-  const int pieces = k_end - k_begin;
-  const int p0 = k_begin + (int)((long)wave * pieces / KS);
-  const int np = k_begin + (int)((long)(wave + 1) * pieces / KS) - p0;
+  const uint32_t pieces = k_end - k_begin;
+  const int p0 = k_begin + (int)(wave * pieces / KS);
+  const int np = k_begin + (int)((wave + 1) * pieces / KS) - p0;
   const int nit = (np + PP - 1) / PP, nq = (np + WP - 1) / WP;
 
   unsigned char* const my = smem + wave * C::WAVE;
@@ -257,32 +257,57 @@ __device__ __forceinline__ void stream_tile(const half_t* x, const uint32_t* pac
 
 // Workgroups are dealt to the 8 XCDs in contiguous runs of jobs (the hardware deals workgroup b to
 // XCD b % 8), split-major.  -1: no job.
-__device__ __forceinline__ int stream_job(int jobs) {
-  const int per_xcd = (jobs + kXcds - 1) / kXcds;
-  const int j = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
-  return (int)(blockIdx.x / kXcds) < per_xcd && j < jobs ? j : -1;
+__device__ __forceinline__ int stream_job(uint32_t jobs) {
+  const uint32_t per_xcd = (jobs + kXcds - 1) / kXcds;
+  const uint32_t j = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+  return blockIdx.x / kXcds < per_xcd && j < jobs ? (int)j : -1;
+}
+// Row and column tile of tile t, row tiles or column tiles as neighbours.
+__device__ __forceinline__ void stream_tile_at(uint32_t t, uint32_t tiles_m, uint32_t tiles_n, bool rows_first, int& mt,
+                                               int& nt) {
+  if (tiles_m == 1) {
+    mt = 0;
+    nt = t;
+    return;
+  }
+  const uint32_t d = rows_first ? tiles_m : tiles_n, q = t / d, r = t - q * d;
+  mt = rows_first ? r : q;
+  nt = rows_first ? q : r;
 }
 
+// The kernels of small layers live for 3-5 us, so what a workgroup does before its first copy counts:
+// the arguments fit the 14 dwords that arrive in registers (one more costs a scalar load from memory
+// first), the tile counts come from M and N, the divisions are unsigned and left out where one tile row or
+// one split makes them trivial (signed 64-bit ones were most of the time to the first copy).  N x K = 256 x
+// 2048 at M = 9 / 64: 3.8 / 3.5 -> 3.15 / 3.0 us; 2048 x 2048 at M = 6: 4.0 -> 3.4; 17920 x 1536 at M = 5: 8.2 ->
+// 7.3; 4096 x 14336 at M = 32: 18.1 -> 17.4.
 template <class C>
 __global__ __launch_bounds__(64 * C::KS) void stream_kernel(const half_t* __restrict__ x,
                                                             const uint32_t* __restrict__ packed,
                                                             const half_t* __restrict__ scales, half_t* __restrict__ y,
                                                             float* __restrict__ part, int M, int N, int K,
-                                                            int log2_group, int tiles_m, int tiles_n, int splits) {
-  const int job = stream_job(tiles_m * tiles_n * splits);
+                                                            int splits_group) {
+  constexpr uint32_t BM = 8 * C::XG, BN = 16 * C::TN;
+  const uint32_t splits = (uint32_t)splits_group >> 8;
+  const int log2_group = splits_group & 255;
+  const uint32_t tiles_m = ((uint32_t)M + BM - 1) / BM, tiles_n = ((uint32_t)N + BN - 1) / BN;
+  const uint32_t tiles = tiles_m * tiles_n;
+  const int job = stream_job(tiles * splits);
   if (job < 0) return;
-  const int tiles = tiles_m * tiles_n;
-  const int split = job / tiles, t = job - split * tiles;
+  const uint32_t pieces = (uint32_t)K >> 6;
+  uint32_t split = 0, k0 = 0, k1 = pieces;
+  if (splits > 1) {  // splits <= 8, K < 2^31: the products fit
+    split = (uint32_t)job / tiles;
+    k0 = split * pieces / splits;
+    k1 = (split + 1) * pieces / splits;
+  }
   // The larger operand is read by one XCD only as far as its L2 can serve it: with more bytes of
   // weights than of x, the row tiles of a column tile are neighbours, else the column tiles of a row
   // tile (256 x 2048 at M = 2048: 12.4 -> 6.9 us).
-  const bool rows_first = 4L * M <= N;
-  const int mt = rows_first ? t % tiles_m : t / tiles_n;
-  const int nt = rows_first ? t / tiles_m : t % tiles_n;
-  const int pieces = K >> 6;
-  const int k0 = (int)((long)split * pieces / splits), k1 = (int)((long)(split + 1) * pieces / splits);
-  stream_tile<C>(x, packed, scales, y, part ? part + (size_t)split * M * N : nullptr, M, N, K, log2_group,
-                 mt * 8 * C::XG, nt * 16 * C::TN, k0, k1, tiles_m == 1);
+  int mt, nt;
+  stream_tile_at(job - split * tiles, tiles_m, tiles_n, M <= N / 4, mt, nt);
+  stream_tile<C>(x, packed, scales, y, part ? part + (size_t)split * M * N : nullptr, M, N, K, log2_group, mt * (int)BM,
+                 nt * (int)BN, k0, k1, tiles_m == 1);
 }
 
 // Several problems of one M, K and group size in one launch: column tiles are numbered through the
@@ -295,15 +320,14 @@ __global__ __launch_bounds__(64 * C::KS) void stream_grouped_kernel(int count, i
                                                                     const GroupTable table) {
   const int job = stream_job(tiles_m * tiles_n);
   if (job < 0) return;
-  const int mt = rows_first ? job % tiles_m : job / tiles_n;
-  const int nt = rows_first ? job / tiles_m : job % tiles_n;
+  int mt, nt;
+  stream_tile_at(job, tiles_m, tiles_n, rows_first, mt, nt);
   const GroupEntry e = group_entry(table, count, nt);
   stream_tile<C>(e.x, e.packed, e.scales, e.y, nullptr, M, e.N, K, log2_group, mt * 8 * C::XG,
                  (nt - e.tile0) * 16 * C::TN, 0, K >> 6, tiles_m == 1);
 }
 
-typedef void (*StreamFn)(const half_t*, const uint32_t*, const half_t*, half_t*, float*, int, int, int, int, int, int,
-                         int);
+typedef void (*StreamFn)(const half_t*, const uint32_t*, const half_t*, half_t*, float*, int, int, int, int);
 typedef void (*StreamGroupedFn)(int, int, int, int, int, int, int, const GroupTable);
 
 struct StreamEntry {
@@ -341,8 +365,8 @@ hipError_t stream_launch(int cfg, int splits, const void* x, const void* packed,
   const int grid = ceil_div(tiles_m * tiles_n * splits, kXcds) * kXcds;
   hipLaunchKernelGGL(e.fn, dim3(grid), dim3(64 * e.ks), 0, stream, static_cast<const half_t*>(x),
                      static_cast<const uint32_t*>(packed), static_cast<const half_t*>(scales),
-                     static_cast<half_t*>(y), splits > 1 ? part : nullptr, M, N, K, group_size == 128 ? 7 : 6, tiles_m,
-                     tiles_n, splits);
+                     static_cast<half_t*>(y), splits > 1 ? part : nullptr, M, N, K,
+                     splits << 8 | (group_size == 128 ? 7 : 6));
   return hipGetLastError();
 }
 
