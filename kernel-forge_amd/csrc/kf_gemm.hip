@@ -41,11 +41,11 @@ constexpr int kXcds = 8;
 // Job of this workgroup in a 1-D grid of ceil(jobs / 8) * 8 workgroups: XCD x (= blockIdx.x % 8)
 // takes jobs x * per_xcd .. + per_xcd - 1.  Job j = split * tiles + tile.  False: no job.
 __device__ __forceinline__ bool gemm_job(int tiles, int splits, int& split, int& tile) {
-  const int jobs = tiles * splits;
-  const int per_xcd = (jobs + kXcds - 1) / kXcds;
-  const int j = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+  const uint32_t jobs = tiles * splits;
+  const uint32_t per_xcd = (jobs + kXcds - 1) / kXcds;
+  const uint32_t j = (blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
   if (j >= jobs) return false;
-  split = j / tiles;
+  split = splits > 1 ? j / (uint32_t)tiles : 0;
   tile = j - split * tiles;
   return true;
 }
@@ -529,23 +529,27 @@ __device__ __forceinline__ void dma4_tile(const half_t* x, const uint32_t* packe
 
 // Rows and columns of job t's tile: bands of group_m row tiles, all column tiles of a band before the next.
 __device__ __forceinline__ void band_tile(int t, int tiles_m, int tiles_n, int group_m, int& mt, int& nt) {
-  const int band = group_m * tiles_n;
-  const int bi = t / band;
-  const int tb = t - bi * band;
-  const int gm = min(group_m, tiles_m - bi * group_m);
-  mt = bi * group_m + tb % gm;
-  nt = tb / gm;
+  const uint32_t band = group_m * tiles_n, bi = (uint32_t)t / band, tb = t - bi * band;
+  const uint32_t gm = min(group_m, tiles_m - (int)bi * group_m);
+  nt = gm > 1 ? tb / gm : tb;
+  mt = bi * group_m + (tb - nt * gm);
 }
 
+// The arguments fit the 14 dwords that arrive in registers, as those of stream_kernel do; the tile counts
+// come from M and N.  Tiles of up to 80 rows gain 1.5-3% of their time by that: 28672 x 4096 at M = 32 21.6 -> 21.1 us,
+// 4096 x 4096 at M = 517 26.5 -> 26.0.  The non-temporal hint on weights that one row tile reads, which helps the
+// streaming tiles, costs 5-15% here (21.1 -> 23.7): a stage takes half of each 128-byte line.
 template <class C>
 __global__ __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(2)))
 void gemm_dma4_kernel(const half_t* __restrict__ x, const uint32_t* __restrict__ packed,
                       const half_t* __restrict__ scales, half_t* __restrict__ y, float* __restrict__ ws, int M, int N,
-                      int K, int log2_group, int stages_per_split, int splits, int tiles_m, int tiles_n,
-                      int group_m) {
+                      int K, uint32_t stages_splits_group) {
+  const int stages_per_split = stages_splits_group >> 8, splits = (stages_splits_group >> 4) & 15;
+  const int log2_group = stages_splits_group & 15;
+  const int tiles_m = ((uint32_t)M + C::BM - 1) / C::BM, tiles_n = ((uint32_t)N + C::BN - 1) / C::BN;
   int split, t, mt, nt;
   if (!gemm_job(tiles_m * tiles_n, splits, split, t)) return;
-  band_tile(t, tiles_m, tiles_n, group_m, mt, nt);
+  band_tile(t, tiles_m, tiles_n, max(1, tiles_m / kXcds), mt, nt);
   const int st_begin = split * stages_per_split;
   const int ns = min(K / C::BK - st_begin, stages_per_split);  // >= 1: no split is empty
   dma4_tile<C>(x, packed, scales, y, ws ? ws + (size_t)split * M * N : nullptr, M, N, K, log2_group, mt * C::BM,
@@ -800,25 +804,26 @@ __global__ __launch_bounds__(256) void splitk_reduce(const float4_t* __restrict_
 typedef void (*GemmFn)(const half_t*, const uint32_t*, const half_t*, half_t*, float*, int, int, int, int, int, int,
                        int, int, int);
 
+typedef void (*GemmDma4Fn)(const half_t*, const uint32_t*, const half_t*, half_t*, float*, int, int, int, uint32_t);
 typedef void (*GemmGroupedFn)(int, int, int, int, int, int, int, const GroupTable);
 
 // A tile of a DMA kernel: its size, k per stage and workgroup.
 struct DmaEntry {
   int bm, bn, bk, threads;
   GemmFn fn;
-  GemmGroupedFn grouped;  // four k-groups only
+  GemmDma4Fn dma4;        // four k-groups, in place of fn
+  GemmGroupedFn grouped;  // ... only
 };
 template <int TM, int TN, int NS>
 constexpr DmaEntry dma4_entry() {
   using C = Dma4Cfg<TM, TN, NS>;
-  return DmaEntry{C::BM, C::BN, C::BK, C::THREADS, gemm_dma4_kernel<C>,
-                  gemm_dma4_grouped_kernel<C>};
+  return DmaEntry{C::BM, C::BN, C::BK, C::THREADS, nullptr, gemm_dma4_kernel<C>, gemm_dma4_grouped_kernel<C>};
 }
 const DmaEntry kDma[] = {
     dma4_entry<2, 4, 4>(), dma4_entry<3, 4, 4>(), dma4_entry<4, 4, 3>(),
     dma4_entry<5, 4, 3>(), dma4_entry<7, 4, 3>(), dma4_entry<8, 4, 3>(),
-    DmaEntry{128, 128, DmaCfg::BK, DmaCfg::THREADS, gemm_dma2_kernel, nullptr},
-    DmaEntry{192, 256, WideCfg::BK, WideCfg::THREADS, gemm_wide_kernel, nullptr},
+    DmaEntry{128, 128, DmaCfg::BK, DmaCfg::THREADS, gemm_dma2_kernel, nullptr, nullptr},
+    DmaEntry{192, 256, WideCfg::BK, WideCfg::THREADS, gemm_wide_kernel, nullptr, nullptr},
 };
 constexpr int kNumDma = sizeof(kDma) / sizeof(kDma[0]);
 
@@ -1085,13 +1090,18 @@ hipError_t gemm_launch(const GemmPlan& p, const void* x, const void* packed, con
     const int tiles_m = ceil_div(M, e.bm);
     const int tiles_n = ceil_div(N, e.bn);
     const int grid_x = ceil_div(tiles_m * tiles_n * p.splits, kXcds) * kXcds;
-    // Bands of M-tiles: one band per XCD when the M-tiles divide evenly, else single rows.
-    int group_m = tiles_m / kXcds;
-    if (group_m < 1) group_m = 1;
-    hipLaunchKernelGGL(e.fn, dim3(grid_x), dim3(e.threads), 0, stream, static_cast<const half_t*>(x),
-                       static_cast<const uint32_t*>(packed), static_cast<const half_t*>(scales),
-                       static_cast<half_t*>(y), part, M, N, K, log2_group, p.kt_per_split, p.splits, tiles_m, tiles_n,
-                       group_m);
+    const half_t* xh = static_cast<const half_t*>(x);
+    const uint32_t* w = static_cast<const uint32_t*>(packed);
+    const half_t* sc = static_cast<const half_t*>(scales);
+    half_t* yh = static_cast<half_t*>(y);
+    if (e.dma4) {
+      hipLaunchKernelGGL(e.dma4, dim3(grid_x), dim3(e.threads), 0, stream, xh, w, sc, yh, part, M, N, K,
+                         (uint32_t)p.kt_per_split << 8 | p.splits << 4 | log2_group);
+    } else {
+      // Bands of M-tiles: one band per XCD when the M-tiles divide evenly, else single rows.
+      hipLaunchKernelGGL(e.fn, dim3(grid_x), dim3(e.threads), 0, stream, xh, w, sc, yh, part, M, N, K, log2_group,
+                         p.kt_per_split, p.splits, tiles_m, tiles_n, std::max(1, tiles_m / kXcds));
+    }
     err = hipGetLastError();
   }
   if (err != hipSuccess || p.splits == 1) return err;
