@@ -177,9 +177,9 @@ int kf_int4_gemm(const void* x, const void* packed, const void* scales, void* y,
  * counterpart in the reference.  The split-K partials go to a device array of
  * KF_NOALLOC_SCRATCH_BYTES that the library holds on each GPU it runs on until the process ends;
  * the call itself allocates nothing (no hipMalloc / hipFree).  Same plan, kernels and results
- * as kf_int4_gemm, bit for bit.  A problem whose plan needs more partials than the scratch holds
- * (kf_int4_gemm_workspace_bytes() > KF_NOALLOC_SCRATCH_BYTES) returns KF_ERR_WORKSPACE without
- * launching.  All calls on one GPU share its scratch: calls that overlap on that GPU (other
+ * as kf_int4_gemm, bit for bit, wherever that plan's partials fit the scratch
+ * (kf_int4_gemm_workspace_bytes() <= KF_NOALLOC_SCRATCH_BYTES); other problems run the best plan that
+ * fits, which sums K in another order.  All calls on one GPU share its scratch: calls that overlap on that GPU (other
  * streams, other threads) race; serialize them.  The first call on a device looks up the scratch
  * address (hipGetSymbolAddress) with that device current. */
 int kf_int4_gemm_noalloc(const void* x, const void* packed, const void* scales, void* y, int M, int N, int K,

@@ -121,9 +121,10 @@ int scratch_ptr(void** out) {
   return KF_OK;
 }
 
-// Validation and plan of one GEMM problem (cus: looked up once per entry point, 0 before).
+// Validation and plan of one GEMM problem (cus: looked up once per entry point, 0 before), with split-K
+// partials of at most max_partials bytes.
 int gemm_check(const void* x, const void* packed, const void* scales, const void* y, int M, int N, int K,
-               int group_size, int* cus, kf::GemmPlan* plan) {
+               int group_size, int* cus, kf::GemmPlan* plan, size_t max_partials = SIZE_MAX) {
   int st = check_common(x, packed, scales, y, M, N, K, group_size);
   if (st) return st;
   if (N % 64 != 0) return fail(KF_ERR_UNSUPPORTED, "int4_gemm needs N to be a multiple of 64, got N=%d", N);
@@ -133,6 +134,8 @@ int gemm_check(const void* x, const void* packed, const void* scales, const void
   if (!aligned(y, 16)) return fail(KF_ERR_INVALID_ARG, "int4_gemm needs y to be 16-byte aligned");
   if (*cus == 0 && (st = cu_count(cus))) return st;
   *plan = kf::gemm_plan(M, N, K, *cus);
+  if (kf::gemm_workspace_bytes(*plan, M, N) > max_partials)
+    *plan = kf::gemm_plan_within(M, N, K, *cus, max_partials);
   // One workgroup per output tile and split, all in grid dimension x.
   const long long tiles =
       (long long)((M + plan->block_m - 1) / plan->block_m) * ((N + plan->block_n - 1) / plan->block_n);
@@ -148,16 +151,11 @@ int gemm_entry(const void* x, const void* packed, const void* scales, void* y, v
                int K, int group_size, void* stream, bool use_scratch = false) {
   int cus = 0;
   kf::GemmPlan plan;
-  int st = gemm_check(x, packed, scales, y, M, N, K, group_size, &cus, &plan);
+  int st = gemm_check(x, packed, scales, y, M, N, K, group_size, &cus, &plan, use_scratch ? kScratchBytes : SIZE_MAX);
   if (st) return st;
   const size_t need = kf::gemm_workspace_bytes(plan, M, N);
   if (use_scratch) {
     ws = nullptr;
-    if (need > kScratchBytes)
-      return fail(KF_ERR_WORKSPACE,
-                  "int4_gemm_noalloc: M=%d N=%d K=%d needs %zu bytes of split-K partials, more than the %zu-byte "
-                  "scratch it holds; call kf_int4_gemm with a workspace",
-                  M, N, K, need, kScratchBytes);
     if (need > 0 && (st = scratch_ptr(&ws))) return st;
   } else if (need > 0) {
     if (!ws) return fail(KF_ERR_WORKSPACE, "split-K workspace of %zu bytes required, got NULL", need);

@@ -912,7 +912,6 @@ constexpr double kSplitUs = 2.324, kSplitUsPerMElem = 1.624, kSplitMargin = 1.03
 constexpr double kDeepSplitMargin = 0.78;
 constexpr int kMaxSplits = 8;        // the largest split count the fit was measured on
 constexpr int kMinSplitK = 512;      // k per split
-constexpr size_t kMaxSplitBytes = 32u << 20;  // partials of a plan; see gemm_plan
 
 }  // namespace
 
@@ -959,17 +958,11 @@ static int small_m_waves(int M, int K) { return K < 2048 || (M <= 8 && K <= 4096
 //   * Narrow layers from there to M = 640 take eight wavefronts, so that k and v can share a launch with q,
 //     whose plan has eight (256 x 2048, four / eight wavefronts: M = 27 3.68 / 3.64 us, 48 3.72 / 3.68, 517 5.8 /
 //     5.1; with thousands of rows four are faster: M = 2048 7.1 / 10.4).
-//   * Partials of a split are held to the scratch of kf_int4_gemm_noalloc, so that entry point takes
-//     every shape it took with the plans before these.  The exception is K >= 65536 on a 128 x 128 grid of
-//     a little over half the CUs (1536 x 1536 x 65536: 144 tiles), which only a long split balances: it
-//     refused those before as well.
-static GemmPlan choose_plan(int M, int N, int K, int cu_count) {
+//   * Partials take max_partials bytes at most; splits of 1 take none, so there is a plan for any limit.
+GemmPlan gemm_plan_within(int M, int N, int K, int cu_count, size_t max_partials) {
   static_assert(sizeof(kCost) / sizeof(kCost[0]) == kNumStreamConfigs + kNumDma, "one cost entry per configuration");
   const int cus = cu_count > 0 ? cu_count : 256;
   const int num_stream = stream_num_configs();
-  const long grid128 = (long)ceil_div(M, 128) * ceil_div(N, 128);
-  const bool beyond_scratch =
-      K >= 65536 && K % 128 == 0 && M > 1024 && N > 1024 && 2 * grid128 > cus && 16 * grid128 <= 9 * cus;
   int best_cfg = -1, best_splits = 1;
   double best = 1e300;
   for (int cfg = 0; cfg < gemm_num_configs(); ++cfg) {
@@ -990,7 +983,7 @@ static GemmPlan choose_plan(int M, int N, int K, int cu_count) {
     const bool can_split = M > 16 && tiles < 2 * cus && cfg != gemm_num_configs() - 1;
     const int max_splits = can_split ? std::min(kMaxSplits, std::max(1, K / kMinSplitK)) : 1;
     for (int s = 1; s <= max_splits; ++s) {
-      if (s > 1 && !beyond_scratch && (size_t)s * M * N * sizeof(float) > kMaxSplitBytes) break;
+      if (s > 1 && (size_t)s * M * N * sizeof(float) > max_partials) break;
       const double cost = plan_cost(cfg, tiles, s, M, N, K, cus);
       if (cost < best) {
         best = cost;
@@ -1015,7 +1008,8 @@ GemmPlan gemm_plan(int M, int N, int K, int cu_count) {
   constexpr uint32_t kEntries = 64;
   static thread_local Entry entries[kEntries];  // M = 0: empty
   Entry& e = entries[((uint32_t)M * 0x9E3779B1u ^ (uint32_t)N * 0x85EBCA6Bu ^ (uint32_t)K * 0xC2B2AE35u) >> 26];
-  if (e.M != M || e.N != N || e.K != K || e.cus != cu_count) e = Entry{M, N, K, cu_count, choose_plan(M, N, K, cu_count)};
+  if (e.M != M || e.N != N || e.K != K || e.cus != cu_count) 
+    e = Entry{M, N, K, cu_count, gemm_plan_within(M, N, K, cu_count, SIZE_MAX)};
   return e.plan;
 }
 

@@ -183,6 +183,8 @@ struct GemmPlan {
   int kt_per_split;// k stages per split (DMA tiles)
 };
 GemmPlan gemm_plan(int M, int N, int K, int cu_count);
+// ... with split-K partials of at most max_partials bytes.
+GemmPlan gemm_plan_within(int M, int N, int K, int cu_count, size_t max_partials);
 // The configuration that runs problems of these plans (one M and K) in one launch with the bits of
 // their own launches, or -1 when there is none or separate launches are predicted to be faster.
 int gemm_group_config(const GemmPlan* plans, const int* N, int count, int M, int K, int cu_count);

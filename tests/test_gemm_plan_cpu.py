@@ -1,7 +1,8 @@
-"""The GEMM's kernel choice on the host: plans and shared launches over the range of K (no GPU).
+"""The GEMM's kernel choice on the host: plans and shared launches over the range of K, plans within a limit
+on the partials (no GPU).
 
-gemm_plan and gemm_group_config are plain functions of the sizes; they are called in the built library, in a
-process of their own so that a crash in them is a failed test.
+gemm_plan, gemm_plan_within and gemm_group_config are plain functions of the sizes; they are called in the
+built library, in a process of their own so that a crash in them is a failed test.
 """
 
 from __future__ import annotations
@@ -12,7 +13,7 @@ import textwrap
 
 from kernelforge import build
 
-CALLS = textwrap.dedent("""
+HEAD = textwrap.dedent("""
     import ctypes, itertools, sys
 
     class Plan(ctypes.Structure):
@@ -21,6 +22,9 @@ CALLS = textwrap.dedent("""
     lib = ctypes.CDLL(sys.argv[1])
     plan = lib._ZN2kf9gemm_planEiiii
     plan.restype = Plan
+""")
+
+GROUPS = HEAD + textwrap.dedent("""
     group = lib._ZN2kf17gemm_group_configEPKNS_8GemmPlanEPKiiiii
     for k, m in itertools.product((64, 128, 192, 256, 320, 2048, 5632), (5, 8, 17, 64, 200, 517, 2048)):
         for ns in ((256, 256), (64, 64, 64), (64, 8960), (4096, 4096)):
@@ -29,8 +33,35 @@ CALLS = textwrap.dedent("""
             print(k, m, ns, group(plans, (ctypes.c_int * len(ns))(*ns), len(ns), m, k, 256), flush=True)
 """)
 
+WITHIN = HEAD + textwrap.dedent("""
+    within = lib._ZN2kf16gemm_plan_withinEiiiim
+    within.restype = Plan
+    limit, over = 32 << 20, 0
+    size = lambda p, m, n: p.splits * m * n * 4 if p.splits > 1 else 0
+    for m, n, k in itertools.product((17, 64, 200, 512, 1024, 1536, 2048, 4096), (64, 1024, 1536, 2560, 8192),
+                                     (64, 2048, 8192, 16384, 32768, 65536, 131072)):
+        free, held = plan(m, n, k, 256), within(m, n, k, 256, ctypes.c_size_t(limit))
+        assert size(held, m, n) <= limit and held.splits >= 1, (m, n, k, held.splits)
+        if size(free, m, n) <= limit:
+            assert bytes(free) == bytes(held), (m, n, k)
+        else:
+            over += 1
+        print(m, n, k, free.splits, held.splits, flush=True)
+    assert over
+""")
+
+
+def _run(calls: str) -> list[str]:
+    run = subprocess.run([sys.executable, "-c", calls, str(build.LIB_PATH)], capture_output=True, text=True, timeout=120)
+    assert run.returncode == 0, f"{run.returncode} after {run.stdout.splitlines()[-1:]}: {run.stderr[-500:]}"
+    return run.stdout.splitlines()
+
 
 def test_shared_launches_are_planned_for_every_k():
-    run = subprocess.run([sys.executable, "-c", CALLS, str(build.LIB_PATH)], capture_output=True, text=True, timeout=120)
-    assert run.returncode == 0, f"{run.returncode} after {run.stdout.splitlines()[-1:]}: {run.stderr[-500:]}"
-    assert len(run.stdout.splitlines()) == 7 * 7 * 4
+    assert len(_run(GROUPS)) == 7 * 7 * 4
+
+
+def test_a_limit_on_the_partials_always_has_a_plan():
+    """The limit is that of the entry point that allocates nothing: it takes every problem, with the plan of
+    the workspace entry point wherever that one fits."""
+    assert len(_run(WITHIN)) == 8 * 5 * 7

@@ -3,8 +3,8 @@
 Its split-K partials live in the library's per-GPU scratch array instead of a caller workspace.
 Checked against kf_int4_gemm (same plan and kernels, a torch-allocated workspace) bit for bit,
 on two calls in a row with split-K where the second problem is smaller (so stale partials of the
-first call sit in the scratch), on plans without split-K (tiled and skinny kernels), and on the
-refusal of a plan whose partials exceed the scratch (no launch).
+first call sit in the scratch), on plans without split-K (tiled and skinny kernels); and against float64
+where the workspace entry point's plan has more partials than the scratch holds.
 """
 
 from __future__ import annotations
@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 import torch
 
-from kernelforge import _lib
+from kernelforge import _lib, ops
 from oracle import int4_oracle as o
 
 pytestmark = pytest.mark.gpu
@@ -92,21 +92,18 @@ def test_plans_without_split_k(m, n, k):
     assert torch.equal(_noalloc(x, p, s, m, n, k), _with_workspace(x, p, s, m, n, k))
 
 
-def test_refuses_a_plan_larger_than_the_scratch():
-    """A long-K problem on few tiles splits K many ways: its partials exceed the scratch, so the
-    entry point returns KF_ERR_WORKSPACE before launching (y stays untouched)."""
-    # On 256 CUs: 128 x 128 tiles split 3 ways (60 MiB of partials), 5 ways (60 MiB), 7 ways (63 MiB).
-    for m, n, k in [(2048, 2560, 16384), (1536, 2048, 32768), (1536, 1536, 65536)]:
-        if _plan(m, n, k)[2] > _lib.KF_NOALLOC_SCRATCH_BYTES:
-            break
-    else:
-        pytest.skip("no candidate plan exceeds the scratch on this device")
-    x = torch.zeros(m, k, dtype=torch.float16, device=DEV)
-    p = torch.zeros(n, k // 8, dtype=torch.int32, device=DEV)
-    s = torch.ones(n, k // G, dtype=torch.float16, device=DEV)
-    y = torch.full((m, n), 7.0, dtype=torch.float16, device=DEV)
-    lib = _lib.load()
-    st = lib.kf_int4_gemm_noalloc(x.data_ptr(), p.data_ptr(), s.data_ptr(), y.data_ptr(), m, n, k, G, _stream())
-    assert st == _lib.KF_ERR_WORKSPACE and "scratch" in _lib.last_error()
-    torch.cuda.synchronize()
-    assert bool((y == 7.0).all())
+def test_serves_a_problem_whose_plan_exceeds_the_scratch():
+    """A long-K problem on few tiles splits K many ways: kf_int4_gemm's partials exceed the scratch, and
+    this entry point runs a plan that fits.  Error bound as in test_gemm_tiles.py."""
+    m, n, k = 2048, 2560, 16384
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert _plan(m, n, k)[2] > _lib.KF_NOALLOC_SCRATCH_BYTES
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(m, k, generator=g, device=DEV).half()
+    p, s = ops.int4_quantize(torch.randn(n, k, generator=g, device=DEV) * 0.02, G)
+    y = _noalloc(x, p, s, m, n, k)
+    w64, x64 = ops.int4_dequant_fp16(p, s, G).double(), x.double()
+    ref = x64 @ w64.T.contiguous()
+    bound = k * 2.0 ** -24 * (x64.abs() @ w64.abs().T.contiguous()) + 2.0 ** -11 * ref.abs() + 2.0 ** -24
+    err = (y.double() - ref).abs()
+    assert bool((err <= bound).all()), f"largest error / bound {float((err / bound).max()):.2f}"
