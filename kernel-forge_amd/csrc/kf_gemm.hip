@@ -992,7 +992,7 @@ GemmPlan gemm_plan_within(int M, int N, int K, int cu_count, size_t max_partials
       }
     }
   }
-  if (best_cfg < 0) best_cfg = num_stream;  // past every grid limit; the caller's check refuses it
+  if (best_cfg < 0) best_cfg = 0;  // past every grid limit, and past this one's; the caller's check refuses it
   GemmPlan p = gemm_plan_with(best_cfg, best_splits, K);
   p.family = family_of(best_cfg, M);
   return p;

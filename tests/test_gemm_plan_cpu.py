@@ -50,6 +50,13 @@ WITHIN = HEAD + textwrap.dedent("""
     assert over
 """)
 
+HUGE = HEAD + textwrap.dedent("""
+    for m, n, k in itertools.product((2 ** 26, 2 ** 30), (2 ** 20, 2 ** 30), (64, 128, 192, 4096)):
+        p = plan(m, n, k, 256)
+        assert (-(-m // p.bm) * -(-n // p.bn) * p.splits + 8) * p.threads > 2 ** 31 - 1, (m, n, k)
+        print(m, n, k, flush=True)
+""")
+
 
 def _run(calls: str) -> list[str]:
     run = subprocess.run([sys.executable, "-c", calls, str(build.LIB_PATH)], capture_output=True, text=True, timeout=120)
@@ -65,3 +72,8 @@ def test_a_limit_on_the_partials_always_has_a_plan():
     """The limit is that of the entry point that allocates nothing: it takes every problem, with the plan of
     the workspace entry point wherever that one fits."""
     assert len(_run(WITHIN)) == 8 * 5 * 7
+
+
+def test_a_problem_past_every_grid_limit_has_a_plan_that_is_past_its_own():
+    """The entry points refuse such a plan; a tile deeper than K is none."""
+    assert len(_run(HUGE)) == 2 * 2 * 4
