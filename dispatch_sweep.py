@@ -8,7 +8,7 @@ the largest M at which the sum of GEMV times over the shapes is below the sum of
 With ``--fp16`` it also times ``F.linear`` on fp16 weights of the same shape (hipBLASLt), the
 baseline the reference's bench/bench_gemm.py:83 calls ``cublas_fp16``.
 
-    python dispatch_sweep.py [--out sweep.json] [--ms 1,2,4,8,16] [--fp16] [--mfma16]
+    python dispatch_sweep.py [--out sweep.json] [--ms 1,2,4,8,16] [--fp16]
 
 A measurement harness beside bench.py, not part of the package.
 """
@@ -113,16 +113,11 @@ def main() -> None:
     ap.add_argument("--shapes", default=",".join(SHAPES))
     ap.add_argument("--out", default=None)
     ap.add_argument("--fp16", action="store_true", help="also time F.linear on fp16 weights (hipBLASLt)")
-    ap.add_argument("--mfma16", action="store_true",
-                    help="int4_gemm builds and reads the MFMA-16 weight copy (ops.MFMA16_CACHE = True); "
-                         "default: the public layout")
     args = ap.parse_args()
-    ops.MFMA16_CACHE = bool(args.mfma16)
     ms = [int(v) for v in args.ms.split(",")]
     shapes = {s: SHAPES[s] for s in args.shapes.split(",")}
     res = sweep(ms, shapes, fp16=args.fp16)
     out = {"results_us": res, "gemv_max_m": crossover(res, ms), "current_GEMV_MAX_M": ops.GEMV_MAX_M,
-           "mfma16_cache": ops.MFMA16_CACHE,
            "device": torch.cuda.get_device_name(0)}
     print(json.dumps({"gemv_max_m": out["gemv_max_m"]}), flush=True)
     if args.out:

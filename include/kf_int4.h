@@ -211,9 +211,9 @@ int kf_int4_reorder_mfma16(const void* packed, const void* scales, void* packed_
 
 /* kf_int4_gemm for a caller that holds the MFMA-16 copy of the same weight.  The kernels read
  * packed / scales: their copies of the public layout into LDS are contiguous per row and faster than
- * the skinny kernel that read the copy was (5632 x 2048 at M = 16: 4.8 us against 5.05).  Results are
- * bit-identical to kf_int4_gemm.  Same requirements, plus a valid copy and K % 128 == 0.  No
- * reference counterpart (see kf_int4_reorder_mfma16). */
+ * the skinny kernel that read the copy was (5632 x 2048 at M = 16: 4.8 us against 5.05).  The copy
+ * is not read; its pointers are checked.  Results are bit-identical to kf_int4_gemm.  Same requirements,
+ * plus K % 128 == 0.  No reference counterpart (see kf_int4_reorder_mfma16). */
 int kf_int4_gemm_mfma16(const void* x, const void* packed, const void* scales, const void* packed_r,
                         const void* scales_r, void* y, void* ws, size_t ws_bytes,
                         int M, int N, int K, int group_size, void* stream);

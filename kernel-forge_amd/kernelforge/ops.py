@@ -184,15 +184,23 @@ def _launch_gemv(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, gr
 
 
 # The MFMA-16 block copy of a weight (kf_int4_reorder_mfma16): the weight in MFMA fragment order, a
-# second copy in device memory and one host wait when it is built.  The streaming kernels read the
-# public layout through LDS in whole lines, faster than fragment-order loads of this copy were (see
-# csrc/kf_stream.hip), so kf_int4_gemm_mfma16 checks the copy and runs the same kernels.  Kept for
-# programs that use it: prepare_mfma16(packed, scales) attaches a copy to one weight, which int4_gemm
-# passes along at M <= MFMA16_MAX_M; MFMA16_CACHE = True makes int4_gemm build and attach one by itself
-# the first time a weight runs a "skinny" plan at M <= MFMA16_MAX_M (outside HIP-graph capture).
+# second copy in device memory.  No kernel reads it: the streaming kernels take the public layout through
+# LDS in whole lines, faster than fragment-order loads of the copy were (see csrc/kf_stream.hip).  The
+# layout's entry points stay for programs that hold such copies; MFMA16_CACHE and prepare_mfma16 are
+# accepted and change neither memory nor route.
 MFMA16_CACHE = False
-MFMA16_MAX_M = 32
-_MFMA16_ATTR = "_kf_mfma16"
+
+
+def _mfma16_sizes(packed: torch.Tensor, scales: torch.Tensor, group_size: int) -> tuple[int, int]:
+    """Bytes of the copy's packed words and scales, for a weight that it can be made of."""
+    if packed.dtype != torch.int32 or scales.dtype != torch.float16 or not packed.is_cuda:
+        raise TypeError("int4_reorder_mfma16 expects int32 packed and fp16 scales on a CUDA device")
+    if not packed.is_contiguous() or not scales.is_contiguous():
+        raise ValueError("packed and scales must be contiguous")
+    pb, sb = ctypes.c_size_t(), ctypes.c_size_t()
+    _lib.check(_lib.load().kf_int4_mfma16_sizes(packed.shape[0], packed.shape[1] * 8, int(group_size), ctypes.byref(pb),
+                                                ctypes.byref(sb)), "mfma16 sizes")
+    return pb.value, sb.value
 
 
 def int4_reorder_mfma16(packed: torch.Tensor, scales: torch.Tensor,
@@ -201,66 +209,21 @@ def int4_reorder_mfma16(packed: torch.Tensor, scales: torch.Tensor,
 
     An internal layout (the public packed format is unchanged); kernel csrc/kf_aux.hip.
     """
-    if packed.dtype != torch.int32 or scales.dtype != torch.float16 or not packed.is_cuda:
-        raise TypeError("int4_reorder_mfma16 expects int32 packed and fp16 scales on a CUDA device")
-    if not packed.is_contiguous() or not scales.is_contiguous():
-        raise ValueError("packed and scales must be contiguous")
+    packed_bytes, scales_bytes = _mfma16_sizes(packed, scales, group_size)
     n, k = packed.shape[0], packed.shape[1] * 8
     lib = _lib.load()
-    pb, sb = ctypes.c_size_t(), ctypes.c_size_t()
-    _lib.check(lib.kf_int4_mfma16_sizes(n, k, int(group_size), ctypes.byref(pb), ctypes.byref(sb)), "mfma16 sizes")
-    packed_r = torch.empty(pb.value // 4, dtype=torch.int32, device=packed.device)
-    scales_r = torch.empty(sb.value // 2, dtype=torch.float16, device=packed.device)
+    packed_r = torch.empty(packed_bytes // 4, dtype=torch.int32, device=packed.device)
+    scales_r = torch.empty(scales_bytes // 2, dtype=torch.float16, device=packed.device)
     with _on(packed.device):
         _lib.check(lib.kf_int4_reorder_mfma16(_ptr(packed), _ptr(scales), _ptr(packed_r), _ptr(scales_r), n, k,
                                               int(group_size), _stream_ptr(packed.device)), "int4_reorder_mfma16")
     return packed_r, scales_r
 
 
-def _mfma16_key(packed: torch.Tensor, scales: torch.Tensor, group_size: int) -> tuple:
-    """What the cached copy must match.  Tensors made under torch.inference_mode() keep no
-    version counter, so an in-place update of them cannot be seen: their key has no versions."""
-    versions = None if packed.is_inference() or scales.is_inference() else (packed._version, scales._version)
-    return (int(group_size), packed.data_ptr(), scales.data_ptr(), versions)
-
-
 def prepare_mfma16(packed: torch.Tensor, scales: torch.Tensor, group_size: int = 128) -> None:
-    """Builds the MFMA-16 copy of a weight now and keeps it on `packed` for int4_gemm.
-
-    The per-weight opt-in: int4_gemm passes the copy along at M <= MFMA16_MAX_M (with MFMA16_CACHE on it would build one by itself on first use, except for tensors
-    created under torch.inference_mode(), which have no version counter to notice in-place
-    updates: for those this is the only way, and the caller promises not to modify packed /
-    scales in place afterwards).  An in-place update of a weight with version counters makes
-    int4_gemm ignore the stale copy.  Not during HIP-graph capture.  The host waits for the copy
-    to be written before it is attached, so a later int4_gemm on any stream sees a complete copy.
-    """
-    if torch.cuda.is_current_stream_capturing():
-        raise RuntimeError("prepare_mfma16 launches a kernel and allocates; call it outside HIP-graph capture")
-    packed_r, scales_r = int4_reorder_mfma16(packed, scales, group_size)
-    done = torch.cuda.Event()
-    done.record(torch.cuda.current_stream(packed.device))
-    done.synchronize()
-    setattr(packed, _MFMA16_ATTR, (_mfma16_key(packed, scales, group_size), packed_r, scales_r))
-
-
-def _mfma16_copy(packed: torch.Tensor, scales: torch.Tensor, group_size: int, m: int):
-    """The MFMA-16 copy of (packed, scales) attached by prepare_mfma16 (or, with MFMA16_CACHE, built
-    here on first use); None when there is none or it does not apply."""
-    if m > MFMA16_MAX_M or packed.shape[1] % 16 != 0:
-        return None
-    cached = getattr(packed, _MFMA16_ATTR, None)
-    if cached is None and not MFMA16_CACHE:
-        return None
-    key = _mfma16_key(packed, scales, group_size)
-    if cached is not None and cached[0] == key:
-        return cached[1], cached[2]
-    if not MFMA16_CACHE or key[3] is None or torch.cuda.is_current_stream_capturing():
-        return None  # inference tensors: only a copy made by prepare_mfma16
-    if gemm_plan(m, packed.shape[0], packed.shape[1] * 8, group_size, packed.device)["kernel"] != "skinny":
-        return None  # copies are built for small-M plans only
-    prepare_mfma16(packed, scales, group_size)
-    cached = getattr(packed, _MFMA16_ATTR)
-    return cached[1], cached[2]
+    """Checks that the MFMA-16 copy of a weight could be made; nothing is built or kept, as no kernel reads
+    the copy (see MFMA16_CACHE)."""
+    _mfma16_sizes(packed, scales, group_size)
 
 
 def int4_gemm(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, group_size: int = 128) -> torch.Tensor:
@@ -278,7 +241,7 @@ def int4_gemm(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, group
 
 
 def _launch_gemm(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, group_size: int) -> torch.Tensor:
-    """kf_int4_gemm (or its MFMA-16-copy variant) on validated inputs."""
+    """kf_int4_gemm on validated inputs."""
     lib = _lib.load()
     m, k = x.shape
     n = packed.shape[0]
@@ -287,15 +250,9 @@ def _launch_gemm(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, gr
     with _on(dev):
         ws_bytes = lib.kf_int4_gemm_workspace_bytes(m, n, k, group_size)
         ws = torch.empty((ws_bytes + 3) // 4, dtype=torch.float32, device=dev) if ws_bytes else None
-        copy = _mfma16_copy(packed, scales, group_size, m)
-        if copy is not None:
-            status = lib.kf_int4_gemm_mfma16(_ptr(x), _ptr(packed), _ptr(scales), _ptr(copy[0]), _ptr(copy[1]),
-                                             _ptr(y), _ptr(ws) if ws is not None else None, ws_bytes, m, n, k,
-                                             group_size, _stream_ptr(dev))
-        else:
-            status = lib.kf_int4_gemm(_ptr(x), _ptr(packed), _ptr(scales), _ptr(y),
-                                      _ptr(ws) if ws is not None else None, ws_bytes, m, n, k, group_size,
-                                      _stream_ptr(dev))
+        status = lib.kf_int4_gemm(_ptr(x), _ptr(packed), _ptr(scales), _ptr(y),
+                                  _ptr(ws) if ws is not None else None, ws_bytes, m, n, k, group_size,
+                                  _stream_ptr(dev))
     _lib.check(status, "int4_gemm")
     return y
 
@@ -467,11 +424,10 @@ def _matmul_grouped(xs: list[torch.Tensor], packed: list[torch.Tensor], scales: 
 
 def _groupable(xs: list[torch.Tensor], packed: list[torch.Tensor]) -> bool:
     """Whether these problems go to kf_int4_gemm_grouped: one M above the GEMV's, one device, every N
-    a multiple of 64, and no MFMA-16 copies in use."""
+    a multiple of 64."""
     m, dev = xs[0].shape[0], xs[0].device
-    return (m > GEMV_MAX_M and len(xs) > 1 and not MFMA16_CACHE and
-            all(x.shape[0] == m and x.device == dev and p.shape[0] % 64 == 0 and not hasattr(p, _MFMA16_ATTR)
-                for x, p in zip(xs, packed)))
+    return (m > GEMV_MAX_M and len(xs) > 1 and
+            all(x.shape[0] == m and x.device == dev and p.shape[0] % 64 == 0 for x, p in zip(xs, packed)))
 
 
 def _launch_gemm_grouped(xs: list[torch.Tensor], packed: list[torch.Tensor], scales: list[torch.Tensor],
@@ -546,8 +502,6 @@ def _launch(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, group_s
         if status:
             _lib.check(status, "int4_gemv")
         return y
-    if MFMA16_CACHE or hasattr(packed, _MFMA16_ATTR):
-        return _launch_gemm(x, packed, scales, group_size)
     y = x.new_empty((m, n))
     ws_bytes = lib.kf_int4_gemm_workspace_bytes(m, n, k, group_size)
     ws = x.new_empty((ws_bytes + 3) // 4, dtype=torch.float32) if ws_bytes else None

@@ -355,21 +355,17 @@ def test_matmul_config4_grid(error_log, layer, m):
     _check(error_log, "int4_matmul", ops.int4_matmul, m, n, k, 128, f"config4_{layer}")
 
 
-@pytest.mark.parametrize("mfma16", [True, False], ids=["mfma16_copy", "public_layout"])
 @pytest.mark.parametrize("m", [2, 3, 4, 5, 6, 7])
 @pytest.mark.parametrize("layer", ["tinyllama_gate_up", "tinyllama_down"])
-def test_gemm_small_m_both_layouts(error_log, monkeypatch, layer, m, mfma16):
-    """The skinny MFMA kernel int4_matmul runs at 3 <= M <= 7 (and int4_gemm at M = 2), reading the
-    cached MFMA-16 copy or the public layout, against the oracle on config 4's gate and down."""
+def test_gemm_small_m(error_log, layer, m):
+    """int4_gemm at the rows around the GEMV / GEMM crossover, against the oracle on config 4's gate and
+    down; int4_matmul above it is the same kernel."""
     n, k = LAYER_SHAPES[layer]
-    monkeypatch.setattr(ops, "MFMA16_CACHE", mfma16)
-    assert ops.gemm_plan(m, n, k, 128)["kernel"] == "skinny"
-    _, _, dp, _ = _weights(n, k, 128)
-    out = _check(error_log, "int4_gemm", ops.int4_gemm, m, n, k, 128, f"small_m_{layer}_{'mfma16' if mfma16 else 'public'}")
-    assert (getattr(dp, ops._MFMA16_ATTR, None) is not None) or not mfma16
-    if m > ops.GEMV_MAX_M:  # the op's own route at this M is the same kernel
+    _, _, dp, ds = _weights(n, k, 128)
+    out = _check(error_log, "int4_gemm", ops.int4_gemm, m, n, k, 128, f"small_m_{layer}")
+    if m > ops.GEMV_MAX_M:
         x = torch.from_numpy(_x(m, k, m * 7 + n + k)).to(DEV)
-        assert torch.equal(ops.int4_matmul(x, dp, _weights(n, k, 128)[3], 128), out)
+        assert torch.equal(ops.int4_matmul(x, dp, ds, 128), out)
 
 
 def test_matmul_ragged_n_follows_the_reference_dispatch():

@@ -1,10 +1,10 @@
-"""MFMA-16 block copy of a weight (kf_int4_reorder_mfma16, kf_int4_gemm_mfma16) and the op-level
-cache behind int4_gemm (needs a GPU).
+"""MFMA-16 block copy of a weight (kf_int4_reorder_mfma16, kf_int4_gemm_mfma16) and the options that once
+attached one to a weight (needs a GPU).
 
 The copy is a pure permutation, checked bit for bit against the oracle's statement of the layout
-(oracle/int4_oracle.py:reorder_mfma16, itself pinned element by element in test_oracle.py).  The
-GEMM reading it must equal the GEMM reading the public layout bit for bit: same dequantization,
-same MFMA order, same fixed-order reduction.
+(oracle/int4_oracle.py:reorder_mfma16, itself pinned element by element in test_oracle.py).  No kernel
+reads it: the GEMM entry point that takes one gives kf_int4_gemm's result whatever the copy holds, and the
+options change neither memory nor route.
 """
 
 from __future__ import annotations
@@ -57,103 +57,55 @@ def test_reorder_matches_oracle(n, k, g):
     assert np.array_equal(sr.cpu().numpy().view(np.uint16), want_s.view(np.uint16))
 
 
-# gate, wide_a and wide_b take two 16-column blocks per skinny workgroup on 256 CUs
-# (SkinnyPlan::col_blocks; N is a multiple of 64 on the GEMM path, so those workgroups are whole).
-LAYERS = {"qo": (2048, 2048), "kv": (256, 2048), "gate": (5632, 2048), "down": (2048, 5632),
-          "qwen_down": (1536, 8960), "ragged": (320, 1152), "wide_a": (4160, 2048), "wide_b": (6016, 1024)}
-
-
-@pytest.mark.parametrize("layer", list(LAYERS))
 @pytest.mark.parametrize("g", [64, 128])
-def test_gemm_with_copy_is_bit_identical(layer, g):
-    """Every M of the skinny range (plus one tiled M, where the copy is not read)."""
-    n, k = LAYERS[layer]
+@pytest.mark.parametrize("m", [1, 8, 16, 64])
+def test_gemm_with_copy_does_not_read_it(m, g):
+    n, k = 320, 1152
     packed, scales, dp, ds = _weight(n, k, g)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).half()
     copy = ops.int4_reorder_mfma16(dp, ds, g)
-    skinny_seen = 0
-    for m in (1, 2, 3, 5, 8, 9, 13, 16, 17, 24, 32, 64):
-        x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).half().to(DEV)
-        ref = _gemm_raw(x, dp, ds, g)
-        got = _gemm_raw(x, dp, ds, g, copy)
-        assert torch.equal(got, ref), f"{layer} M={m}"
-        skinny_seen += ops.gemm_plan(m, n, k, g)["kernel"] == "skinny"
-    assert skinny_seen >= 5
-    # and against the oracle at one M, so the check is not only self-consistency
-    x = o.seeded_case(8, n, k, g, seed=3)[1]
-    y = _gemm_raw(torch.from_numpy(x).to(DEV), dp, ds, g, copy).float().cpu().numpy()
-    assert o.max_rel_err(y, o.linear_ref_fp32(x, packed, scales, g)) <= 2e-3
+    ref = _gemm_raw(x.to(DEV), dp, ds, g)
+    assert torch.equal(_gemm_raw(x.to(DEV), dp, ds, g, copy), ref)
+    copy[0].fill_(-1)
+    copy[1].fill_(float("nan"))
+    assert torch.equal(_gemm_raw(x.to(DEV), dp, ds, g, copy), ref)
+    assert o.max_rel_err(ref.float().cpu().numpy(), o.linear_ref_fp32(x.numpy(), packed, scales, g)) <= 2e-3
 
 
-def test_op_cache_builds_reuses_and_invalidates():
-    n, k, g = 2048, 2048, 128
-    _, _, dp, ds = _weight(n, k, g)
-    x = torch.randn(8, k, device=DEV).half()
-    old = ops.MFMA16_CACHE
-    try:
-        ops.MFMA16_CACHE = False
-        plain = ops.int4_gemm(x, dp, ds, g)
-        assert getattr(dp, "_kf_mfma16", None) is None
-        ops.MFMA16_CACHE = True
-        y1 = ops.int4_gemm(x, dp, ds, g)
-        first = getattr(dp, "_kf_mfma16")
-        y2 = ops.int4_gemm(x, dp, ds, g)
-        assert getattr(dp, "_kf_mfma16") is first  # reused
-        assert torch.equal(y1, plain) and torch.equal(y2, plain)
-        # an in-place update of the weight invalidates the copy
-        packed2, scales2, dp2, ds2 = _weight(n, k, g, seed=9)
-        dp.copy_(dp2)
-        ds.copy_(ds2)
-        y3 = ops.int4_gemm(x, dp, ds, g)
-        assert getattr(dp, "_kf_mfma16") is not first
-        assert torch.equal(y3, ops.int4_gemm(x, dp2, ds2, g))
-        # a tiled-kernel M builds nothing
-        _, _, dp3, ds3 = _weight(5632, 2048, g, seed=4)
-        ops.int4_gemm(torch.randn(64, 2048, device=DEV).half(), dp3, ds3, g)
-        assert getattr(dp3, "_kf_mfma16", None) is None
-    finally:
-        ops.MFMA16_CACHE = old
+@pytest.mark.parametrize("m", [4, 8, 64])
+def test_options_change_neither_memory_nor_route(monkeypatch, m):
+    g, k = 128, 2048
+    weights = [_weight(n, k, g, seed=n)[2:] for n in (2048, 256, 256)]
+    x = torch.randn(m, k, device=DEV).half()
+    lib, launched = _lib.load(), []
 
+    class Spy:
+        def __getattr__(self, name):
+            if "workspace" not in name:
+                launched.append(name)
+            return getattr(lib, name)
 
-def test_default_builds_no_copy_but_uses_a_prepared_one():
-    """The copy is opt-in: by default int4_gemm attaches nothing; a copy attached with
-    prepare_mfma16 is read (same bits) and ignored once the weight is updated in place."""
-    assert ops.MFMA16_CACHE is False
-    n, k, g = 2048, 2048, 128
-    _, _, dp, ds = _weight(n, k, g, seed=5)
-    x = torch.randn(8, k, device=DEV).half()
-    plain = ops.int4_gemm(x, dp, ds, g)
-    assert getattr(dp, "_kf_mfma16", None) is None
-    ops.prepare_mfma16(dp, ds, g)
-    copy = getattr(dp, "_kf_mfma16")
-    assert torch.equal(ops.int4_gemm(x, dp, ds, g), plain) and getattr(dp, "_kf_mfma16") is copy
-    _, _, dp2, ds2 = _weight(n, k, g, seed=6)
-    dp.copy_(dp2)
-    ds.copy_(ds2)
-    assert torch.equal(ops.int4_gemm(x, dp, ds, g), ops.int4_gemm(x, dp2, ds2, g))
-    assert getattr(dp, "_kf_mfma16") is copy  # stale, not rebuilt without MFMA16_CACHE, not read
+    def call():
+        launched.clear()
+        ys = [ops.int4_linear(x, *weights[0], g),
+              *ops.int4_linear_grouped([x] * 3, [p for p, _ in weights], [s for _, s in weights], g)]
+        torch.cuda.synchronize()
+        return ys, list(launched), torch.cuda.memory_allocated()
 
-
-def test_graph_capture_uses_cached_copy(monkeypatch):
+    monkeypatch.setattr(ops._lib, "load", Spy)
+    call()  # whatever the first call sets up
+    ys, route, memory = call()
+    expected = ["kf_int4_gemv", "kf_int4_gemv_grouped"] if m <= ops.GEMV_MAX_M else ["kf_int4_gemm", "kf_int4_gemm_grouped"]
+    assert route == expected
     monkeypatch.setattr(ops, "MFMA16_CACHE", True)
-    n, k, g = 5632, 2048, 128
-    _, _, dp, ds = _weight(n, k, g)
-    static_x = torch.randn(4, k, device=DEV).half()
-    eager = ops.int4_gemm(static_x, dp, ds, g)  # builds the copy outside capture
-    assert getattr(dp, "_kf_mfma16", None) is not None
-    s = torch.cuda.Stream()
-    s.wait_stream(torch.cuda.current_stream())
-    with torch.cuda.stream(s):
-        ops.int4_gemm(static_x, dp, ds, g)
-    torch.cuda.current_stream().wait_stream(s)
-    graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
-        static_y = ops.int4_gemm(static_x, dp, ds, g)
-    for i in range(3):
-        graph.replay()
-        torch.cuda.synchronize()
-        assert torch.equal(static_y, eager), f"replay {i}"
-        ops.int4_gemm(static_x, dp, ds, g)
-        torch.cuda.synchronize()
+    for p, s in weights:
+        ops.prepare_mfma16(p, s, g)
+    again, route2, memory2 = call()
+    assert route2 == route and all(torch.equal(a, b) for a, b in zip(again, ys))
+    assert memory2 == memory + sum(y.untyped_storage().nbytes() for y in ys)  # the first results are still held
+    # An in-place update of a weight is what the next call computes with.
+    weights[0][0].copy_(_weight(2048, k, g, seed=9)[2])
+    assert not torch.equal(call()[0][0], ys[0])
 
 
 def test_mfma16_rejections():
@@ -170,16 +122,9 @@ def test_mfma16_rejections():
         ops.int4_reorder_mfma16(dp.float(), ds, 128)
 
 
-def test_inference_mode_weights_use_only_a_prepared_copy():
-    """Inference tensors carry no version counter: no implicit copy; prepare_mfma16 opts in."""
-    n, k, g = 2048, 2048, 128
-    packed, scales, _, _ = _weight(n, k, g)
-    with torch.inference_mode():
-        dp = torch.from_numpy(packed).to(DEV)
-        ds = torch.from_numpy(scales).to(DEV)
-        x = torch.randn(8, k, device=DEV).half()
-        plain = ops.int4_gemm(x, dp, ds, g)
-        assert getattr(dp, "_kf_mfma16", None) is None
-        ops.prepare_mfma16(dp, ds, g)
-        assert getattr(dp, "_kf_mfma16", None) is not None
-        assert torch.equal(ops.int4_gemm(x, dp, ds, g), plain)
+def test_prepare_refuses_what_has_no_copy():
+    _, _, dp, ds = _weight(64, 192, 64)
+    with pytest.raises(ValueError, match="multiple of 128"):
+        ops.prepare_mfma16(dp, ds, 64)
+    with pytest.raises(TypeError):
+        ops.prepare_mfma16(dp.float(), ds, 64)
