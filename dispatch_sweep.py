@@ -80,7 +80,7 @@ def sweep(ms: list[int], shapes: dict, group: int = 128, fp16: bool = False) -> 
             if n % 64 == 0:
                 row["gemm_us"] = time_us(lambda c: ops.int4_gemm(x, dev[c][0], dev[c][1], group), copies)
                 plan = ops.gemm_plan(m, n, k, group)
-                row["gemm_kernel"] = f"{plan['kernel']}/{plan['splits']}"  # tile-table index (or skinny) / splits
+                row["gemm_kernel"] = f"{plan['kernel']}/{plan['splits']}"  # configuration / splits
             row["tflops_best"] = 2 * m * n * k / min(v for kk, v in row.items() if kk.endswith("_us")) / 1e6
             if w16:
                 row["fp16_us"] = time_us(lambda c: torch.nn.functional.linear(x, w16[c]), len(w16))

@@ -151,11 +151,11 @@ int kf_int4_gemv_qkv_rope(const void* x, const void* packed, const void* scales,
  * which counted floats instead of bytes. */
 size_t kf_int4_gemm_workspace_bytes(int M, int N, int K, int group_size);
 
-/* The kernel kf_int4_gemm() runs for (M, N, K, G) on the current device: *kernel is
- * KF_GEMM_SKINNY (a streaming tile at M <= 32) or the index of a kernel family in [0, *num_kernels)
- * (kf_gemm.hip lists them), *splits the split-K factor (1 = no workspace), *block_m x *block_n the
- * output tile.  Any output pointer may be NULL.  For diagnostics and tests; no reference counterpart. */
-#define KF_GEMM_SKINNY (-1)
+/* The kernel kf_int4_gemm() runs for (M, N, K, G) on the current device: *kernel is the index of its
+ * configuration in [0, *num_kernels) (the streaming tiles of kf_stream.hip, then the LDS-DMA tiles of
+ * kf_gemm.hip, in the order of their tables; tiles of one size with four and eight wavefronts are two
+ * configurations), *splits the split-K factor (1 = no workspace), *block_m x *block_n the output tile.  Any
+ * output pointer may be NULL.  For diagnostics and tests; no reference counterpart. */
 int kf_int4_gemm_plan(int M, int N, int K, int group_size, int* kernel, int* num_kernels,
                       int* splits, int* block_m, int* block_n);
 

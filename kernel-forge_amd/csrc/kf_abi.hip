@@ -378,8 +378,8 @@ int kf_int4_gemm_plan(int M, int N, int K, int group_size, int* kernel, int* num
   const int st = cu_count(&cus);
   if (st) return st;
   const kf::GemmPlan p = kf::gemm_plan(M, N, K, cus);
-  if (kernel) *kernel = p.family;
-  if (num_kernels) *num_kernels = kf::gemm_num_families();
+  if (kernel) *kernel = p.cfg;
+  if (num_kernels) *num_kernels = kf::gemm_num_configs();
   if (splits) *splits = p.splits;
   if (block_m) *block_m = p.block_m;
   if (block_n) *block_n = p.block_n;

@@ -915,20 +915,6 @@ constexpr int kMinSplitK = 512;      // k per split
 
 }  // namespace
 
-int gemm_num_families() { return 7; }
-
-// Kernel family reported for a configuration: streaming tiles at M <= 32 (-1), with K over 4 wavefronts
-// (0), over 8 with up to 24 rows (1) or more (2); DMA tiles of 32 or 64 rows (3), 48 or 80 (5), 112 or
-// 128 (6); 192 x 256 (4).
-static int family_of(int cfg, int M) {
-  if (cfg < stream_num_configs()) {
-    const StreamTile t = stream_tile_of(cfg);
-    return M <= 32 ? -1 : (t.ks == 4 ? 0 : (t.bm <= 24 ? 1 : 2));
-  }
-  const int bm = kDma[cfg - stream_num_configs()].bm;
-  return bm == 192 ? 4 : (bm >= 112 ? 6 : (bm == 48 || bm == 80 ? 5 : 3));
-}
-
 // Modelled time of `tiles` workgroups of a configuration per split.  Each XCD runs its share of the
 // workgroups, spread over its CUs.
 static double plan_cost(int cfg, long tiles, int splits, int M, double n, int K, int cus) {
@@ -993,9 +979,7 @@ GemmPlan gemm_plan_within(int M, int N, int K, int cu_count, size_t max_partials
     }
   }
   if (best_cfg < 0) best_cfg = 0;  // past every grid limit, and past this one's; the caller's check refuses it
-  GemmPlan p = gemm_plan_with(best_cfg, best_splits, K);
-  p.family = family_of(best_cfg, M);
-  return p;
+  return gemm_plan_with(best_cfg, best_splits, K);
 }
 
 // The plan is a function of its arguments; each thread keeps the last ones it asked for (the workspace

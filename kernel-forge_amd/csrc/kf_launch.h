@@ -175,7 +175,6 @@ hipError_t reorder_mfma16_launch(const void* packed, const void* scales, void* p
 // ---- MFMA GEMM (any M, N % 64 == 0) --------------------------------------
 struct GemmPlan {
   int cfg;         // configuration: streaming tiles first, then the DMA tiles (kf_gemm.hip)
-  int family;      // kernel family reported by kf_int4_gemm_plan (-1: streaming tiles at M <= 32)
   int block_m;     // output tile
   int block_n;
   int threads;     // workgroup size
@@ -195,7 +194,6 @@ bool gemm_same_sums(const GemmPlan& a, const GemmPlan& b);
 // Plan with an explicit configuration and split count (tuning).
 GemmPlan gemm_plan_with(int cfg, int splits, int K);
 int gemm_num_configs();
-int gemm_num_families();
 size_t gemm_workspace_bytes(const GemmPlan& p, int M, int N);
 hipError_t gemm_launch(const GemmPlan& p, const void* x, const void* packed, const void* scales, void* y,
                        void* ws, int M, int N, int K, int group_size, hipStream_t stream);

@@ -260,8 +260,9 @@ def _launch_gemm(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, gr
 def gemm_plan(m: int, n: int, k: int, group_size: int = 128, device: torch.device | None = None) -> dict:
     """The kernel int4_gemm runs for an [m, k] x [n, k]^T problem on `device` (default: current).
 
-    Returns {"kernel": "skinny" (a streaming tile at M <= 32) or the kernel family's index,
-    "num_kernels": families, "splits": split-K factor, "tile": (BM, BN)}.  Diagnostics; no reference counterpart.
+    Returns {"kernel": the configuration's index (the streaming tiles, then the LDS-DMA tiles),
+    "num_kernels": configurations, "splits": split-K factor, "tile": (BM, BN)}.  Diagnostics; no reference
+    counterpart.
     """
     lib = _lib.load()
     out = [ctypes.c_int() for _ in range(5)]
@@ -269,7 +270,7 @@ def gemm_plan(m: int, n: int, k: int, group_size: int = 128, device: torch.devic
         status = lib.kf_int4_gemm_plan(int(m), int(n), int(k), int(group_size), *[ctypes.byref(v) for v in out])
     _lib.check(status, "gemm_plan")
     kernel, num, splits, bm, bn = (v.value for v in out)
-    return {"kernel": "skinny" if kernel < 0 else kernel, "num_kernels": num, "splits": splits, "tile": (bm, bn)}
+    return {"kernel": kernel, "num_kernels": num, "splits": splits, "tile": (bm, bn)}
 
 
 def int4_matmul(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, group_size: int = 128) -> torch.Tensor:

@@ -17,7 +17,7 @@ HEAD = textwrap.dedent("""
     import ctypes, itertools, sys
 
     class Plan(ctypes.Structure):
-        _fields_ = [(f, ctypes.c_int) for f in ("cfg", "family", "bm", "bn", "threads", "splits", "stages")]
+        _fields_ = [(f, ctypes.c_int) for f in ("cfg", "bm", "bn", "threads", "splits", "stages")]
 
     lib = ctypes.CDLL(sys.argv[1])
     plan = lib._ZN2kf9gemm_planEiiii

@@ -1,8 +1,8 @@
-"""Every tile of int4_gemm at its edges against an exact reference (needs a GPU).
+"""Every configuration of int4_gemm at its edges against an exact reference (needs a GPU).
 
-Shapes are the smallest that the dispatcher gives to each tile on a 256-CU device, with rows left over in
-the last row tile, columns in the last column tile where N allows it, K = 64 mod 128 where the tile takes
-it, and one split-K case per tile that splits.  The reference is float64 on the operand the kernels
+Shapes are small ones that the dispatcher gives to each configuration (tile, wavefronts, kernel) on a 256-CU
+device, with rows left over in the last row tile, columns in the last column tile where N allows it, K = 64
+mod 128 where the tile takes it, and one split-K case per configuration that splits.  The reference is float64 on the operand the kernels
 use, W = fp16(q * s).  Error bound per element: K fp32 additions of exact products, and the fp16
 rounding of the result: K 2^-24 sum |x w| + 2^-11 |y| (+ the smallest fp16 step).
 """
@@ -19,33 +19,34 @@ from oracle import int4_oracle as o
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
 
-# (tile, splits, M, N, K)
+# (configuration, tile, splits, M, N, K)
 CASES = [
-    ((8, 16), 1, 17, 64, 1856), ((8, 16), 8, 33, 64, 4224), ((16, 16), 1, 129, 256, 1088),
-    ((16, 16), 8, 33, 128, 4224), ((16, 32), 1, 385, 320, 1088), ((16, 32), 7, 33, 384, 8960),
-    ((16, 64), 1, 161, 1472, 448), ((24, 16), 1, 193, 320, 576), ((24, 16), 8, 81, 128, 7424),
-    ((32, 16), 1, 193, 320, 448), ((32, 16), 8, 49, 256, 4224), ((32, 32), 1, 513, 384, 1088),
-    ((32, 32), 8, 97, 256, 8960), ((32, 48), 1, 193, 1728, 832), ((32, 48), 4, 63, 1472, 7424),
-    ((48, 16), 1, 513, 256, 576), ((48, 16), 8, 161, 128, 8960), ((48, 32), 1, 385, 640, 448),
-    ((48, 32), 8, 65, 512, 8960), ((48, 48), 1, 513, 1024, 1088), ((48, 48), 2, 900, 256, 7424),
-    ((32, 32), 1, 513, 256, 448), ((32, 32), 7, 25, 2304, 8960), ((48, 48), 1, 513, 1024, 448),
-    ((48, 48), 5, 47, 4608, 8960), ((64, 32), 1, 600, 640, 448), ((64, 32), 5, 49, 1472, 4224),
-    ((64, 48), 1, 900, 640, 448), ((64, 48), 2, 900, 384, 7424), ((64, 64), 1, 769, 1024, 1856),
-    ((64, 64), 2, 900, 512, 4224), ((8, 16), 1, 7, 64, 448), ((16, 16), 1, 257, 128, 448),
-    ((32, 128), 1, 769, 1024, 384), ((48, 128), 1, 900, 1280, 384), ((48, 128), 2, 900, 768, 4224),
-    ((64, 128), 1, 900, 1728, 384), ((64, 128), 3, 900, 640, 4224), ((80, 128), 1, 769, 2560, 384),
-    ((80, 128), 2, 900, 1280, 4224), ((112, 128), 1, 900, 3072, 384), ((112, 128), 2, 900, 1472, 4224),
-    ((128, 128), 1, 600, 6400, 640), ((128, 128), 2, 900, 2048, 5632), ((128, 128), 1, 900, 2560, 448),
-    ((128, 128), 3, 900, 2304, 6272), ((192, 256), 1, 900, 8960, 384),
+    (0, (8, 16), 1, 9, 64, 2112), (0, (8, 16), 8, 33, 64, 4160), (1, (16, 16), 1, 17, 1472, 1088),
+    (1, (16, 16), 8, 33, 128, 4160), (2, (16, 32), 1, 33, 2304, 832), (2, (16, 32), 7, 33, 384, 8960),
+    (3, (16, 64), 1, 33, 4608, 192), (4, (24, 16), 1, 17, 2304, 832), (4, (24, 16), 5, 33, 384, 4160),
+    (5, (32, 16), 1, 17, 2304, 192), (5, (32, 16), 8, 49, 256, 4160), (6, (32, 32), 1, 49, 2304, 1088),
+    (6, (32, 32), 5, 49, 768, 4224), (7, (32, 48), 1, 17, 8960, 448), (7, (32, 48), 8, 17, 1472, 14336),
+    (8, (48, 16), 1, 33, 3072, 576), (8, (48, 16), 6, 33, 640, 4160), (9, (48, 32), 1, 33, 4608, 576),
+    (9, (48, 32), 5, 33, 1472, 4160), (10, (48, 48), 1, 385, 1280, 1088), (10, (48, 48), 5, 769, 128, 11520),
+    (11, (32, 32), 1, 7, 4608, 192), (11, (32, 32), 7, 17, 2304, 11520), (12, (48, 48), 1, 33, 8960, 192),
+    (12, (48, 48), 2, 1025, 512, 5632), (13, (64, 32), 1, 33, 6400, 192), (13, (64, 32), 5, 49, 1472, 4160),
+    (14, (64, 48), 1, 49, 8960, 320), (14, (64, 48), 8, 49, 1472, 11520), (15, (64, 64), 1, 97, 6400, 832),
+    (15, (64, 64), 2, 1025, 384, 4160), (16, (8, 16), 1, 7, 64, 448), (17, (16, 16), 1, 7, 64, 192),
+    (18, (32, 128), 1, 385, 1472, 128), (18, (32, 128), 7, 193, 640, 14336), (19, (48, 128), 1, 600, 1728, 128),
+    (19, (48, 128), 6, 129, 1728, 11520), (20, (64, 128), 1, 1025, 1472, 128), (20, (64, 128), 8, 97, 1728, 14336),
+    (21, (80, 128), 1, 1301, 1728, 128), (21, (80, 128), 7, 900, 320, 11520), (22, (112, 128), 1, 2047, 1472, 384),
+    (22, (112, 128), 2, 900, 1472, 4224), (23, (128, 128), 1, 2047, 1728, 640),
+    (23, (128, 128), 5, 2047, 320, 14336), (24, (128, 128), 1, 1025, 1728, 192),
+    (24, (128, 128), 5, 900, 1472, 4160), (25, (192, 256), 1, 900, 4608, 128),
 ]
 
 
-@pytest.mark.parametrize("tile,splits,m,n,k", CASES)
-def test_tile_edges(tile, splits, m, n, k):
+@pytest.mark.parametrize("config,tile,splits,m,n,k", CASES)
+def test_tile_edges(config, tile, splits, m, n, k):
     group = 128 if k % 128 == 0 else 64
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
         plan = ops.gemm_plan(m, n, k, group)
-        assert (plan["tile"], plan["splits"]) == (tile, splits)
+        assert (plan["kernel"], plan["tile"], plan["splits"]) == (config, tile, splits)
     rng = np.random.Generator(np.random.PCG64(m * 7 + n + k))
     w = (rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02)).astype(np.float32)
     packed, scales = o.quantize_weight(w, group)
@@ -57,3 +58,8 @@ def test_tile_edges(tile, splits, m, n, k):
     out = ops.int4_gemm(x.to(DEV), torch.from_numpy(packed).to(DEV), torch.from_numpy(scales).to(DEV), group)
     err = (out.to(torch.float64) - ref).abs()
     assert bool((err <= bound).all()), f"largest error / bound {float((err / bound).max()):.2f}"
+
+
+def test_every_configuration_has_a_case():
+    num = ops.gemm_plan(64, 2048, 2048)["num_kernels"]
+    assert {c[0] for c in CASES} == set(range(num))

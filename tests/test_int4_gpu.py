@@ -318,24 +318,28 @@ def test_gemm_n_multiple_of_64_not_128(error_log, n):
     _check(error_log, "int4_gemm", ops.int4_gemm, 37, n, 512, 64, f"n{n}")
 
 
-# Ragged shapes that reach every tile-table kernel, with and without split-K: N not a multiple
-# of the tile width, M just past a tile boundary, K % 256 != 0 (no 256-k-stage tile) and
-# K % 128 != 0.  (M, N, K) -> kernel/splits as the dispatcher picks them on 256 CUs.
+# Ragged shapes over the streaming and the LDS-DMA tiles, with and without split-K: N not a multiple
+# of the tile width, M just past a tile boundary, K % 128 != 0.  (Every configuration by itself:
+# test_gemm_tiles.py.)
 EDGE_CASES = [(513, 2112, 384), (1000, 320, 4224), (1000, 2112, 384), (1500, 640, 8960), (33, 64, 1152),
               (33, 320, 4224), (300, 960, 2048), (33, 192, 2304), (33, 640, 8960), (47, 704, 5120),
               (130, 1600, 640), (65, 192, 4160), (900, 1472, 6272), (600, 1216, 7424), (1300, 6080, 640)]
 
 
 @pytest.mark.parametrize("m,n,k,group", [(m, n, k, g) for m, n, k in EDGE_CASES for g in (64, 128) if k % g == 0])
-def test_gemm_edge_shapes_every_tile(error_log, m, n, k, group):
+def test_gemm_edge_shapes(error_log, m, n, k, group):
     _check(error_log, "int4_gemm", ops.int4_gemm, m, n, k, group, f"edge_{m}x{n}x{k}")
 
 
-def test_edge_shapes_reach_every_tile_and_split():
+def _kinds(plans):
+    """(streaming or LDS-DMA tile, splits K) of each plan: the DMA tiles are 128 or 256 columns wide."""
+    return {("dma" if p["tile"][1] >= 128 else "stream", p["splits"] > 1) for p in plans}
+
+
+def test_edge_shapes_reach_both_kinds_of_tile_and_split_k():
     plans = [ops.gemm_plan(m, n, k, 64) for m, n, k in EDGE_CASES]
-    num = plans[0]["num_kernels"]
-    assert {p["kernel"] for p in plans} == set(range(num))
-    assert {p["kernel"] for p in plans if p["splits"] > 1} >= {1, 2, 3, 5, 6}
+    assert _kinds(plans) == {("stream", False), ("stream", True), ("dma", False), ("dma", True)}
+    assert len({p["kernel"] for p in plans}) >= 8
 
 
 @pytest.mark.parametrize("m", [1, 8, 9, 128])
@@ -392,7 +396,7 @@ def test_gemm_rejects_n_not_multiple_of_64():
                                              ("qwen_down", 1536, True), ("tinyllama_gate_up", 16, False),
                                              ("tinyllama_gate_up", 768, False)])
 def test_gemm_is_deterministic(layer, m, splitk):
-    """Split-K partials, the DMA kernel's in-block k-group halves and the skinny kernel's
+    """Split-K partials, the DMA kernel's in-block k-group halves and the streaming tiles'
     per-wave K slices are reduced in fixed order: repeated calls are bitwise identical."""
     n, k = LAYER_SHAPES[layer]
     _, _, dp, ds = _weights(n, k, 128)
@@ -403,20 +407,13 @@ def test_gemm_is_deterministic(layer, m, splitk):
     assert all(torch.equal(outs[0], o_) for o_ in outs[1:])
 
 
-def test_dispatcher_covers_every_gemm_kernel():
-    """The GEMM shapes of this file reach every kernel of the tile table, the skinny kernel, and
-    split-K on both a register-staged tile and the DMA tile, so each is checked above."""
+def test_layer_shapes_reach_both_kinds_of_tile_and_ask_for_a_workspace_where_they_split():
     cases = [(m, *LAYER_SHAPES[layer]) for layer in LAYER_SHAPES for m in (1, 8, 9, 16, 17, 32, 64, 65, 128)]
     cases += [(m, *LAYER_SHAPES[layer]) for layer in ("tinyllama_gate_up", "tinyllama_down")
               for m in (200, 256, 512, 2048)]
     cases += [(33, 128, 4160), (65, 192, 512), (17, 5632, 2048), (300, 2048, 5632), (1536, 1536, 8960)]
     plans = [ops.gemm_plan(m, n, k, 128) for m, n, k in cases]
-    kernels = {p["kernel"] for p in plans}
-    num = plans[0]["num_kernels"]
-    assert kernels == {"skinny", *range(num)}, f"kernels reached: {sorted(map(str, kernels))} of {num} + skinny"
-    split_kernels = {p["kernel"] for p in plans if p["splits"] > 1}
-    assert 2 in split_kernels, f"no split-K case for the DMA kernel: {split_kernels}"
-    assert split_kernels - {2, 6}, f"split-K only on the DMA kernels: {split_kernels}"
+    assert _kinds(plans) >= {("stream", False), ("stream", True), ("dma", False)}
     for (m, n, k), p in zip(cases, plans):
         ws = _lib.load().kf_int4_gemm_workspace_bytes(m, n, k, 128)
         assert (ws > 0) == (p["splits"] > 1)
@@ -651,7 +648,7 @@ def test_quantize_linears_swaps_decoder_linears():
 @pytest.mark.parametrize("layer,m", [("tinyllama_gate_up", 1), ("tinyllama_gate_up", 4), ("tinyllama_gate_up", 16),
                                      ("tinyllama_gate_up", 128), ("tinyllama_down", 64)])
 def test_hip_graph_capture_replays_match_eager(layer, m):
-    """Capture int4_linear (GEMV, skinny, tiled GEMM, GEMM + split-K) in a graph; every replay
+    """Capture int4_linear (GEMV, streaming tiles, LDS-DMA tiles, GEMM + split-K) in a graph; every replay
     equals eager bitwise."""
     n, k = LAYER_SHAPES[layer]
     _, _, dp, ds = _weights(n, k, 128)

@@ -1,7 +1,7 @@
 """The C ABI's size limits, exercised at their edges on the GPU (needs an MI355X).
 
 * N = KF_MAX_ROWS (2^25 - 64) rows: the GEMV's largest grid (one wavefront per two rows), the
-  skinny and the tiled GEMM across 2^19 column tiles, and the on-device quantizer over 2^28
+  streaming and LDS-DMA GEMM across 2^19 column tiles, and the on-device quantizer over 2^28
   words;
 * a grouped GEMV launch whose two problems add up to exactly KF_MAX_ROWS rows;
 * long K: rows of 2^20 and 2^24 weights (512 KiB and 8 MiB of packed words per row), past every

@@ -3,7 +3,7 @@
 Its split-K partials live in the library's per-GPU scratch array instead of a caller workspace.
 Checked against kf_int4_gemm (same plan and kernels, a torch-allocated workspace) bit for bit,
 on two calls in a row with split-K where the second problem is smaller (so stale partials of the
-first call sit in the scratch), on plans without split-K (tiled and skinny kernels); and against float64
+first call sit in the scratch), on plans without split-K (streaming and LDS-DMA tiles); and against float64
 where the workspace entry point's plan has more partials than the scratch holds.
 """
 
