@@ -323,7 +323,8 @@ def test_gemm_n_multiple_of_64_not_128(error_log, n):
 # test_gemm_tiles.py.)
 EDGE_CASES = [(513, 2112, 384), (1000, 320, 4224), (1000, 2112, 384), (1500, 640, 8960), (33, 64, 1152),
               (33, 320, 4224), (300, 960, 2048), (33, 192, 2304), (33, 640, 8960), (47, 704, 5120),
-              (130, 1600, 640), (65, 192, 4160), (900, 1472, 6272), (600, 1216, 7424), (1300, 6080, 640)]
+              (130, 1600, 640), (65, 192, 4160), (900, 1472, 6272), (600, 1216, 7424), (1300, 6080, 640),
+              (33, 1472, 8960), (193, 1472, 14336)]
 
 
 @pytest.mark.parametrize("m,n,k,group", [(m, n, k, g) for m, n, k in EDGE_CASES for g in (64, 128) if k % g == 0])
@@ -391,29 +392,34 @@ def test_gemm_rejects_n_not_multiple_of_64():
         ops.int4_gemm(x, dp, ds, 128)
 
 
-@pytest.mark.parametrize("layer,m,splitk", [("tinyllama_kv", 128, False), ("tinyllama_down", 64, True),
-                                             ("qwen_down", 32, True), ("tinyllama_down", 2048, False),
-                                             ("qwen_down", 1536, True), ("tinyllama_gate_up", 16, False),
-                                             ("tinyllama_gate_up", 768, False)])
-def test_gemm_is_deterministic(layer, m, splitk):
+DETERMINISM = [("tinyllama_kv", 128), ("tinyllama_down", 64), ("qwen_down", 33), ("tinyllama_down", 2048),
+               ("qwen_down", 517), ("qwen_down", 1536), ("tinyllama_gate_up", 16), ("tinyllama_gate_up", 768)]
+
+
+@pytest.mark.parametrize("layer,m", DETERMINISM)
+def test_gemm_is_deterministic(layer, m):
     """Split-K partials, the DMA kernel's in-block k-group halves and the streaming tiles'
     per-wave K slices are reduced in fixed order: repeated calls are bitwise identical."""
     n, k = LAYER_SHAPES[layer]
     _, _, dp, ds = _weights(n, k, 128)
     x = torch.from_numpy(_x(m, k, 99)).to(DEV)
-    ws = _lib.load().kf_int4_gemm_workspace_bytes(m, n, k, 128)
-    assert (ws > 0) == splitk, f"expected {'a' if splitk else 'no'} split-K workspace at M={m}"
     outs = [ops.int4_gemm(x, dp, ds, 128) for _ in range(3)]
     assert all(torch.equal(outs[0], o_) for o_ in outs[1:])
+
+
+def test_determinism_cases_split_k_and_do_not():
+    plans = [ops.gemm_plan(m, *LAYER_SHAPES[layer], 128) for layer, m in DETERMINISM]
+    assert _kinds(plans) >= {("stream", False), ("dma", False), ("dma", True)}
 
 
 def test_layer_shapes_reach_both_kinds_of_tile_and_ask_for_a_workspace_where_they_split():
     cases = [(m, *LAYER_SHAPES[layer]) for layer in LAYER_SHAPES for m in (1, 8, 9, 16, 17, 32, 64, 65, 128)]
     cases += [(m, *LAYER_SHAPES[layer]) for layer in ("tinyllama_gate_up", "tinyllama_down")
               for m in (200, 256, 512, 2048)]
-    cases += [(33, 128, 4160), (65, 192, 512), (17, 5632, 2048), (300, 2048, 5632), (1536, 1536, 8960)]
+    cases += [(33, 128, 4160), (65, 192, 512), (17, 5632, 2048), (300, 2048, 5632), (1536, 1536, 8960),
+              (33, 1536, 8960), (517, 1536, 8960)]
     plans = [ops.gemm_plan(m, n, k, 128) for m, n, k in cases]
-    assert _kinds(plans) >= {("stream", False), ("stream", True), ("dma", False)}
+    assert _kinds(plans) == {("stream", False), ("stream", True), ("dma", False), ("dma", True)}
     for (m, n, k), p in zip(cases, plans):
         ws = _lib.load().kf_int4_gemm_workspace_bytes(m, n, k, 128)
         assert (ws > 0) == (p["splits"] > 1)

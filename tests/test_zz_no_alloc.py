@@ -63,16 +63,17 @@ def _noalloc(x, p, s, m, n, k):
     return y
 
 
-# (M, N, K): a split-K plan (TinyLlama down at M = 64), then a smaller split-K plan picked from
-# ragged shapes; then plans without split-K.
-FIRST = (64, 2048, 5632)
-SMALLER = [(33, 320, 4224), (33, 64, 1152), (65, 192, 4160), (33, 640, 8960), (47, 704, 5120), (32, 1536, 8960)]
+# (M, N, K) of deep and ragged shapes; the test takes the one with the most partials that fit the scratch, then
+# a smaller one.
+SPLIT_CANDIDATES = [(517, 1536, 8960), (160, 4096, 14336), (33, 320, 4224), (33, 64, 4160), (65, 192, 4160),
+                    (33, 640, 8960), (47, 704, 5120), (33, 1536, 8960), (64, 2048, 5632)]
 
 
 def test_two_calls_in_a_row_match_the_workspace_entry_point():
-    big = _plan(*FIRST)
-    assert big[1] > 1 and 0 < big[2] <= _lib.KF_NOALLOC_SCRATCH_BYTES, f"expected a split-K plan, got {big}"
-    second = [c for c in SMALLER if _plan(*c)[1] > 1 and 0 < _plan(*c)[2] < big[2] and c[0] * c[1] < FIRST[0] * FIRST[1]]
+    split = [(_plan(*c)[2], c) for c in SPLIT_CANDIDATES if _plan(*c)[1] > 1]
+    split = sorted(c for c in split if c[0] <= _lib.KF_NOALLOC_SCRATCH_BYTES)
+    FIRST = split[-1][1]
+    second = [c for ws, c in split if ws < split[-1][0] and c[0] * c[1] < FIRST[0] * FIRST[1]]
     assert second, "no smaller split-K plan among the candidates"
     SECOND = second[0]
     for seed, (m, n, k) in enumerate((FIRST, SECOND)):
