@@ -937,9 +937,6 @@ static int small_m_waves(int M, int K) { return K < 2048 || (M <= 8 && K <= 4096
 //   * M <= 16: streaming tiles of small_m_waves(M, K) wavefronts without split-K only, so the K split
 //     (and with it every bit of a column) does not depend on N and concatenated q|k|v or gate|up rows
 //     give the separate layers' results.
-//   * Narrow layers from there to M = 640 take eight wavefronts, so that k and v can share a launch with q,
-//     whose plan has eight (256 x 2048, four / eight wavefronts: M = 27 3.68 / 3.64 us, 48 3.72 / 3.68, 517 5.8 /
-//     5.1; with thousands of rows four are faster: M = 2048 7.1 / 10.4).
 //   * Partials take max_partials bytes at most; splits of 1 take none, so there is a plan for any limit.
 GemmPlan gemm_plan_within(int M, int N, int K, int cu_count, size_t max_partials) {
   static_assert(sizeof(kCost) / sizeof(kCost[0]) == kNumStreamConfigs + kNumDma, "one cost entry per configuration");
@@ -953,7 +950,6 @@ GemmPlan gemm_plan_within(int M, int N, int K, int cu_count, size_t max_partials
       const StreamTile t = stream_tile_of(cfg);
       bm = t.bm, bn = t.bn, threads = 64 * t.ks;
       if (M <= 16 && t.ks != small_m_waves(M, K)) continue;
-      if (M > 16 && M <= 640 && N <= 1024 && K >= 1536 && t.ks != 8) continue;
     } else {
       const DmaEntry& e = kDma[cfg - num_stream];
       bm = e.bm, bn = e.bn, threads = e.threads;

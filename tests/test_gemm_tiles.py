@@ -28,14 +28,14 @@ CASES = [
     (6, (32, 32), 7, 81, 384, 10048), (7, (32, 48), 1, 17, 11264, 192), (7, (32, 48), 8, 17, 1472, 10048),
     (8, (48, 16), 1, 65, 1728, 832), (8, (48, 16), 8, 33, 512, 10048), (9, (48, 32), 1, 193, 1280, 448),
     (9, (48, 32), 8, 65, 512, 9024), (10, (48, 48), 1, 33, 8960, 1856), (10, (48, 48), 4, 65, 1472, 10048),
-    (11, (32, 32), 1, 17, 6400, 192), (11, (32, 32), 5, 17, 4608, 9024), (12, (48, 48), 1, 33, 8960, 192),
-    (12, (48, 48), 7, 33, 1728, 10048), (13, (64, 32), 1, 33, 6144, 192), (13, (64, 32), 7, 1025, 64, 9024),
+    (11, (32, 32), 1, 17, 6400, 192), (11, (32, 32), 7, 81, 384, 9024), (12, (48, 48), 1, 33, 8960, 192),
+    (12, (48, 48), 7, 33, 1728, 10048), (13, (64, 32), 1, 33, 6144, 192), (13, (64, 32), 7, 161, 384, 9024),
     (14, (64, 48), 1, 49, 8960, 320), (14, (64, 48), 4, 97, 1472, 9024), (15, (64, 64), 1, 97, 6400, 4160),
-    (15, (64, 64), 3, 49, 4608, 9024), (16, (8, 16), 1, 7, 64, 832), (17, (16, 16), 1, 7, 64, 192),
-    (18, (32, 128), 1, 513, 1472, 128), (18, (32, 128), 7, 17, 4608, 7424), (19, (48, 128), 1, 769, 1472, 128),
-    (19, (48, 128), 6, 129, 1728, 8960), (20, (64, 128), 1, 1025, 1472, 128), (20, (64, 128), 8, 97, 1728, 11520),
-    (21, (80, 128), 1, 1301, 1728, 128), (21, (80, 128), 8, 145, 1728, 11520), (22, (112, 128), 1, 2047, 1472, 384),
-    (22, (112, 128), 5, 81, 6400, 5632), (23, (128, 128), 1, 2047, 1728, 640),
+    (15, (64, 64), 3, 49, 4608, 9024), (16, (8, 16), 1, 7, 64, 832), (16, (8, 16), 8, 17, 64, 6272),
+    (17, (16, 16), 1, 7, 64, 192), (18, (32, 128), 1, 513, 1472, 128), (18, (32, 128), 7, 17, 4608, 7424),
+    (19, (48, 128), 1, 769, 1472, 128), (19, (48, 128), 6, 129, 1728, 8960), (20, (64, 128), 1, 1025, 1472, 128),
+    (20, (64, 128), 8, 97, 1728, 11520), (21, (80, 128), 1, 1301, 1728, 128), (21, (80, 128), 8, 145, 1728, 11520),
+    (22, (112, 128), 1, 2047, 1472, 384), (22, (112, 128), 5, 81, 6400, 5632), (23, (128, 128), 1, 2047, 1728, 640),
     (23, (128, 128), 5, 2047, 320, 11520), (24, (128, 128), 1, 1301, 1728, 192),
     (24, (128, 128), 6, 769, 1472, 9024), (25, (192, 256), 1, 1301, 8960, 128),
 ]
