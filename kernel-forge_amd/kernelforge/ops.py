@@ -79,14 +79,14 @@ def _on(device: torch.device):
 
 
 def _eager_shape(x, packed, scales, group_size) -> tuple[int, int, int, int] | None:
-    """(M, N, K, device index) of a call that every check below accepts as it is: plain contiguous tensors
-    of the right types and shapes on the current device, no tracer looking, a kernel for this M and N.
+    """(M, N, K, device index) of a call on a 2-D x that every check below accepts as it is: plain contiguous
+    tensors of the right types and shapes on the current device, no tracer looking, a kernel for this M and N.
     None for anything else, which then takes the checked path step by step (same results, and the
     errors in their order).  One pass over the attributes: the checks one function at a time, the two
     reshapes and the device context cost 4 of an eager call's 11.5 us of host time (12.3 -> 7 us above the
     GEMV's M, with the plan kept per thread)."""
     if (torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() > 0 or type(x) not in _PLAIN
-            or type(packed) not in _PLAIN or type(scales) not in _PLAIN or x.dim() != 2 or packed.dim() != 2):
+            or type(packed) not in _PLAIN or type(scales) not in _PLAIN or packed.dim() != 2):
         return None
     m, k = x.shape
     n, words = packed.shape
@@ -521,7 +521,7 @@ def int4_linear(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, gro
     Leading dimensions are flattened into M like nn.Linear; the bias add is a
     separate fp16 add, as in the reference (kernelforge/ops.py:287-302).
     """
-    shape = _eager_shape(x, packed, scales, group_size) if isinstance(x, torch.Tensor) else None
+    shape = _eager_shape(x, packed, scales, group_size) if isinstance(x, torch.Tensor) and x.dim() == 2 else None
     if shape is not None:
         y = _launch(x, packed, scales, int(group_size), *shape)
         if bias is None:
