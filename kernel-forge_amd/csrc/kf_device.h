@@ -160,6 +160,7 @@ __device__ __forceinline__ GroupEntry group_entry(const GroupTable& table, int c
   int p = 0;
 #pragma unroll
   for (int i = 1; i < kMaxGemmGroup; ++i) p += i < count && nt >= table.slot[i].tile0 ? 1 : 0;
+  p = __builtin_amdgcn_readfirstlane(p);  // uniform: one scalar address, not a chain of vector adds
   typedef const __attribute__((address_space(1))) half_t* gh_t;
   typedef const __attribute__((address_space(1))) uint32_t* gu_t;
   typedef __attribute__((address_space(1))) half_t* gy_t;

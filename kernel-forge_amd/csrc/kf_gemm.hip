@@ -868,46 +868,47 @@ namespace {
 // graph-replayed timings of every configuration and split count on 1571 (M, N, K) points: the TinyLlama,
 // Qwen2.5 and hidden-4096 layer shapes, deep and narrow layers and random sizes, N = 64 .. 28672, K = 384 ..
 // 65536, M = 5 .. 2300, weights rotated through more than the MALL, on MI355X; then small random changes kept
-// where the time of the chosen configurations fell.  The rms error is 6.3%; over those points the plan takes
-// 1.004x the time of the best configuration measured, 2.4% of them more than 1.05x and the worst 1.18x.  Fitted
-// without 339 of them: 1.005x on those, 3.2% more than 1.05x.
+// where the time of the chosen configurations, or of the shared launches of 721 sets of siblings, fell.  The rms
+// error is 6.6%; over those points the plan takes 1.004x the time of the best configuration measured, 2.7% of
+// them more than 1.05x and the worst 1.18x.  Fitted without 339 of them, 1.005x on those.
 struct CostTerms {
   int resident;
   double c[6];
 };
 const CostTerms kCost[] = {
-    {2, {1.986, 0.4153, 0.2482, 0, 0.2089, 0.03732}},  // 8 x 16, 8 wavefronts
-    {2, {1.845, 0.4258, 0.3692, 0, 0.2073, 0.03818}},  // 16 x 16, 8 wavefronts
-    {1, {0.8989, 1.644, 0.8401, 0.01794, 0, 0.04079}},  // 16 x 32, 8 wavefronts
-    {1, {0.5789, 2.181, 1.31, 0.2099, 0, 0.04975}},  // 16 x 64, 8 wavefronts
-    {1, {1.121, 1.374, 0.6625, 0, 0, 0.06604}},  // 24 x 16, 8 wavefronts
-    {1, {1.136, 1.296, 0.6933, 0, 0, 0.06841}},  // 32 x 16, 8 wavefronts
-    {1, {0.8871, 1.985, 0.9994, 0.0633, 0, 0.06261}},  // 32 x 32, 8 wavefronts
-    {1, {1.019, 1.957, 1.299, 0.06349, 0, 0.07241}},  // 32 x 48, 8 wavefronts
-    {1, {1.04, 1.783, 0.8209, 0, 0, 0.06783}},  // 48 x 16, 8 wavefronts
-    {1, {1.259, 1.723, 1.253, 0, 0, 0.06859}},  // 48 x 32, 8 wavefronts
-    {1, {1.29, 2.13, 1.649, 0.007682, 0, 0.06816}},  // 48 x 48, 8 wavefronts
-    {3, {2.001, 0.4321, 0.6378, 0.1131, 0.6246, 0.06697}},  // 32 x 32, 4 wavefronts
+    {2, {1.984, 0.4153, 0.2482, 0, 0.2089, 0.03732}},  // 8 x 16, 8 wavefronts
+    {2, {1.845, 0.4258, 0.3692, 0, 0.2073, 0.03661}},  // 16 x 16, 8 wavefronts
+    {1, {0.886, 1.644, 0.8801, 0.01794, 0, 0.04079}},  // 16 x 32, 8 wavefronts
+    {1, {0.579, 2.181, 1.31, 0.2099, 0, 0.04975}},  // 16 x 64, 8 wavefronts
+    {1, {1.117, 1.392, 0.6625, 0, 0, 0.05753}},  // 24 x 16, 8 wavefronts
+    {1, {1.136, 1.264, 0.7326, 0, 0, 0.05531}},  // 32 x 16, 8 wavefronts
+    {1, {0.8871, 1.904, 1.01, 0.06335, 0, 0.06971}},  // 32 x 32, 8 wavefronts
+    {1, {1.019, 2.211, 1.189, 0.06349, 0, 0.06941}},  // 32 x 48, 8 wavefronts
+    {1, {1.04, 1.797, 0.8525, 0, 0, 0.06783}},  // 48 x 16, 8 wavefronts
+    {1, {1.259, 1.727, 1.253, 0, 0, 0.06864}},  // 48 x 32, 8 wavefronts
+    {1, {1.29, 2.13, 1.649, 0.007682, 0, 0.06996}},  // 48 x 48, 8 wavefronts
+    {3, {2.001, 0.3777, 0.6995, 0.1152, 0.6246, 0.06622}},  // 32 x 32, 4 wavefronts
     {2, {2.182, 0.8556, 1.111, 0.09628, 0.7392, 0.06249}},  // 48 x 48, 4 wavefronts
-    {2, {1.927, 0.8336, 0.969, 0, 0.8278, 0.05605}},  // 64 x 32, 4 wavefronts
-    {1, {1.209, 2.199, 2.21, 0, 0, 0.05848}},  // 64 x 48, 4 wavefronts
-    {1, {1.285, 2.572, 2.684, 0, 0, 0.0555}},  // 64 x 64, 4 wavefronts
+    {2, {1.973, 0.8494, 0.969, 0, 1.071, 0.05605}},  // 64 x 32, 4 wavefronts
+    {1, {1.268, 2.544, 2.267, 0, 0, 0.05075}},  // 64 x 48, 4 wavefronts
+    {1, {1.407, 3.238, 2.549, 0, 0, 0.05075}},  // 64 x 64, 4 wavefronts
     {4, {1.961, 0.2121, 0.2981, 0.01678, 0.3614, 0.0314}},  // 8 x 16, 4 wavefronts
-    {3, {1.772, 0.1784, 0.2508, 0, 0.7393, 0.04036}},  // 16 x 16, 4 wavefronts
-    {2, {2.797, 0.7188, 2.733, 0, 0.565, 0.05338}},  // 32 x 128, 8 wavefronts
+    {3, {1.708, 0.1784, 0.2774, 0, 0.7866, 0.04328}},  // 16 x 16, 4 wavefronts
+    {2, {2.592, 0.7188, 2.733, 0, 0.565, 0.05338}},  // 32 x 128, 8 wavefronts
     {1, {1.143, 2.937, 3.828, 0, 0, 0.04331}},  // 48 x 128, 8 wavefronts
     {2, {3.103, 1.157, 3.993, 0, 0.3402, 0.04573}},  // 64 x 128, 8 wavefronts
-    {1, {0.9014, 3.96, 4.759, 0, 0, 0.04338}},  // 80 x 128, 8 wavefronts
-    {1, {1.188, 4.192, 6.754, 0, 0, 0.02955}},  // 112 x 128, 8 wavefronts
-    {1, {0.5374, 5.407, 6.61, 0, 0, 0.03055}},  // 128 x 128, 8 wavefronts
+    {1, {0.8987, 4.095, 4.752, 0, 0, 0.04338}},  // 80 x 128, 8 wavefronts
+    {1, {1.188, 3.945, 6.805, 0, 0, 0.02955}},  // 112 x 128, 8 wavefronts
+    {1, {0.5004, 5.407, 6.61, 0, 0, 0.03066}},  // 128 x 128, 8 wavefronts
     {2, {3.71, 1.076, 4.24, 0, 4.835, 0.01889}},  // 128 x 128, 4 wavefronts
-    {1, {2.347, 5.555, 20.57, 0, 0, 0.01319}},  // 192 x 256, 8 wavefronts
+    {1, {2.347, 5.555, 19.64, 0, 0, 0.0132}},  // 192 x 256, 8 wavefronts
 };
 // Split-K costs one more launch plus the fp32 partials (same fit), and is taken only when the
 // model predicts it at least 2% faster.  One margin for all sizes: asking for a workspace at fixed rows of deep
 // layers made 2048 x 5632 at M = 64 / 900 take 9.6 / 34.0 us split where 7.6 / 30.2 unsplit are possible, and
 // 2048 x 12416 at M = 1773 107 where 93 are.
-constexpr double kSplitUs = 2.391, kSplitUsPerMElem = 1.314, kSplitMargin = 1.02;
+constexpr double kSplitUs = 2.268, kSplitUsPerMElem = 1.372, kSplitMargin = 1.02;
+constexpr double kSiblingUs = 0.5;   // see gemm_plan_within
 constexpr int kMaxSplits = 8;        // the largest split count the fit was measured on
 constexpr int kMinSplitK = 512;      // k per split
 
@@ -928,20 +929,27 @@ static double plan_cost(int cfg, long tiles, int splits, int M, double n, int K,
 
 // At M <= 16 the K split over wavefronts depends on M and K alone (see gemm_plan).  Four wavefronts
 // leave room for more workgroups per CU, which wide layers want; eight shorten a long K.  Best tile
-// with 4 / 8 (us): 17920 x 1536 at M = 6 / 16: 8.6 / 10.2 and 9.6 / 12.1; 11264 x 2048: 6.3 / 7.4 and
-// 7.1 / 7.2; 2560 x 2048: 4.1 / 4.1 and 4.7 / 4.4; 28672 x 4096: 19.6 / 22.3 and 25.1 / 23.9; 4096 x
-// 4096: 5.8 / 5.4 and 7.2 / 5.9; 4096 x 14336: 13.2 / 12.0 and 17.8 / 14.1.
+// with 4 / 8 (us): 17920 x 1536 at M = 6 / 16: 7.5 / 8.5 and 8.4 / 10.6; 11264 x 2048: 5.5 / 6.1 and
+// 6.1 / 6.6; 2560 x 2048: 3.5 / 3.4 and 4.5 / 3.7; 28672 x 4096: 15.9 / 18.0 and 22.9 / 21.5; 4096 x
+// 4096: 5.1 / 4.6 and 6.5 / 5.2; 4096 x 14336: 11.2 / 9.4 and 17.0 / 12.3.
 static int small_m_waves(int M, int K) { return K < 2048 || (M <= 8 && K <= 4096) ? 4 : 8; }
 
 // Kernel choice: the configuration and split-K factor with the smallest modelled time.
 //   * M <= 16: streaming tiles of small_m_waves(M, K) wavefronts without split-K only, so the K split
 //     (and with it every bit of a column) does not depend on N and concatenated q|k|v or gate|up rows
 //     give the separate layers' results.
+//   * Narrow layers (k and v) get kSiblingUs off where they sum in the order of the K x K layer's plan (q),
+//     so that they can share its launch: that saves a call with its siblings 2-4 us, and costs a call by itself
+//     at most the half (q|k|v of 1024 + 2 x 128 columns, K = 1024, M = 27: 3.5 us together, 6.4 where q and k, v
+//     take different wavefront counts).  Over 779 measured sets q|k|v takes 0.947x the time without it, over 273
+//     narrow layers a call by itself 1.003x.
 //   * Partials take max_partials bytes at most; splits of 1 take none, so there is a plan for any limit.
 GemmPlan gemm_plan_within(int M, int N, int K, int cu_count, size_t max_partials) {
   static_assert(sizeof(kCost) / sizeof(kCost[0]) == kNumStreamConfigs + kNumDma, "one cost entry per configuration");
   const int cus = cu_count > 0 ? cu_count : 256;
   const int num_stream = stream_num_configs();
+  const bool narrow = M > 16 && N <= 1024 && 4 * N <= K;
+  const GemmPlan square = narrow ? gemm_plan(M, K, K, cu_count) : GemmPlan{};
   int best_cfg = -1, best_splits = 1;
   double best = 1e300;
   for (int cfg = 0; cfg < gemm_num_configs(); ++cfg) {
@@ -962,7 +970,8 @@ GemmPlan gemm_plan_within(int M, int N, int K, int cu_count, size_t max_partials
     const int max_splits = can_split ? std::min(kMaxSplits, std::max(1, K / kMinSplitK)) : 1;
     for (int s = 1; s <= max_splits; ++s) {
       if (s > 1 && (size_t)s * M * N * sizeof(float) > max_partials) break;
-      const double cost = plan_cost(cfg, tiles, s, M, N, K, cus);
+      double cost = plan_cost(cfg, tiles, s, M, N, K, cus);
+      if (narrow && s == 1 && gemm_same_sums(square, gemm_plan_with(cfg, 1, K))) cost -= kSiblingUs;
       if (cost < best) {
         best = cost;
         best_cfg = cfg;
@@ -1006,9 +1015,9 @@ bool gemm_same_sums(const GemmPlan& a, const GemmPlan& b) {
 // of its own plan.  All plans have to be of one kind (gemm_same_sums); the tile is the one with the
 // smallest modelled time for all columns together, taken where that is less than the sum of the
 // separate launches.  Separate / grouped, us: q|k|v of 2048 + 2 x 256 columns, K = 2048, at M = 16 / 64 /
-// 200 (k|v): 11.3 / 4.4, 12.2 / 5.5, 15.4 / 12.1; gate|up of 2 x 5632: 10.7 / 7.4, 14.0 / 12.4, 25.9 / 19.2;
-// 2 x 14336, K = 4096, at M = 128 / 517 / 1024: 50.7 / 39.6, 164 / 160, 252 / 261 (the worst; asking for a
-// predicted gain of 3% left that one grouped and lost 8% at 2 x 8960, K = 1536, M = 200).
+// 200: 10.2 / 4.1, 10.8 / 5.6, 13.0 / 9.5; gate|up of 2 x 5632: 9.5 / 7.0, 12.6 / 11.8, 24.8 / 18.4; 2 x 14336, K =
+// 4096, at M = 64 / 128 / 517: 33.7 / 32.0, 52.1 / 40.5, 167 / 165.  The worst of 279 sets: 2 x 15360, K = 3968, at M =
+// 27 31.7 / 32.7.
 int gemm_group_config(const GemmPlan* plans, const int* N, int count, int M, int K, int cu_count) {
   const int cus = cu_count > 0 ? cu_count : 256;
   double best = 0.0, columns = 0.0;

@@ -21,21 +21,21 @@ DEV = "cuda"
 
 # (configuration, tile, splits, M, N, K)
 CASES = [
-    (0, (8, 16), 1, 9, 64, 2112), (0, (8, 16), 8, 17, 64, 9024), (1, (16, 16), 1, 17, 64, 1088),
-    (1, (16, 16), 8, 17, 192, 9024), (2, (16, 32), 1, 33, 2304, 1088), (2, (16, 32), 8, 33, 320, 10048),
-    (3, (16, 64), 1, 33, 4608, 320), (4, (24, 16), 1, 17, 2304, 1856), (4, (24, 16), 6, 17, 640, 10048),
-    (5, (32, 16), 1, 17, 2304, 832), (5, (32, 16), 8, 49, 192, 9024), (6, (32, 32), 1, 17, 4608, 1856),
-    (6, (32, 32), 7, 81, 384, 10048), (7, (32, 48), 1, 17, 11264, 192), (7, (32, 48), 8, 17, 1472, 10048),
-    (8, (48, 16), 1, 65, 1728, 832), (8, (48, 16), 8, 33, 512, 10048), (9, (48, 32), 1, 193, 1280, 448),
-    (9, (48, 32), 8, 65, 512, 9024), (10, (48, 48), 1, 33, 8960, 1856), (10, (48, 48), 4, 65, 1472, 10048),
-    (11, (32, 32), 1, 17, 6400, 192), (11, (32, 32), 7, 81, 384, 9024), (12, (48, 48), 1, 33, 8960, 192),
-    (12, (48, 48), 7, 33, 1728, 10048), (13, (64, 32), 1, 33, 6144, 192), (13, (64, 32), 7, 161, 384, 9024),
-    (14, (64, 48), 1, 49, 8960, 320), (14, (64, 48), 4, 97, 1472, 9024), (15, (64, 64), 1, 97, 6400, 4160),
-    (15, (64, 64), 3, 49, 4608, 9024), (16, (8, 16), 1, 7, 64, 832), (16, (8, 16), 8, 17, 64, 6272),
-    (17, (16, 16), 1, 7, 64, 192), (18, (32, 128), 1, 513, 1472, 128), (18, (32, 128), 7, 17, 4608, 7424),
-    (19, (48, 128), 1, 769, 1472, 128), (19, (48, 128), 6, 129, 1728, 8960), (20, (64, 128), 1, 1025, 1472, 128),
+    (0, (8, 16), 1, 17, 64, 1088), (0, (8, 16), 8, 17, 64, 9024), (1, (16, 16), 1, 33, 64, 832),
+    (1, (16, 16), 8, 17, 192, 9024), (2, (16, 32), 1, 33, 2304, 1088), (2, (16, 32), 7, 33, 384, 10048),
+    (3, (16, 64), 1, 33, 4608, 320), (4, (24, 16), 1, 17, 2304, 1856), (4, (24, 16), 6, 33, 320, 10048),
+    (5, (32, 16), 1, 1025, 64, 320), (5, (32, 16), 8, 17, 384, 10048), (6, (32, 32), 1, 17, 4608, 1856),
+    (6, (32, 32), 6, 97, 320, 9024), (7, (32, 48), 1, 17, 8960, 576), (7, (32, 48), 8, 17, 1472, 10048),
+    (8, (48, 16), 1, 65, 1728, 832), (8, (48, 16), 7, 385, 64, 10048), (9, (48, 32), 1, 33, 6144, 320),
+    (9, (48, 32), 8, 65, 512, 9024), (10, (48, 48), 1, 33, 8960, 1856), (10, (48, 48), 4, 65, 1472, 9024),
+    (11, (32, 32), 1, 17, 6400, 192), (11, (32, 32), 5, 17, 4608, 9024), (12, (48, 48), 1, 33, 8960, 192),
+    (12, (48, 48), 7, 33, 1728, 10048), (13, (64, 32), 1, 97, 6400, 192), (13, (64, 32), 6, 49, 2560, 9024),
+    (14, (64, 48), 1, 49, 8960, 1088), (14, (64, 48), 5, 49, 2304, 9024), (15, (64, 64), 1, 97, 6400, 2112),
+    (15, (64, 64), 2, 2047, 256, 9024), (16, (8, 16), 1, 7, 64, 832), (16, (8, 16), 8, 17, 64, 7424),
+    (17, (16, 16), 1, 7, 64, 192), (18, (32, 128), 1, 513, 1472, 128), (18, (32, 128), 7, 17, 4608, 5632),
+    (19, (48, 128), 1, 900, 1472, 128), (19, (48, 128), 6, 129, 1728, 8960), (20, (64, 128), 1, 1025, 1472, 384),
     (20, (64, 128), 8, 97, 1728, 11520), (21, (80, 128), 1, 1301, 1728, 128), (21, (80, 128), 8, 145, 1728, 11520),
-    (22, (112, 128), 1, 2047, 1472, 384), (22, (112, 128), 5, 81, 6400, 5632), (23, (128, 128), 1, 2047, 1728, 640),
+    (22, (112, 128), 1, 2047, 1472, 384), (22, (112, 128), 7, 97, 4608, 6272), (23, (128, 128), 1, 2047, 1728, 640),
     (23, (128, 128), 5, 2047, 320, 11520), (24, (128, 128), 1, 1301, 1728, 192),
     (24, (128, 128), 6, 769, 1472, 9024), (25, (192, 256), 1, 1301, 8960, 128),
 ]
