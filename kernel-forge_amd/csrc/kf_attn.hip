@@ -4,7 +4,11 @@
 //
 // q fp16 [heads, d]; cache_k fp16 [kv_heads, d, max_seq] (K transposed); cache_v fp16
 // [kv_heads, max_seq, d]; mask fp16 rows of max_seq additive values; out fp16 [heads, d].  Scores,
-// softmax and the weighted sum stay in fp32; the output is rounded once.
+// softmax and the weighted sum stay in fp32; the output is rounded once.  Error against 64 bits (32 heads on 4, d =
+// 64, max_seq 96 .. 288, q of 1, 2 and 4 times unit variance, 120 draws): 2.08e-4 of the result, what rounding the exact
+// result to fp16 gives, with __expf as with expf (0.3 us slower); the library's three launches, which round scores
+// and probabilities to fp16, 4.7e-4 to 9.1e-4.  Whole models of 4 to 22 layers are 0.983x as far from 64 bits as with
+// those (0.93x to 1.06x by seed); the two differ by 3e-3 of the logits, each being about that far off.
 //
 // What bounds it: latency.  The work of a TinyLlama layer at max_seq = 160 is 40 KiB of K and V per KV
 // head; as three library launches (a batched product, a softmax over fp16 scores, a batched product)

@@ -19,8 +19,8 @@
 //   * Every byte of a stage goes global -> LDS through LDS-DMA; the weights stay PACKED in LDS (4
 //     bits per weight: 4x less LDS traffic than an fp16 W_hat tile) and each wavefront dequantizes
 //     its own columns' words.
-//   * LDS layouts are XOR-swizzled so every fragment read is free of bank conflicts on gfx950's
-//     64-bank LDS.
+//   * LDS layouts are XOR-swizzled: sixteen consecutive lanes of a fragment read touch all 64 banks
+//     (SQ_LDS_BANK_CONFLICT is 14-19% of SQ_LDS_IDX_ACTIVE in the four-k-group tiles).
 //   * MFMA operands: lane l serves row / column l % 16 and k-group g = l / 16.
 //   * Tiles are ordered in bands of group_m M-tiles (all N-tiles of a band before the next
 //     band); the (split, tile) jobs of a launch, split-major, are dealt to the 8 XCDs in
@@ -73,8 +73,8 @@ __device__ __forceinline__ bool gemm_job(int tiles, int splits, int& split, int&
 // newer one may still be in flight.
 //
 // LDS stage layout (bytes): x rows of A_ROW = 2 BK bytes with 16-byte chunk c at slot
-// c ^ a_swz(row); packed rows of BK / 2 bytes with 16-byte chunk h at h ^ b_swz(row).  Every
-// read phase of the MFMA fragments is free of bank conflicts.  Three stages rotate.  Scales:
+// c ^ a_swz(row); packed rows of BK / 2 bytes with 16-byte chunk h at h ^ b_swz(row).  Sixteen
+// consecutive lanes of a fragment read touch all banks.  Three stages rotate.  Scales:
 // a stage lies inside one group (G >= 64 = BK), so they live in their own ring of three slabs of
 // 4-byte slots, one slab per group, fetched by the k-group 0 wavefronts with the first stage of the
 // group (that stage costs those two wavefronts one more DMA, and their wait count for it is one

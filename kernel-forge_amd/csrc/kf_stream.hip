@@ -23,14 +23,16 @@
 //     and starts the next copy into the same buffer before its MFMAs, so the copy runs under them
 //     (two or four buffers in LDS measured no faster: the other wavefronts of the CU hide the
 //     rest, and the LDS holds more workgroups instead).
-//   * Weights: one instruction copies 8 rows x 128 bytes, a "step" of WP = 4 pieces; WS steps are in
-//     flight, because these come from HBM.  Scales: 2 bytes per column and 64-k piece, copied
-//     with the step into 4-byte slots.
+//   * Weights: one instruction copies 8 rows x 128 bytes, a "step" of WP = 4 pieces, into one of WS
+//     slots.  Copies complete in order and an iteration waits for its x, so only a step issued right
+//     after that x stays in flight over an iteration; the others have landed one iteration after their
+//     issue.  Scales: 2 bytes per column and 64-k piece, copied with the step into 4-byte slots.
 //   * MFMA operands: lane l serves row / column l % 16 and k-group g = l / 16.  In sub-step t (0, 1)
 //     of a piece it supplies k = 16 g + 8 t .. + 7 for both operands: x chunk 2 g + t of its row,
 //     packed word 2 g + t of its column.  16-byte chunks are XOR-swizzled within their row (by
 //     the row's position in the 256-byte bank window), which permutes lanes inside one line of the
-//     copy and keeps every fragment read free of bank conflicts.
+//     copy and spreads sixteen consecutive lanes of a fragment read over all banks (counted all the same:
+//     SQ_LDS_BANK_CONFLICT is 34-47% of SQ_LDS_IDX_ACTIVE).
 //   * The MFMAs take the weights as their first operand, so each 16 x 16 block comes out
 //     transposed: lane l, element r holds row l % 16, column 4 (l / 16) + r (8-byte stores of y).
 //   * The loop is rolled on purpose.  The kernels live for 3-20 us; a version with the steps

@@ -82,8 +82,8 @@ SIBLING_GROUPS = (("q_proj", "k_proj", "v_proj"), ("gate_proj", "up_proj"))
 class _SiblingLaunch:
     """One ops.int4_linear_grouped call for sibling KFLinearInt4 modules called on the same input.
 
-    The first sibling called on an input launches the group (one GEMV launch at decode sizes, the
-    per-problem kernels above them: every output is bit-identical to the sibling's own
+    The first sibling called on an input launches the group (one GEMV launch at decode sizes, as few
+    GEMM launches as the plans allow above them: every output is bit-identical to the sibling's own
     int4_linear) and keeps the other outputs until their modules are called with that same input
     object.  A call with another input while outputs are still waiting - another tensor, or the
     same tensor updated in place since (its version counter moved; tensors made under

@@ -23,10 +23,12 @@ from torch._subclasses.fake_tensor import FakeTensor
 
 from kernelforge import _lib
 
-# Measured GEMV/GEMM crossover on one MI355X (dispatch_sweep.py beside bench.py): the
-# largest M at which the sum of GEMV times over the layer shapes beats the GEMM's
-# (reference rule, bench/sweep_int4_dispatch.py:51-57).  Above it int4_gemm runs the
-# streaming MFMA kernel for small and medium M, then the LDS-DMA tiles.
+# Largest M that goes to the GEMV; above it int4_gemm runs the streaming MFMA kernel for small and
+# medium M, then the LDS-DMA tiles.  The reference's rule (bench/sweep_int4_dispatch.py:51-57: the
+# largest M at which the sum of GEMV times over the layer shapes beats the GEMM's) gives 3 on one MI355X
+# (dispatch_sweep.py beside bench.py; GEMV / GEMM over 8 shapes, us: M = 3 32.2 / 35.3, M = 4 36.3 / 35.8,
+# M = 5 43.7 / 36.5).  M = 4 stays on the GEMV all the same: the sums are 1.4% apart, and the GEMV
+# multiplies by the exact q s where the GEMM's matrix cores take fp16(q s).
 GEMV_MAX_M = 4
 # The reference's int4_matmul sends M <= 7 to its GEMV, which accepts every N, and M >= 8
 # to its GEMM, which rejects N % 64 != 0 (kernelforge/ops.py:193,204-214).  Our MFMA kernels
