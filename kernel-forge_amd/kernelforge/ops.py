@@ -530,7 +530,7 @@ def int4_linear(x: torch.Tensor, packed: torch.Tensor, scales: torch.Tensor, gro
             return y
         y = y + bias
         # A bias of more dimensions broadcasts the sum: back to the output's shape, or refused, as below.
-        return y if y.shape == shape[:2] else y.reshape(shape[:2])
+        return y if y.dim() == 2 and y.numel() == shape[0] * shape[1] else y.reshape(shape[:2])
     lead = x.shape[:-1]
     x2 = x.reshape(-1, x.shape[-1])
     if not x2.is_contiguous():
